@@ -361,7 +361,7 @@ static int check_params(aco_params &prm, int min_n)
 // Instance checks: finite, non-negative, symmetric distances; every
 // customer servable by a vehicle of its own (otherwise construction could
 // never visit it: kernel.cl:438-479 would not terminate).
-static int check_instance(const aco_problem *pb, int width, std::vector<int> &nnl, bool &int16)
+static int check_instance(const aco_problem *pb, int width, std::vector<int> &nnl, bool &int16, bool &packed)
 {
     const int n = pb->n;
     if (n < 3 || n > kMaxNodes) return set_error(ACO_ERR_ARG, "aco_create: need 3 <= n <= 4096");
@@ -370,15 +370,20 @@ static int check_instance(const aco_problem *pb, int width, std::vector<int> &nn
     if (isnan(pb->max_dist) || !(pb->service_time >= 0.0f) || !isfinite(pb->service_time))
         return set_error(ACO_ERR_ARG, "bad max_dist or service_time");
     int16 = true;
+    float longest = 0.0f;
     for (int i = 0; i < n; ++i)
         for (int j = 0; j < n; ++j) {
             const float d = pb->dist[(size_t)i * n + j];
             if (!isfinite(d) || d < 0.0f) return set_error(ACO_ERR_ARG, "distances must be finite and >= 0");
             if (d != pb->dist[(size_t)j * n + i]) return set_error(ACO_ERR_ARG, "distance matrix is not symmetric");
             int16 = int16 && d <= 65535.0f && d == floorf(d);
+            longest = d > longest ? d : longest;
         }
-    for (int i = 0; i < n; ++i)
+    packed = int16 && longest <= (float)kPackedMax;
+    for (int i = 0; i < n; ++i) {
         if (pb->demand[i] < 0) return set_error(ACO_ERR_ARG, "negative demand");
+        packed = packed && pb->demand[i] <= kPackedDemand && pb->dist[(size_t)i * n + i] == 0.0f;
+    }
     for (int i = 1; i < n; ++i) {
         if (pb->demand[i] > pb->capacity)
             return set_error(ACO_ERR_INFEASIBLE, "customer " + std::to_string(i) + " demand exceeds capacity");
@@ -452,13 +457,14 @@ int aco_create_batch(const aco_problem *pbs, int32_t count, const aco_params *pr
     if (rc) return rc;
     std::vector<std::vector<int>> nnl(count);
     std::vector<int> nn_ls(count);
-    std::vector<char> int16(count);
+    std::vector<char> int16(count), packed(count);
     for (int b = 0; b < count; ++b) {
         nn_ls[b] = prm.nn_ls > 0 ? prm.nn_ls : pbs[b].n - 2;
-        bool i16 = false;
-        rc = check_instance(&pbs[b], std::max(prm.k, nn_ls[b]), nnl[b], i16);
+        bool i16 = false, pk = false;
+        rc = check_instance(&pbs[b], std::max(prm.k, nn_ls[b]), nnl[b], i16, pk);
         if (rc) return rc;
         int16[b] = i16;
+        packed[b] = pk;
     }
 
     int ndev = 0;
@@ -601,6 +607,7 @@ int aco_create_batch(const aco_problem *pbs, int32_t count, const aco_params *pr
         dp.Q = pb->capacity; dp.D = pb->max_dist; dp.svc = pb->service_time;
         dp.alpha = prm.alpha; dp.rho = prm.rho;
         dp.has_d = isfinite(pb->max_dist) ? 1 : 0;
+        dp.packed = packed[b] ? 1 : 0;
         dp.dem16 = 1;
         for (int i = 0; i < n; ++i)
             if (pb->demand[i] < 0 || pb->demand[i] > 65535) dp.dem16 = 0;

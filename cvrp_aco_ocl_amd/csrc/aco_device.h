@@ -39,7 +39,7 @@ __device__ __forceinline__ int wave_id()
 // DPP controls: quad_perm [1,0,3,2] (lane ^ 1), quad_perm [2,3,0,1]
 // (lane ^ 2), row_shl / row_shr by 4 and 8 (lane +- 4, +- 8 within a row of
 // 16 lanes).  Out-of-row reads give 0.
-enum { kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppShl4 = 0x104, kDppShr4 = 0x114, kDppShl8 = 0x108,
+enum { kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppMirror = 0x140, kDppHalfMirror = 0x141, kDppShl4 = 0x104, kDppShr4 = 0x114, kDppShl8 = 0x108,
        kDppShr8 = 0x118 };
 
 template <int CTRL>
@@ -110,6 +110,8 @@ __device__ __forceinline__ unsigned long long wave_reduce_u64(unsigned long long
 constexpr float kEps = 0.001f;         // utilities.h:19
 constexpr int kMaxNodes = 4096;        // 12-bit node ids in reduction keys
 constexpr int kMaxRas = 16;
+constexpr int kPackedMax = 8190;       // largest distance of the packed 16-bit relocate
+constexpr int kPackedDemand = 8191;    // and largest demand
 constexpr int kMaxMovesPerRoute = 1 << 14;
 constexpr int kMaxMovesFactor = 64;    // swap/relocate cap = 64*n per call
 
@@ -137,6 +139,7 @@ struct DevProblem {
     float tau0_nn;            // 1/(n * L_nn) for the nearest-neighbour tau0 rule
     int has_d;                // max_dist is finite
     int dem16;                // every demand is in [0, 65535]
+    int packed;               // integer distances in [0, kPackedMax], 0 to itself; demands <= kPackedDemand
     unsigned long long seed;  // Philox key of this instance
     const float *dist;        // n*P
     const float *d0;          // n, distance to the depot (column 0)

@@ -106,6 +106,10 @@ __device__ __forceinline__ LsLds ls_bind(int n, int ring, int rowbytes, bool per
 }
 
 
+// The loads written above stay above, their uses below: the scheduler would
+// otherwise spread independent LDS reads out and wait for each in turn.
+__device__ __forceinline__ void loads_issued() { __builtin_amdgcn_sched_barrier(0); }
+
 __device__ __forceinline__ float Dd(const DevProblem &p, int a, int b)
 {
     return p.dist[(size_t)a * p.P + b];
@@ -630,16 +634,24 @@ template <int W> __device__ __forceinline__ unsigned wave_offsets(int wave)
     return every << wave;
 }
 
+// Node at a tour position (PK: the packed search's tour, in dtw's space).
+template <bool PK>
+__device__ __forceinline__ int tour_node(const LsLds &L, int pos)
+{
+    typedef unsigned short __attribute__((may_alias)) u16;
+    return PK ? (int)reinterpret_cast<const u16 *>(L.dtw)[pos] >> 1 : L.tour[pos];
+}
+
 // Copy the rows of the window offsets in `need` (bit q: position base + q):
 // offset q is issued by wave q mod W, so a run of up to W offsets is one row
 // per wave and each wave finds its own with a few scalar instructions.
-template <int W, typename RT>
+template <int W, typename RT, bool PK = false>
 __device__ __forceinline__ void rows_issue(const DevProblem &p, const LsLds &L, const RowRing<RT> &rr,
                                            int base, unsigned need, int wave, int lane)
 {
     for (unsigned m = need & wave_offsets<W>(wave); m; m &= m - 1u) {
         const int pos = base + __builtin_ctz(m);
-        row_copy_wave<RT>(p, __builtin_amdgcn_readfirstlane(L.tour[pos]), rr.at(pos), lane);
+        row_copy_wave<RT>(p, __builtin_amdgcn_readfirstlane(tour_node<PK>(L, pos)), rr.at(pos), lane);
     }
 }
 
@@ -663,14 +675,14 @@ __device__ __forceinline__ void window_clear(RowWindow &w, int lo, int hi)
 
 // Make the rows of window offsets [0, cnt) present (cnt <= W+2), spread
 // over the waves; a barrier follows when any was missing.
-template <int W, typename RT>
+template <int W, typename RT, bool PK = false>
 __device__ __forceinline__ void rows_ensure(const DevProblem &p, const LsLds &L, const RowRing<RT> &rr,
                                             RowWindow &w, int cnt, int tid)
 {
     const unsigned need = ((1u << cnt) - 1u) & ~w.mask;
     w.mask |= (1u << cnt) - 1u;
     if (need) {
-        rows_issue<W, RT>(p, L, rr, w.base, need, wave_id(), tid & 63);
+        rows_issue<W, RT, PK>(p, L, rr, w.base, need, wave_id(), tid & 63);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
     }
@@ -681,7 +693,7 @@ __device__ __forceinline__ void rows_ensure(const DevProblem &p, const LsLds &L,
 // waited for before the round's barrier.  Enabled per launch when the ring
 // holds both rounds' positions (2W+2 <= R): the positions of this round and
 // the next never share a slot.
-template <int W, typename RT>
+template <int W, typename RT, bool PK = false>
 __device__ __forceinline__ unsigned prefetch_issue(const DevProblem &p, const LsLds &L, const RowRing<RT> &rr,
                                                    bool on, const RowWindow &w, int off, int S, int tid)
 {
@@ -690,7 +702,7 @@ __device__ __forceinline__ unsigned prefetch_issue(const DevProblem &p, const Ls
     const int avail = S - pos0 < W ? S - pos0 : W;
     if (avail <= 0) return 0;
     const unsigned want = ((1u << avail) - 1u) & ~(w.mask >> off);
-    if (want) rows_issue<W, RT>(p, L, rr, pos0, want, wave_id(), tid & 63);
+    if (want) rows_issue<W, RT, PK>(p, L, rr, pos0, want, wave_id(), tid & 63);
     return want;
 }
 
@@ -1180,6 +1192,435 @@ __device__ __forceinline__ void ls_relocate(const DevProblem &p, LsLds &L, const
     if (tid == 0) moves += done;
 }
 
+// ----------------------------------------------------- packed relocate ----
+
+// Instances whose distances are integers up to kPackedMax (and demands up to
+// kPackedDemand; DevProblem::packed) take this relocate.  Same rounds, rows
+// and order as ls_relocate; the difference is the arithmetic: eight
+// consecutive edges per lane (512 per trip), gains as packed 16-bit
+// integers, exact because no intermediate leaves 16 bits, and the capacity
+// test of each edge's route beside them, so only candidates that fit leave
+// the trip (70% of the scans at 1001 nodes meet an improving insertion, 15
+// to 27% one that fits).  A trip costs about 110 instructions for 512
+// edges, one of relocate_scan about 100 for 128.
+// Measured with 256 ants at 1001 nodes: relocate 1.18 -> 0.93 ms of a search
+// of 2.24 -> 2.00 ms; 480 ants at 481 nodes 0.38 -> 0.36 ms; 256 instances of
+// 64 ants 10.7 -> 10.2 ms.  What bounds it there is the round around the
+// scans: two barriers, the row ring's upkeep and the move itself.
+//
+// A swap has four row reads per candidate instead of one, which no packing
+// saves: the same scheme measured slower there (1001 nodes 0.86 -> 1.00 ms),
+// so swaps keep ls_swap.
+//
+// Arrays by position, 16 bits each:
+//   t2    2 * node (the byte offset of its row entry)
+//   w     edge (q, q+1)
+//   rx    route; a depot carries the route that starts at it, so rx[q] is
+//         also the route of edge q
+//   room  free capacity of that route (-kRoomMax past the tour's end)
+// t2 and w lie in dtw's space, rx in ridx's, room in tour's (tour is written
+// back from t2 afterwards).
+
+constexpr int kRoomMax = 16000;   // beyond any demand: a larger room decides the same
+static_assert(kRoomMax > kPackedDemand && kRoomMax + kPackedDemand < 32768, "room test fits 16 bits");
+constexpr short kFarDist = 16383;   // row entry of a node's own distance while relocating
+static_assert(kFarDist + 2 * kPackedMax < 32768 && 3 * kPackedMax < 32768, "gains fit 16 bits");
+
+typedef short __attribute__((ext_vector_type(2))) s16x2;
+typedef unsigned __attribute__((ext_vector_type(4), may_alias)) u32x4;
+typedef unsigned short __attribute__((may_alias)) u16_alias;
+
+// Eight 16-bit entries as four pairs.
+struct Oct16 { s16x2 p[4]; };
+
+__device__ __forceinline__ unsigned bits16(s16x2 v) { return __builtin_bit_cast(unsigned, v); }
+__device__ __forceinline__ s16x2 pair16(unsigned v) { return __builtin_bit_cast(s16x2, v); }
+__device__ __forceinline__ s16x2 both16(int v) { return s16x2{(short)v, (short)v}; }
+
+__device__ __forceinline__ Oct16 oct16(const unsigned short *a, int x)
+{
+    const u32x4 v = reinterpret_cast<const u32x4 *>(a)[x];
+    const unsigned e0 = v.x, e1 = v.y, e2 = v.z, e3 = v.w;
+    return {{pair16(e0), pair16(e1), pair16(e2), pair16(e3)}};
+}
+
+// Row entry at a byte offset (t2).
+__device__ __forceinline__ unsigned short row_at(const unsigned short *row, unsigned off)
+{
+    return *reinterpret_cast<const u16_alias *>(reinterpret_cast<const char *>(row) + off);
+}
+__device__ __forceinline__ Oct16 row_gather(const unsigned short *row, const Oct16 &t)
+{
+    Oct16 r;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const unsigned o = bits16(t.p[u]);
+        r.p[u] = s16x2{(short)row_at(row, o & 0xFFFFu), (short)row_at(row, o >> 16)};
+    }
+    return r;
+}
+
+// The entries one position earlier (prev's upper half comes first) or later
+// (next's lower half comes last).
+__device__ __forceinline__ Oct16 entries_before(const Oct16 &v, unsigned prev)
+{
+    Oct16 r;
+    r.p[0] = pair16(__builtin_amdgcn_alignbit(bits16(v.p[0]), prev, 16));
+#pragma unroll
+    for (int u = 1; u < 4; ++u) r.p[u] = pair16(__builtin_amdgcn_alignbit(bits16(v.p[u]), bits16(v.p[u - 1]), 16));
+    return r;
+}
+__device__ __forceinline__ Oct16 entries_after(const Oct16 &v, unsigned next)
+{
+    Oct16 r;
+#pragma unroll
+    for (int u = 0; u < 3; ++u) r.p[u] = pair16(__builtin_amdgcn_alignbit(bits16(v.p[u + 1]), bits16(v.p[u]), 16));
+    r.p[3] = pair16(__builtin_amdgcn_alignbit(next, bits16(v.p[3]), 16));
+    return r;
+}
+
+// Some entry is negative; the signs as a mask in position order.
+__device__ __forceinline__ bool any_negative(const Oct16 &f)
+{
+    return ((bits16(f.p[0]) | bits16(f.p[1]) | bits16(f.p[2]) | bits16(f.p[3])) & 0x80008000u) != 0;
+}
+__device__ __forceinline__ unsigned sign_mask(const Oct16 &f)
+{
+    unsigned m = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const unsigned b = bits16(f.p[u]);
+        m |= ((b >> 15) & 1u) << (2 * u) | (b >> 31) << (2 * u + 1);
+    }
+    return m;
+}
+// Bits of the positions below lim in the lane's eight from q0 on.
+__device__ __forceinline__ unsigned bits_below(int lim, int q0)
+{
+    const int c = lim - q0;
+    return (1u << (c < 0 ? 0 : c > 8 ? 8 : c)) - 1u;
+}
+
+__device__ __forceinline__ int room16(int q) { return q > kRoomMax ? kRoomMax : q < -kRoomMax ? -kRoomMax : q; }
+
+struct PackedTour {
+    unsigned short *t2, *w, *rx, *room;
+    int len;   // entries allocated (the tour, then zero padding to whole lanes)
+    int octs;  // lanes' worth of tour positions
+};
+__device__ __forceinline__ PackedTour packed_bind(const LsLds &L, int n, int S)
+{
+    PackedTour T;
+    T.len = (2 * n + 23) & ~7;
+    T.t2 = reinterpret_cast<unsigned short *>(L.dtw);
+    T.w = T.t2 + T.len;
+    T.rx = reinterpret_cast<unsigned short *>(L.ridx);
+    T.room = reinterpret_cast<unsigned short *>(L.tour);
+    T.octs = (S + 7) >> 3;
+    return T;
+}
+
+// t2, w and rx from the tour (after ls_routes).
+template <int W>
+__device__ __forceinline__ void packed_fill(const DevProblem &p, const LsLds &L, const PackedTour &T, int S, int tid)
+{
+    for (int q = tid; q < T.len; q += LsW<W>::threads) {
+        const bool in = q < S;
+        const int v = in ? L.tour[q] : 0, x = q + 1 < S ? L.tour[q + 1] : 0;
+        const unsigned short e = gload(p.dist16 + (size_t)v * p.P + x);
+        T.t2[q] = (unsigned short)(2 * v);
+        T.w[q] = q + 1 < S ? e : (unsigned short)0;
+        if (!in) T.rx[q] = 0x0FFF;   // no route
+        else if (v == 0 && q > 0) T.rx[q] = (unsigned short)(T.rx[q] + 1);
+    }
+    __syncthreads();
+}
+
+// Per-route load, distance + service and customer count, one thread per
+// route (the sums in tour order), then the free capacity by position.
+template <int W>
+__device__ __forceinline__ void packed_tables(const DevProblem &p, LsLds &L, const PackedTour &T, int R, int S, int tid)
+{
+    constexpr int U = 4;   // positions whose loads are issued together
+    for (int r = tid; r < R; r += LsW<W>::threads) {
+        const int beg = L.zpos[r], end = L.zpos[r + 1];
+        int load = 0;
+        float dist = 0.0f;
+        for (int i = beg + 1; i <= end; i += U) {
+            int t[U], e[U], dm[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int q = i + u <= end ? i + u : end;
+                t[u] = T.t2[q];
+                e[u] = T.w[q - 1];
+            }
+            loads_issued();
+#pragma unroll
+            for (int u = 0; u < U; ++u) dm[u] = L.dem[t[u] >> 1];
+            loads_issued();
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (i + u > end) continue;
+                load += dm[u];
+                dist += (float)e[u];
+            }
+        }
+        L.rl[r] = load;
+        L.rd[r] = dist + p.svc * (float)(end - beg - 1);
+        L.rc[r] = (short)(end - beg - 1);
+    }
+    __syncthreads();
+    for (int q = tid; q < T.len; q += LsW<W>::threads) {
+        const int r = q < S - 1 ? T.rx[q] : -1;
+        T.room[q] = (unsigned short)(r >= 0 ? room16(p.Q - L.rl[r]) : -kRoomMax);
+    }
+    __syncthreads();
+}
+
+// Smallest value over the wave.
+__device__ __forceinline__ int wave_min_i32(int v)
+{
+    auto low = [](int a, int b) { return a < b ? a : b; };
+    v = low(v, __builtin_amdgcn_mov_dpp(v, kDppXor1, 0xF, 0xF, true));
+    v = low(v, __builtin_amdgcn_mov_dpp(v, kDppXor2, 0xF, 0xF, true));
+    v = low(v, __builtin_amdgcn_mov_dpp(v, kDppHalfMirror, 0xF, 0xF, true));
+    v = low(v, __builtin_amdgcn_mov_dpp(v, kDppMirror, 0xF, 0xF, true));
+    const int r0 = __builtin_amdgcn_readlane(v, 0), r1 = __builtin_amdgcn_readlane(v, 16);
+    const int r2 = __builtin_amdgcn_readlane(v, 32), r3 = __builtin_amdgcn_readlane(v, 48);
+    return low(low(r0, r1), low(r2, r3));
+}
+
+// Relocate of position i (relocate_scan above): first accepted j or -1.
+// Edges are taken in order; the row entry of n1 itself holds kFarDist, which
+// rules out its own two edges.  An edge is a candidate when its route is
+// n1's or has room, and the position j it stands for holds a customer: the
+// edge's end before i, its start after i.
+__device__ __forceinline__ int packed_relocate_scan(const DevProblem &p, const LsLds &L, const PackedTour &T, int S,
+                                                    int i, const unsigned short *rowP, unsigned short *rowB, int lane,
+                                                    const ScanStop &stop, int &evc)
+{
+    const unsigned t1 = T.t2[i], ts1 = T.t2[i + 1];
+    const int a1 = T.w[i - 1], b1 = T.w[i], r1 = T.rx[i];
+    loads_issued();
+    const int c1 = row_at(rowP, ts1), dn1 = L.dem[t1 >> 1];
+    if (lane == 0) *reinterpret_cast<u16_alias *>(reinterpret_cast<char *>(rowB) + t1) = kFarDist;
+    group_sync();
+    const s16x2 gain1 = both16(a1 + b1 - c1), own = both16(r1), dem1 = both16(dn1), one = both16(1);
+    for (int b8 = 0; 8 * b8 < S - 1; b8 += kLanes) {
+        const int x = b8 + lane, xc = x < T.octs ? x : T.octs - 1;
+        const int hi = 8 * (b8 + kLanes) < T.len ? 8 * (b8 + kLanes) : T.len - 1;
+        const Oct16 t = oct16(T.t2, xc), w = oct16(T.w, xc), rx = oct16(T.rx, xc), room = oct16(T.room, xc);
+        const unsigned thi = T.t2[hi], key = read_key(stop.key);
+        loads_issued();
+        const Oct16 v = row_gather(rowB, t);
+        const unsigned vhi = row_at(rowB, thi);
+        loads_issued();
+        const Oct16 vs = entries_after(v, (unsigned)wave_next((int)bits16(v.p[0]), (int)vhi));
+        Oct16 f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const s16x2 g = ((v.p[u] + vs.p[u]) - w.p[u]) - gain1;
+            const s16x2 same = (rx.p[u] ^ own) - one, full = room.p[u] - dem1;
+            f.p[u] = g & (same | ~full);
+        }
+        if (__ballot(any_negative(f) && x < T.octs)) {
+            Oct16 z;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) z.p[u] = t.p[u] - one;   // negative at depots
+            const unsigned zs = sign_mask(z);
+            const unsigned ze = (zs >> 1) | (((unsigned)wave_next((int)zs, thi == 0 ? 1 : 0) & 1u) << 7);
+            const unsigned before = bits_below(i, 8 * x);
+            unsigned m = x < T.octs ? sign_mask(f) & ~((before & ze) | (~before & zs)) : 0u;
+            int q = -1;
+            if (!p.has_d) {
+                const u64 ml = __ballot(m != 0);
+                if (ml) {
+                    const int l = __builtin_ctzll(ml);
+                    q = 8 * (b8 + l) + __builtin_ctz((unsigned)__builtin_amdgcn_readlane((int)m, l));
+                }
+            } else {
+                int best = 1 << 30;
+                const bool own1 = !(((L.rd[r1] - p.svc) - (float)(a1 + b1)) + (float)c1 > p.D);
+                while (__ballot(m != 0)) {
+                    const bool on = m != 0;
+                    const int e = on ? 8 * x + __builtin_ctz(m) : 0;
+                    m &= m - 1u;
+                    const unsigned t0 = T.t2[e], t1e = T.t2[e + 1];
+                    const int rm = T.w[e], r2 = T.rx[e];
+                    loads_issued();
+                    const int add = (int)row_at(rowB, t0) + (int)row_at(rowB, t1e);
+                    const float dist2 = ((L.rd[r2] + p.svc) - (float)rm) + (float)add;
+                    const bool ok = on & ((r2 == r1) | (own1 & !(dist2 > p.D)));
+                    best = ok && e < best ? e : best;
+                }
+                if (__ballot(best < (1 << 30))) q = wave_min_i32(best);
+            }
+            if (q >= 0) {
+                const int js = q < i ? q + 1 : q;
+                // customers in [1, js] other than n1 itself
+                evc = js - (int)T.rx[js] - (i <= js ? 1 : 0);
+                return js;
+            }
+        }
+        // stopped early: a lower wave has a move and this result is dropped
+        if (__builtin_amdgcn_readfirstlane((int)key) > (int)stop.mine) break;
+    }
+    // every customer but n1
+    evc = p.n - 2;
+    return -1;
+}
+
+// Four consecutive 16-bit entries.
+typedef unsigned short __attribute__((ext_vector_type(4), may_alias)) u16x4;
+
+template <int W>
+__device__ __forceinline__ void packed_relocate(const DevProblem &p, LsLds &L, const PackedTour &T,
+                                                const RowRing<unsigned short> &rr, bool pf_on, int S, int tid,
+                                                unsigned &round, long long &ev, int &moves)
+{
+    const int lane = tid & 63, w = wave_id();
+    const int cap = kMaxMovesFactor * p.n;
+    int done = 0, i0 = 1, parity = 0;
+    RowWindow win = {0, 0u};
+    while (i0 < S - 1 && done < cap) {
+        // rows of positions i0-1 .. i0+W-1: d(pred, .) gives c1, d(n1, .) the gains
+        window_move(win, i0 - 1);
+        rows_ensure<W, unsigned short, true>(p, L, rr, win, min(W + 1, S - i0), tid);
+        const unsigned pfw = prefetch_issue<W, unsigned short, true>(p, L, rr, pf_on, win, W + 1, S - 1, tid);
+        const int i = i0 + w;
+        int j = -1, evc = 0;
+        const ScanStop stop = {reinterpret_cast<const unsigned *>(L.res + LsW<W>::res_first), round_key(++round, w)};
+        // uniform per wave (scalar branches); the route must keep a customer
+        bool scan = i < S - 1;
+        if (scan) {
+            const int t = T.t2[i], r = T.rx[i];
+            loads_issued();
+            scan = __builtin_amdgcn_readfirstlane(t) != 0;
+            if (scan) scan = __builtin_amdgcn_readfirstlane((int)L.rc[r]) >= 2;
+        }
+        if (scan) j = packed_relocate_scan(p, L, T, S, i, rr.at(i - 1), rr.at(i), lane, stop, evc);
+        if (j >= 0 && lane == 0) atomicMax(reinterpret_cast<unsigned *>(L.res + LsW<W>::res_first), stop.mine);
+        int *res = L.res + W * parity;
+        parity ^= 1;
+        if (lane == 0) res[w] = j;
+        prefetch_wait(win, pfw, W + 1);
+        __syncthreads();
+        int js;
+        const int wstar = round_pick<W>(res, stop.key, round, lane, js);
+        if (lane == 0 && (wstar < 0 || w <= wstar)) ev += evc;
+        if (wstar < 0) {   // see ls_relocate
+            i0 += W;
+            continue;
+        }
+        const int is = i0 + wstar;
+        const bool up = is < js;
+        const int lo = up ? is : js, hi = up ? js : is;
+        // every value the move needs, read by every thread before any write:
+        // x is the insertion's other neighbour (pn2 before j, sn2 after it);
+        // the new edges are (pn1, sn1) = c1, (n1, n2) = e_n2 and (n1, x) = e_x
+        const unsigned t1 = T.t2[is], ts1 = T.t2[is + 1], t2 = T.t2[js], tx = T.t2[up ? js + 1 : js - 1];
+        const int a1 = T.w[is - 1], b1 = T.w[is], rm = T.w[up ? js : js - 1], r1 = T.rx[is], r2 = T.rx[js];
+        loads_issued();
+        const unsigned short *rowP = rr.at(is - 1), *rowB = rr.at(is);
+        const int c1 = row_at(rowP, ts1), e_n2 = row_at(rowB, t2), e_x = row_at(rowB, tx);
+        const int dn1 = L.dem[t1 >> 1], rl1 = L.rl[r1], rl2 = L.rl[r2], rc1 = L.rc[r1], rc2 = L.rc[r2];
+        const float rd1 = L.rd[r1], rd2 = L.rd[r2];
+        loads_issued();
+        // shift, in place: positions [lo, hi] move by one towards is, n1
+        // lands at js in the route of the node that was there; edges and
+        // routes move with the positions, and the rooms of the two routes
+        // change.  Four positions per thread, read before the barrier and
+        // written after it; tours longer than a block's reach are taken in
+        // the direction of the move, so a source is read before it is
+        // written.
+        constexpr int NT = LsW<W>::threads;
+        const int quads = (S + 3) >> 2, nch = (quads + NT - 1) / NT;
+        const int room1 = room16(p.Q - (rl1 - dn1)), room2 = room16(p.Q - (r1 != r2 ? rl2 + dn1 : rl2));
+        for (int c = 0; c < nch; ++c) {
+            const int x = (up ? c : nch - 1 - c) * NT + tid, q0 = 4 * x;
+            const bool in = x < quads;
+            u16x4 t = {}, e = {}, r = {}, m = {};
+            unsigned tn = 0, en = 0, rn = 0, mn = 0;   // the neighbour on the source side
+            const bool shift = in && q0 <= hi && q0 + 3 >= lo - 1;
+            if (in) {
+                r = reinterpret_cast<const u16x4 *>(T.rx)[x];
+                m = reinterpret_cast<const u16x4 *>(T.room)[x];
+            }
+            if (shift) {
+                const int qn = up ? q0 + 4 : q0 > 0 ? q0 - 1 : 0;
+                t = reinterpret_cast<const u16x4 *>(T.t2)[x];
+                e = reinterpret_cast<const u16x4 *>(T.w)[x];
+                tn = T.t2[qn];
+                en = T.w[qn];
+                rn = T.rx[qn];
+                mn = T.room[qn];
+            }
+            __syncthreads();
+            if (c == 0 && tid == NT - 1) {
+                // by a thread of the last wave, which has the least to shift
+                const int add = e_n2 + e_x, gain = -(a1 + b1 + rm) + (add + c1);
+                if (r1 != r2) {
+                    L.rl[r1] = rl1 - dn1;
+                    L.rl[r2] = rl2 + dn1;
+                    L.rd[r1] = ((rd1 - p.svc) - (float)(a1 + b1)) + (float)c1;
+                    L.rd[r2] = ((rd2 + p.svc) - (float)rm) + (float)add;
+                    L.rc[r1] = (short)(rc1 - 1);
+                    L.rc[r2] = (short)(rc2 + 1);
+                } else {
+                    L.rd[r1] = rd1 + (float)gain;
+                }
+            }
+            const unsigned ts[4] = {t.x, t.y, t.z, t.w}, es[4] = {e.x, e.y, e.z, e.w}, rs[4] = {r.x, r.y, r.z, r.w},
+                           ms[4] = {m.x, m.y, m.z, m.w};
+            unsigned to[4], eo[4], ro[4], mo[4];
+            bool rooms = false;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int q = q0 + k;
+                const unsigned st = up ? (k < 3 ? ts[k < 3 ? k + 1 : 3] : tn) : (k > 0 ? ts[k > 0 ? k - 1 : 0] : tn);
+                const unsigned se = up ? (k < 3 ? es[k < 3 ? k + 1 : 3] : en) : (k > 0 ? es[k > 0 ? k - 1 : 0] : en);
+                const unsigned sr = up ? (k < 3 ? rs[k < 3 ? k + 1 : 3] : rn) : (k > 0 ? rs[k > 0 ? k - 1 : 0] : rn);
+                const unsigned sm = up ? (k < 3 ? ms[k < 3 ? k + 1 : 3] : mn) : (k > 0 ? ms[k > 0 ? k - 1 : 0] : mn);
+                const bool mv = shift & (q >= lo) & (q <= hi), last = q == js;
+                to[k] = mv ? (last ? t1 : st) : ts[k];
+                ro[k] = mv ? (last ? (unsigned)r2 : sr) : rs[k];
+                mo[k] = mv ? (last ? (unsigned)(unsigned short)room2 : sm) : ms[k];
+                unsigned ev_ = es[k];
+                if (shift) {
+                    if (up) {
+                        if (q >= lo && q < hi) ev_ = se;
+                        if (q == is - 1) ev_ = (unsigned)c1;
+                        if (q == js - 1) ev_ = (unsigned)e_n2;
+                        if (q == js) ev_ = (unsigned)e_x;
+                    } else {
+                        if (q > lo && q <= hi) ev_ = se;
+                        if (q == is) ev_ = (unsigned)c1;
+                        if (q == js) ev_ = (unsigned)e_n2;
+                        if (q == js - 1) ev_ = (unsigned)e_x;
+                    }
+                }
+                eo[k] = ev_;
+                if (r1 != r2 && q < S - 1) {
+                    if ((int)ro[k] == r1) { mo[k] = (unsigned)(unsigned short)room1; rooms = true; }
+                    if ((int)ro[k] == r2) { mo[k] = (unsigned)(unsigned short)room2; rooms = true; }
+                }
+            }
+            if (shift) {
+                reinterpret_cast<u16x4 *>(T.t2)[x] = u16x4{(unsigned short)to[0], (unsigned short)to[1], (unsigned short)to[2], (unsigned short)to[3]};
+                reinterpret_cast<u16x4 *>(T.w)[x] = u16x4{(unsigned short)eo[0], (unsigned short)eo[1], (unsigned short)eo[2], (unsigned short)eo[3]};
+                reinterpret_cast<u16x4 *>(T.rx)[x] = u16x4{(unsigned short)ro[0], (unsigned short)ro[1], (unsigned short)ro[2], (unsigned short)ro[3]};
+            }
+            if (in && (shift || rooms))
+                reinterpret_cast<u16x4 *>(T.room)[x] = u16x4{(unsigned short)mo[0], (unsigned short)mo[1], (unsigned short)mo[2], (unsigned short)mo[3]};
+            __syncthreads();
+        }
+        window_clear(win, lo, hi);
+        i0 = is;
+        ++done;
+    }
+    if (tid == 0) moves += done;
+}
+
 // ---------------------------------------------------------- one ant ----
 
 // Local search of ant a of one instance by the W waves of the calling block,
@@ -1287,10 +1728,28 @@ __device__ void local_search_ant(const DevProblem &p, const DevState &s, int a, 
         ls_swap<W, RT>(p, L, rr, pf_on, S, tid, round, ev, moves);
     }
     if (flags & kLsRelocate) {
-        ls_edges<W>(p, L, 0, S - 2, tid);
-        __syncthreads();
-        ls_routes<W>(p, L, S, tid, true);
-        ls_relocate<W, RT>(p, L, rr, pf_on, S, tid, round, ev, moves);
+        bool packed = false;
+        if constexpr (sizeof(RT) == 2) {
+            if (p.packed) {
+                packed = true;
+                // a swap keeps the depots' positions and the route indices
+                if (!(flags & kLsSwap)) ls_routes<W>(p, L, S, tid, false);
+                else __syncthreads();
+                const int R = __builtin_amdgcn_readfirstlane(L.res[LsW<W>::res_r]);
+                const PackedTour T = packed_bind(L, p.n, S);
+                packed_fill<W>(p, L, T, S, tid);
+                packed_tables<W>(p, L, T, R, S, tid);
+                packed_relocate<W>(p, L, T, rr, pf_on, S, tid, round, ev, moves);
+                for (int q = tid; q < S; q += NT) L.tour[q] = T.t2[q] >> 1;
+                __syncthreads();   // the edges below take t2's space
+            }
+        }
+        if (!packed) {
+            ls_edges<W>(p, L, 0, S - 2, tid);
+            __syncthreads();
+            ls_routes<W>(p, L, S, tid, true);
+            ls_relocate<W, RT>(p, L, rr, pf_on, S, tid, round, ev, moves);
+        }
     }
     __builtin_amdgcn_s_setprio(0);
     ls_edges<W>(p, L, 0, S - 2, tid);
