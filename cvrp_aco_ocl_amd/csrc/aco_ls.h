@@ -112,7 +112,7 @@ __device__ __forceinline__ void loads_issued() { __builtin_amdgcn_sched_barrier(
 
 __device__ __forceinline__ float Dd(const DevProblem &p, int a, int b)
 {
-    return p.dist[(size_t)a * p.P + b];
+    return gload(p.dist + (size_t)a * p.P + b);
 }
 
 // dtw[q] = d(tour[q], tour[q+1]) for q in [lo, hi]
@@ -212,29 +212,65 @@ __device__ __forceinline__ void group_sync()
 // d(n1, n2), so one pass evaluates both: one round of memory latency per
 // position instead of two.
 //
-// Candidate q (q may lie past rend: the caller masks it).  Loads are
-// unconditional (clamped, in-bounds indices) so a lane's candidates have
-// all their loads in flight at once.  ok*: in the row (rp < nn_ls), inside
-// the radius and, for the predecessor scan, not adjacent; gains as the
-// reference computes them; xs = s2, xp = p2.
-__device__ __forceinline__ void two_opt_cand(const DevProblem &p, const LsLds &L, int rend, int pos1, int q,
-                                             int n1, int s1, int p1, float rads, float radp,
-                                             const unsigned short *rowpos, bool &oks, bool &okp, float &gs,
-                                             float &gp, int &rp, int &n2, int &xs, int &xp)
+// A lane's candidates of one trip: positions q0, q0 + 8, ... (past rend:
+// clamped and masked).  Every LDS read, then every global read is requested
+// before any is used, unconditionally (clamped, in-bounds indices): the
+// scan is bound by the latency of these reads, by their cache lines when
+// ants fill the device.  The distances are read from the 16-bit matrix
+// where the search uses 16-bit rows (half the lines of the fp32 rows for
+// the same values).  256 instances of 64 ants: search 13.1 -> 12.6 ms on
+// fresh tours; 101 nodes, 2-opt alone: 62 -> 60 us.  Reading the row
+// position only where a candidate improves measured slower (12.9 ms, 64
+// us): it puts a second latency behind the first.
+// ok*: in the row (rp < nn_ls), inside the radius and, for the predecessor
+// scan, not adjacent; gains as the reference computes them; xs = s2,
+// xp = p2.
+template <typename RT>
+__device__ __forceinline__ float opt_dist(const DevProblem &p, int a, int b)
 {
-    const int qq = q <= rend ? q : rend;
-    n2 = L.tour[qq];
-    xs = qq == rend ? 0 : L.tour[qq + 1];
-    xp = L.tour[qq - 1];
-    const float ews = L.dtw[qq], ewp = L.dtw[qq - 1];
-    rp = rowpos[n2];
-    const float dn = Dd(p, n1, n2);
-    const float dxs = Dd(p, s1, xs), dxp = Dd(p, p1, xp);
-    const bool base = (q <= rend) & (q != pos1) & (rp < p.nn_ls);
-    oks = base & (rads - dn > kEps);
-    okp = base & (radp - dn > kEps) & !(xp == n1 || p1 == n2);
-    gs = -rads + dn + dxs - ews;
-    gp = -radp + dn + dxp - ewp;
+    if constexpr (sizeof(RT) == 2) return (float)gload(p.dist16 + (size_t)a * p.P + b);
+    else return Dd(p, a, b);
+}
+
+template <int U> struct OptCands {
+    bool oks[U], okp[U];
+    float gs[U], gp[U];
+    int rp[U], n2[U], xs[U], xp[U];
+};
+
+template <typename RT, int U>
+__device__ __forceinline__ void two_opt_cands(const DevProblem &p, const LsLds &L, int rend, int pos1, int q0, int n1,
+                                              int s1, int p1, float rads, float radp, const unsigned short *rowpos,
+                                              OptCands<U> &c)
+{
+    float ews[U], ewp[U], dn[U], dxs[U], dxp[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int q = q0 + u * kOptGroup, qq = q <= rend ? q : rend;
+        c.n2[u] = L.tour[qq];
+        c.xs[u] = qq == rend ? 0 : L.tour[qq + 1];
+        c.xp[u] = L.tour[qq - 1];
+        ews[u] = L.dtw[qq];
+        ewp[u] = L.dtw[qq - 1];
+    }
+    loads_issued();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        dn[u] = opt_dist<RT>(p, n1, c.n2[u]);
+        dxs[u] = opt_dist<RT>(p, s1, c.xs[u]);
+        dxp[u] = opt_dist<RT>(p, p1, c.xp[u]);
+        c.rp[u] = gload(rowpos + c.n2[u]);
+    }
+    loads_issued();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int q = q0 + u * kOptGroup;
+        const bool base = (q <= rend) & (q != pos1) & (c.rp[u] < p.nn_ls);
+        c.oks[u] = base & (rads - dn[u] > kEps);
+        c.okp[u] = base & (radp - dn[u] > kEps) & !(c.xp[u] == n1 || p1 == c.n2[u]);
+        c.gs[u] = -rads + dn[u] + dxs[u] - ews[u];
+        c.gp[u] = -radp + dn[u] + dxp[u] - ewp[u];
+    }
 }
 
 // Candidates per lane per trip of a 2-opt scan: positions q, q+8, q+16 and
@@ -246,6 +282,7 @@ constexpr int kOptUnroll = 4;
 // move) with h1..h4 set (same in all lanes of the group).  The evaluated
 // moves are the sequential pair's: the successor scan's up to its move, or
 // all of them plus the predecessor scan's up to its move.
+template <typename RT>
 __device__ __forceinline__ int two_opt_scans(const DevProblem &p, const LsLds &L, int rbeg, int rend, int pos1,
                                              int n1, int s1, int p1, float rads, float radp, int gl,
                                              long long &evals, int &h1, int &h2, int &h3, int &h4)
@@ -254,28 +291,32 @@ __device__ __forceinline__ int two_opt_scans(const DevProblem &p, const LsLds &L
     const unsigned short *rowpos = p.nnpos + (size_t)n1 * p.n;
     u64 bs = ~0ull, bp = ~0ull;
     int cs = 0, cp = 0;
-    // the first trip's candidates, kept for the evaluated-move count
-    bool oks_k[U], okp_k[U];
-    int rp_k[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) { oks_k[u] = okp_k[u] = false; rp_k[u] = 0; }
+    // the first trip's candidates, kept for the evaluated-move count (one
+    // trip covers most routes)
+    unsigned oks_k = 0, okp_k = 0;
+    int rp_k[U] = {};
     for (int q0 = rbeg + 1 + gl; q0 <= rend; q0 += U * kOptGroup) {
-        bool oks[U], okp[U];
-        float gs[U], gp[U];
-        int rp[U], a[U], xs[U], xp[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            two_opt_cand(p, L, rend, pos1, q0 + u * kOptGroup, n1, s1, p1, rads, radp, rowpos, oks[u], okp[u],
-                         gs[u], gp[u], rp[u], a[u], xs[u], xp[u]);
-        const bool first = q0 == rbeg + 1 + gl;
+        OptCands<U> c;
+        two_opt_cands<RT, U>(p, L, rend, pos1, q0, n1, s1, p1, rads, radp, rowpos, c);
+        unsigned oks = 0, okp = 0;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            cs += oks[u];
-            cp += okp[u];
-            const u64 kr = ((u64)rp[u] << 32) | ((u64)a[u] << 16);
-            if (oks[u] && gs[u] < -kEps) bs = (kr | (u64)xs[u]) < bs ? (kr | (u64)xs[u]) : bs;
-            if (okp[u] && gp[u] < -kEps) bp = (kr | (u64)xp[u]) < bp ? (kr | (u64)xp[u]) : bp;
-            if (first) { oks_k[u] = oks[u]; okp_k[u] = okp[u]; rp_k[u] = rp[u]; }
+            oks |= (unsigned)c.oks[u] << u;
+            okp |= (unsigned)c.okp[u] << u;
+            const bool is = c.oks[u] && c.gs[u] < -kEps, ip = c.okp[u] && c.gp[u] < -kEps;
+            if (is || ip) {
+                const u64 kr = ((u64)c.rp[u] << 32) | ((u64)c.n2[u] << 16);
+                if (is) bs = (kr | (u64)c.xs[u]) < bs ? (kr | (u64)c.xs[u]) : bs;
+                if (ip) bp = (kr | (u64)c.xp[u]) < bp ? (kr | (u64)c.xp[u]) : bp;
+            }
+        }
+        cs += __builtin_popcount(oks);
+        cp += __builtin_popcount(okp);
+        if (q0 == rbeg + 1 + gl) {
+            oks_k = oks;
+            okp_k = okp;
+#pragma unroll
+            for (int u = 0; u < U; ++u) rp_k[u] = c.rp[u];
         }
     }
     int kind = 0;
@@ -295,19 +336,15 @@ __device__ __forceinline__ int two_opt_scans(const DevProblem &p, const LsLds &L
     const int rps = (int)(best >> 32);
     int cnt = 0;
     if (rend - rbeg <= U * kOptGroup) {
+        const unsigned ok = kind == 1 ? oks_k : okp_k;
 #pragma unroll
-        for (int u = 0; u < U; ++u) cnt += (kind == 1 ? oks_k[u] : okp_k[u]) && rp_k[u] <= rps;
+        for (int u = 0; u < U; ++u) cnt += ((ok >> u) & 1u) && rp_k[u] <= rps;
     } else {
         for (int q0 = rbeg + 1 + gl; q0 <= rend; q0 += U * kOptGroup) {
+            OptCands<U> c;
+            two_opt_cands<RT, U>(p, L, rend, pos1, q0, n1, s1, p1, rads, radp, rowpos, c);
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                bool oks, okp;
-                float gs, gp;
-                int rp, a, xs, xp;
-                two_opt_cand(p, L, rend, pos1, q0 + u * kOptGroup, n1, s1, p1, rads, radp, rowpos, oks, okp, gs,
-                             gp, rp, a, xs, xp);
-                cnt += (kind == 1 ? oks : okp) && rp <= rps;
-            }
+            for (int u = 0; u < U; ++u) cnt += (kind == 1 ? c.oks[u] : c.okp[u]) && c.rp[u] <= rps;
         }
     }
     // the predecessor scan runs after the whole successor scan
@@ -376,7 +413,7 @@ __device__ __forceinline__ int two_opt_next(const LsLds &L, int rbeg, int l, int
 // kernel.cl:126-277 for route r at positions [rbeg, rend] (rbeg holds the
 // depot), run by the kOptGroup lanes gl = 0.. of one group; RANDOM scans
 // the positions in the order of perm (localSearch.cpp:180-294).
-template <bool RANDOM>
+template <bool RANDOM, typename RT>
 __device__ __forceinline__ void two_opt_route(const DevProblem &p, LsLds &L, int r, int rbeg,
                                               int rend, int gl, long long &evals, int &moves_total)
 {
@@ -399,7 +436,7 @@ __device__ __forceinline__ void two_opt_route(const DevProblem &p, LsLds &L, int
             // the depot
             const float rads = L.dtw[pos1], radp = pos1 == rbeg ? L.dtw[rend] : L.dtw[pos1 - 1];
             const bool found =
-                two_opt_scans(p, L, rbeg, rend, pos1, n1, s1, p1, rads, radp, gl, evals, h1, h2, h3, h4) != 0;
+                two_opt_scans<RT>(p, L, rbeg, rend, pos1, n1, s1, p1, rads, radp, gl, evals, h1, h2, h3, h4) != 0;
             if (!found) {
                 if (n1 == 0) dlb0 = true;
                 else if (gl == 0) L.dlb[n1] = 1;
@@ -424,8 +461,8 @@ __device__ __forceinline__ void two_opt_route(const DevProblem &p, LsLds &L, int
             group_sync();
             // edge weights: the two new edges, the segment between reversed
             if (gl == 0) {
-                L.dtw[ph1] = Dd(p, h1, h3);
-                L.dtw[ph3] = Dd(p, h2, h4);
+                L.dtw[ph1] = opt_dist<RT>(p, h1, h3);
+                L.dtw[ph3] = opt_dist<RT>(p, h2, h4);
             }
             const int ed = (ph3 - ph1 - 1) / 2;
             for (int t = gl; t < ed; t += kOptGroup) {
@@ -466,7 +503,7 @@ __device__ __forceinline__ u64 two_opt_pack(int kind, int h1, int h2, int h3, in
 // sequential search would see.  After a move at the first position the
 // search continues right after it and scans the second again.  Halves
 // exchange their results with one DPP swap (16-lane groups are DPP rows).
-template <bool RANDOM>
+template <bool RANDOM, typename RT>
 __device__ __forceinline__ void two_opt_route_pair(const DevProblem &p, LsLds &L, int r, int rbeg, int rend,
                                                    int gl16, long long &evals, int &moves_total)
 {
@@ -494,7 +531,7 @@ __device__ __forceinline__ void two_opt_route_pair(const DevProblem &p, LsLds &L
                 const int s1 = pos1 == rend ? 0 : L.tour[pos1 + 1];
                 const int p1 = pos1 == rbeg ? L.tour[rend] : L.tour[pos1 - 1];
                 const float rads = L.dtw[pos1], radp = pos1 == rbeg ? L.dtw[rend] : L.dtw[pos1 - 1];
-                kind = two_opt_scans(p, L, rbeg, rend, pos1, n1, s1, p1, rads, radp, hl, ev, h1, h2, h3, h4);
+                kind = two_opt_scans<RT>(p, L, rbeg, rend, pos1, n1, s1, p1, rads, radp, hl, ev, h1, h2, h3, h4);
             }
             const u64 mine = two_opt_pack(kind, h1, h2, h3, h4);
             const u64 other = dpp_xor8_u64(mine, lane);
@@ -538,8 +575,8 @@ __device__ __forceinline__ void two_opt_route_pair(const DevProblem &p, LsLds &L
             const int tb = h2 == 0 ? rbeg : L.pos[h2];
             group_sync();
             if (gl16 == 0) {
-                L.dtw[ph1] = Dd(p, h1, h3);
-                L.dtw[ph3] = Dd(p, h2, h4);
+                L.dtw[ph1] = opt_dist<RT>(p, h1, h3);
+                L.dtw[ph3] = opt_dist<RT>(p, h2, h4);
             }
             const int ed = (ph3 - ph1 - 1) / 2;
             for (int t = gl16; t < ed; t += G) {
@@ -1673,11 +1710,11 @@ __device__ void local_search_ant(const DevProblem &p, const DevState &s, int a, 
         if (R <= NT / (2 * kOptGroup)) {
             // a group of 16 lanes per route: two positions at a time
             const int grp = tid / (2 * kOptGroup), gl = tid % (2 * kOptGroup);
-            if (grp < R) two_opt_route_pair<false>(p, L, grp, L.zpos[grp], L.zpos[grp + 1] - 1, gl, ev, moves);
+            if (grp < R) two_opt_route_pair<false, RT>(p, L, grp, L.zpos[grp], L.zpos[grp + 1] - 1, gl, ev, moves);
         } else {
             const int grp = tid / kOptGroup, gl = tid % kOptGroup;
             for (int r = grp; r < R; r += NT / kOptGroup)
-                two_opt_route<false>(p, L, r, L.zpos[r], L.zpos[r + 1] - 1, gl, ev, moves);
+                two_opt_route<false, RT>(p, L, r, L.zpos[r], L.zpos[r + 1] - 1, gl, ev, moves);
         }
         __syncthreads();
     }
@@ -1704,7 +1741,7 @@ __device__ void local_search_ant(const DevProblem &p, const DevState &s, int a, 
                 const int rbeg = L.zpos[grp], rend = L.zpos[grp + 1] - 1;
                 if (gl == 0) route_permutation(L, rbeg, rend - rbeg + 1, pm_jump(zant, (unsigned long long)rbeg));
                 group_sync();
-                two_opt_route_pair<true>(p, L, grp, rbeg, rend, gl, ev, moves);
+                two_opt_route_pair<true, RT>(p, L, grp, rbeg, rend, gl, ev, moves);
             }
         } else {
             const int grp = tid / kOptGroup, gl = tid % kOptGroup;
@@ -1712,7 +1749,7 @@ __device__ void local_search_ant(const DevProblem &p, const DevState &s, int a, 
                 const int rbeg = L.zpos[r], rend = L.zpos[r + 1] - 1;
                 if (gl == 0) route_permutation(L, rbeg, rend - rbeg + 1, pm_jump(zant, (unsigned long long)rbeg));
                 group_sync();
-                two_opt_route<true>(p, L, r, rbeg, rend, gl, ev, moves);
+                two_opt_route<true, RT>(p, L, r, rbeg, rend, gl, ev, moves);
             }
         }
         __syncthreads();
