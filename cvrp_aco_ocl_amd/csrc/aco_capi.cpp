@@ -28,31 +28,6 @@ int set_error(int code, const std::string &msg)
     return code;
 }
 
-static uint64_t splitmix64(uint64_t x)
-{
-    uint64_t z = x + 0x9E3779B97F4A7C15ull;
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    return z ^ (z >> 31);
-}
-
-// Lane seed: 1 + splitmix64(seed + golden * (1 + 64*ant + lane)) mod (2^31-2).
-// (The reference derives lane seeds from time(NULL), g_aco.cpp:715-719.)
-// Seed of the random-order 2-opt's scan-order stream (the reference draws
-// it from instance->rnd_seed, problem.cpp:213; here it follows the colony
-// seed).
-static int32_t ls_seed_of(uint64_t seed)
-{
-    return (int32_t)(1 + splitmix64(seed ^ 0xC2B2AE3D27D4EB4Full) % 2147483646ull);
-}
-
-static int32_t pm_seed(uint64_t seed, int ant, int lane)
-{
-    const uint64_t z = splitmix64(seed + 0x9E3779B97F4A7C15ull *
-                                  (uint64_t)(1 + (uint64_t)ant * kLanes + (uint64_t)lane));
-    return (int32_t)(1 + z % 2147483646ull);
-}
-
 }  // namespace cvrp
 
 using namespace cvrp;
@@ -70,7 +45,6 @@ struct InstanceData {
     int Q = 0;
     float D = INFINITY, svc = 0.0f;
     uint64_t seed = 0;
-    int32_t ls_seed0 = 1;     // initial state of the scan-order stream
     int setup_beta = 2;       // eta^beta on the device for beta 1 or 2 (0: uploaded)
     bool setup_prior = false, setup_int16 = false, nnl_given = false;
     DevProblem dp{};
@@ -564,7 +538,6 @@ int aco_create_batch(const aco_problem *pbs, int32_t count, const aco_params *pr
         I.D = pb->max_dist;
         I.svc = pb->service_time;
         I.seed = prm.seed + (uint64_t)b;
-        I.ls_seed0 = ls_seed_of(I.seed);
         const int P = I.P;
         const size_t bytes = carve_instance(I, m, k, nnP, ras, prm.bsf_capacity, nullptr);
         CHK(hipMalloc(&I.arena, bytes));
@@ -762,38 +735,17 @@ int aco_init(aco_ctx *c)
 {
     int rc = need(c, false);
     if (rc) return rc;
-    const int m = c->m;
-    static const int zeros[kCtrlWords] = {0};
-    static const long long zeros64[kTotWords] = {0};
-    static const float inf = INFINITY;
-    std::vector<std::vector<int32_t>> pms(c->inst.size());
-    for (size_t b = 0; b < c->inst.size(); ++b) {
-        InstanceData &I = c->inst[b];
-        std::vector<int32_t> &pm = pms[b];
-        pm.resize((size_t)m * kLanes);
-        for (int a = 0; a < m; ++a)
-            for (int l = 0; l < kLanes; ++l) pm[(size_t)a * kLanes + l] = pm_seed(I.seed, a, l);
-        HIP_TRY(hipMemcpyAsync(I.ds.pm, pm.data(), pm.size() * 4, hipMemcpyHostToDevice, c->stream));
-        HIP_TRY(hipMemcpyAsync(I.ds.ctrl, zeros, sizeof(zeros), hipMemcpyHostToDevice, c->stream));
-        HIP_TRY(hipMemcpyAsync(I.ds.ctrl + kCtrlLsSeed, &c->inst[b].ls_seed0, 4, hipMemcpyHostToDevice, c->stream));
-        HIP_TRY(hipMemcpyAsync(I.ds.totals, zeros64, sizeof(zeros64), hipMemcpyHostToDevice, c->stream));
-        HIP_TRY(hipMemcpyAsync(I.ds.lens + m, &inf, 4, hipMemcpyHostToDevice, c->stream));
-        HIP_TRY(hipMemsetAsync(I.ds.sizes + m, 0, 4, c->stream));
-    }
-    HIP_TRY(launch_stamp_clock(c->bt, c->stream));
+    HIP_TRY(launch_state_init(c->bt, c->m, c->stream));
     if (c->prm.tau0_rule == ACO_TAU0_FIRST_COLONY) {
         // g_aco.cpp:79-92: colony on tau = 0.5, then tau0 = 1/(rho * L_bsf)
         HIP_TRY(launch_pheromone_init(c->bt, kTau0Arg, 0.5f, c->stream));
-        if ((rc = run_gather(c))) return rc;
         if ((rc = run_construct(c))) return rc;
         if ((rc = run_statistics(c))) return rc;
         HIP_TRY(launch_pheromone_init(c->bt, kTau0Bsf, 0.0f, c->stream));
-        if ((rc = run_gather(c))) return rc;
     } else {
         HIP_TRY(launch_pheromone_init(c->bt, kTau0Nn, 0.0f, c->stream));
-        if ((rc = run_gather(c))) return rc;
     }
-    HIP_TRY(hipStreamSynchronize(c->stream));  // pm staging vectors go out of scope
+    HIP_TRY(hipStreamSynchronize(c->stream));
     c->inited = true;
     return ACO_OK;
 }
@@ -828,7 +780,7 @@ int aco_pheromone_init(aco_ctx *c, float tau0)
     if (rc) return rc;
     if (!(tau0 >= 0.0f) || !isfinite(tau0)) return set_error(ACO_ERR_ARG, "tau0 must be finite and >= 0");
     HIP_TRY(launch_pheromone_init(c->bt, kTau0Arg, tau0, c->stream));
-    return run_gather(c);
+    return ACO_OK;
 }
 
 int aco_iteration(aco_ctx *c)
