@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -73,6 +74,8 @@ struct aco_ctx {
     int max_n = 0;
     bool int16_rows = true;   // every distance an integer in [0, 65535]
     void *setup_scratch = nullptr;   // candidate lists during aco_create
+    int32_t *best = nullptr;         // pinned: size, length and tour of a best-so-far slot (2 + 2 max_n words)
+    std::mutex best_mutex;           // held from the launch that fills it until it has been read
 };
 
 #define HIP_TRY(expr)                                                                      \
@@ -719,6 +722,7 @@ int aco_destroy(aco_ctx *c)
     if (c->graph) (void)hipGraphDestroy(c->graph);
     for (void *p : c->allocs) (void)hipFree(p);
     if (c->setup_scratch) (void)hipFree(c->setup_scratch);
+    if (c->best) (void)hipHostFree(c->best);
     for (int i = 0; i < c->lss.count; ++i) {
         (void)hipStreamDestroy(c->lss.aux[i]);
         (void)hipEventDestroy(c->lss.join[i]);
@@ -837,19 +841,16 @@ int aco_get_best_at(aco_ctx *c, int32_t b, int32_t *tour, int32_t cap, int32_t *
 {
     int rc = need_inst(c, b, true);
     if (rc) return rc;
-    const InstanceData &I = c->inst[b];
-    int sz = 0;
-    float L = 0.0f;
-    HIP_TRY(hipMemcpyAsync(&sz, I.ds.sizes + c->m, 4, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipMemcpyAsync(&L, I.ds.lens + c->m, 4, hipMemcpyDeviceToHost, c->stream));
+    const std::lock_guard<std::mutex> lock(c->best_mutex);
+    if (!c->best) HIP_TRY(hipHostMalloc((void **)&c->best, (size_t)(2 + 2 * c->max_n) * 4, hipHostMallocDefault));
+    HIP_TRY(launch_best_pack(c->bt, b, c->best, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
+    const int sz = c->best[0];
     if (size) *size = sz;
-    if (len) *len = L;
+    if (len) memcpy(len, c->best + 1, 4);
     if (tour) {
         if (cap < sz) return set_error(ACO_ERR_ARG, "tour buffer too small");
-        HIP_TRY(hipMemcpyAsync(tour, I.ds.tours + (size_t)c->m * I.T, (size_t)sz * 4,
-                               hipMemcpyDeviceToHost, c->stream));
-        HIP_TRY(hipStreamSynchronize(c->stream));
+        memcpy(tour, c->best + 2, (size_t)sz * 4);
     }
     return ACO_OK;
 }

@@ -275,6 +275,7 @@ hipError_t launch_pheromone_update(const DevBatch &b, hipStream_t st);
 hipError_t launch_gather(const DevBatch &b, hipStream_t st);
 hipError_t launch_pheromone_init(const DevBatch &b, int mode, float tau0, hipStream_t st);
 hipError_t launch_state_init(const DevBatch &b, int m, hipStream_t st);
+hipError_t launch_best_pack(const DevBatch &b, int inst, int *out, hipStream_t st);
 hipError_t launch_stamp_clock(const DevBatch &b, hipStream_t st);
 size_t construct_lds_bytes(int n, int selection);
 size_t local_search_lds_bytes(int n, int ring, int row16, int flags);
