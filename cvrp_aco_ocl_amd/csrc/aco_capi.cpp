@@ -53,6 +53,114 @@ struct InstanceData {
     void *arena = nullptr;
 };
 
+// Device-to-host copies through two pinned buffers in turn.  The pieces of
+// one readback are packed into a buffer; when it is full it is copied out
+// while the other one is being filled.  A pitched matrix travels with its
+// padding, as one run of bytes, and loses it on the way out: the runtime's
+// 2-D copies go row by row (7 us each: 14 ms for two matrices of 1001 rows)
+// into pageable memory, and into any memory where the rows are not whole
+// words; this takes 0.4 ms.  Several small arrays need one wait.
+// 512 KB a buffer: the runtime keeps freed pinned blocks of this size, so
+// neither this context nor the next one pays for pinning (with 1 or 2 MB
+// aco_create of a 242-node instance after another context's end took 1.56
+// instead of 0.88 ms), and a chunk's transfer still covers its launch.
+// Reading 243 tours of 242 nodes: 2.1 -> 0.08 ms.
+// One context, one readback at a time (the mutex); the buffers are made by
+// the first readback and live as long as the context.
+struct Readback {
+    static constexpr size_t kBytes = size_t(512) << 10;
+    struct Piece {
+        unsigned char *dst;
+        size_t dpitch, pitch, width, rows, off;
+    };
+    std::mutex mutex;
+    unsigned char *buf[2] = {nullptr, nullptr};
+    hipEvent_t done[2] = {nullptr, nullptr};
+    std::vector<Piece> pieces[2];
+    size_t used = 0;
+    int cur = 0;
+
+    hipError_t init()
+    {
+        for (int i = 0; i < 2; ++i) {
+            hipError_t e = hipSuccess;
+            if (!buf[i]) e = hipHostMalloc((void **)&buf[i], kBytes, hipHostMallocDefault);
+            if (e == hipSuccess && !done[i]) e = hipEventCreateWithFlags(&done[i], hipEventDisableTiming);
+            if (e != hipSuccess) return e;
+            pieces[i].clear();
+        }
+        used = 0;
+        return hipSuccess;
+    }
+    ~Readback()
+    {
+        for (int i = 0; i < 2; ++i) {
+            if (done[i]) (void)hipEventDestroy(done[i]);
+            if (buf[i]) (void)hipHostFree(buf[i]);
+        }
+    }
+    // waits for buffer i's transfers and copies its pieces out
+    hipError_t drain(int i)
+    {
+        if (pieces[i].empty()) return hipSuccess;
+        const hipError_t e = hipEventSynchronize(done[i]);
+        if (e != hipSuccess) return e;
+        for (const Piece &p : pieces[i]) {
+            if (p.dpitch == p.width && p.pitch == p.width) memcpy(p.dst, buf[i] + p.off, p.width * p.rows);
+            else
+                for (size_t r = 0; r < p.rows; ++r)
+                    memcpy(p.dst + r * p.dpitch, buf[i] + p.off + r * p.pitch, p.width);
+        }
+        pieces[i].clear();
+        return hipSuccess;
+    }
+    // the current buffer is full: copy the other one out, then fill it
+    hipError_t turn(hipStream_t st)
+    {
+        hipError_t e = hipEventRecord(done[cur], st);
+        if (e != hipSuccess) return e;
+        cur ^= 1;
+        used = 0;
+        return drain(cur);
+    }
+    // `rows` rows of `width` bytes, device pitch spitch (at most kBytes, and
+    // the last row's padding is allocated too), to host rows of pitch dpitch
+    hipError_t get2d(void *dst, size_t dpitch, const void *src, size_t spitch, size_t width, size_t rows, hipStream_t st)
+    {
+        unsigned char *d = static_cast<unsigned char *>(dst);
+        const unsigned char *s = static_cast<const unsigned char *>(src);
+        if (!width) return hipSuccess;
+        while (rows) {
+            hipError_t e = hipSuccess;
+            if (used + spitch > kBytes && (e = turn(st)) != hipSuccess) return e;
+            const size_t nr = std::min(rows, (kBytes - used) / spitch);
+            e = hipMemcpyAsync(buf[cur] + used, s, spitch * nr, hipMemcpyDeviceToHost, st);
+            if (e != hipSuccess) return e;
+            pieces[cur].push_back({d, dpitch, spitch, width, nr, used});
+            used = (used + spitch * nr + 63) & ~size_t(63);
+            d += nr * dpitch;
+            s += nr * spitch;
+            rows -= nr;
+        }
+        return hipSuccess;
+    }
+    // contiguous bytes (taken as rows of at most 64 KB)
+    hipError_t get(void *dst, const void *src, size_t bytes, hipStream_t st)
+    {
+        const size_t w = size_t(64) << 10, rows = bytes / w, rest = bytes - rows * w;
+        hipError_t e = get2d(dst, w, src, w, w, rows, st);
+        if (e != hipSuccess) return e;
+        return get2d(static_cast<unsigned char *>(dst) + rows * w, rest, static_cast<const unsigned char *>(src) + rows * w,
+                     rest, rest, 1, st);
+    }
+    hipError_t finish(hipStream_t st)
+    {
+        hipError_t e = drain(cur ^ 1);
+        if (e == hipSuccess) e = hipEventRecord(done[cur], st);
+        return e == hipSuccess ? drain(cur) : e;
+    }
+};
+
 struct aco_ctx {
     aco_params prm{};
     int m = 0, device = 0;
@@ -74,8 +182,7 @@ struct aco_ctx {
     int max_n = 0;
     bool int16_rows = true;   // every distance an integer in [0, 65535]
     void *setup_scratch = nullptr;   // candidate lists during aco_create
-    int32_t *best = nullptr;         // pinned: size, length and tour of a best-so-far slot (2 + 2 max_n words)
-    std::mutex best_mutex;           // held from the launch that fills it until it has been read
+    Readback rb;
 };
 
 #define HIP_TRY(expr)                                                                      \
@@ -293,6 +400,19 @@ static int run_iteration_steps(aco_ctx *c)
     if ((rc = run_local_search(c)) != ACO_OK) return rc;
     if ((rc = run_statistics(c)) != ACO_OK) return rc;
     return run_pheromone(c);
+}
+
+// fn(readback, stream) requests the copies; everything has arrived on return.
+template <typename F>
+static int read_back(aco_ctx *c, F &&fn)
+{
+    const std::lock_guard<std::mutex> lock(c->rb.mutex);
+    HIP_TRY(c->rb.init());
+    hipError_t e = fn(c->rb, c->stream);
+    if (e == hipSuccess) e = c->rb.finish(c->stream);
+    if (e != hipSuccess) (void)hipStreamSynchronize(c->stream);   // no transfer stays in flight
+    HIP_TRY(e);
+    return ACO_OK;
 }
 
 static int need(aco_ctx *c, bool inited)
@@ -722,7 +842,6 @@ int aco_destroy(aco_ctx *c)
     if (c->graph) (void)hipGraphDestroy(c->graph);
     for (void *p : c->allocs) (void)hipFree(p);
     if (c->setup_scratch) (void)hipFree(c->setup_scratch);
-    if (c->best) (void)hipHostFree(c->best);
     for (int i = 0; i < c->lss.count; ++i) {
         (void)hipStreamDestroy(c->lss.aux[i]);
         (void)hipEventDestroy(c->lss.join[i]);
@@ -841,16 +960,18 @@ int aco_get_best_at(aco_ctx *c, int32_t b, int32_t *tour, int32_t cap, int32_t *
 {
     int rc = need_inst(c, b, true);
     if (rc) return rc;
-    const std::lock_guard<std::mutex> lock(c->best_mutex);
-    if (!c->best) HIP_TRY(hipHostMalloc((void **)&c->best, (size_t)(2 + 2 * c->max_n) * 4, hipHostMallocDefault));
-    HIP_TRY(launch_best_pack(c->bt, b, c->best, c->stream));
+    const std::lock_guard<std::mutex> lock(c->rb.mutex);
+    HIP_TRY(c->rb.init());
+    static_assert((2 + 2 * kMaxNodes) * 4 <= Readback::kBytes, "a tour fits one buffer");
+    int32_t *best = reinterpret_cast<int32_t *>(c->rb.buf[0]);
+    HIP_TRY(launch_best_pack(c->bt, b, best, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
-    const int sz = c->best[0];
+    const int sz = best[0];
     if (size) *size = sz;
-    if (len) memcpy(len, c->best + 1, 4);
+    if (len) memcpy(len, best + 1, 4);
     if (tour) {
         if (cap < sz) return set_error(ACO_ERR_ARG, "tour buffer too small");
-        memcpy(tour, c->best + 2, (size_t)sz * 4);
+        memcpy(tour, best + 2, (size_t)sz * 4);
     }
     return ACO_OK;
 }
@@ -866,15 +987,14 @@ int aco_get_ants_at(aco_ctx *c, int32_t b, int32_t *tours, int32_t stride, int32
     if (rc) return rc;
     const InstanceData &I = c->inst[b];
     const int m1 = c->m + 1;
-    if (tours) {
-        if (stride < I.T) return set_error(ACO_ERR_ARG, "stride must be >= 2n");
-        HIP_TRY(hipMemcpy2DAsync(tours, (size_t)stride * 4, I.ds.tours, (size_t)I.T * 4, (size_t)I.T * 4, m1,
-                                 hipMemcpyDeviceToHost, c->stream));
-    }
-    if (sizes) HIP_TRY(hipMemcpyAsync(sizes, I.ds.sizes, (size_t)m1 * 4, hipMemcpyDeviceToHost, c->stream));
-    if (lens) HIP_TRY(hipMemcpyAsync(lens, I.ds.lens, (size_t)m1 * 4, hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return ACO_OK;
+    if (tours && stride < I.T) return set_error(ACO_ERR_ARG, "stride must be >= 2n");
+    return read_back(c, [&](Readback &rb, hipStream_t st) {
+        const size_t w = (size_t)I.T * 4;
+        hipError_t e = tours ? rb.get2d(tours, (size_t)stride * 4, I.ds.tours, w, w, m1, st) : hipSuccess;
+        if (e == hipSuccess && sizes) e = rb.get(sizes, I.ds.sizes, (size_t)m1 * 4, st);
+        if (e == hipSuccess && lens) e = rb.get(lens, I.ds.lens, (size_t)m1 * 4, st);
+        return e;
+    });
 }
 
 int aco_get_ants(aco_ctx *c, int32_t *tours, int32_t stride, int32_t *sizes, float *lens)
@@ -1033,12 +1153,12 @@ int aco_get_pheromone_at(aco_ctx *c, int32_t b, float *tau, float *ti)
     int rc = need_inst(c, b, false);
     if (rc) return rc;
     const InstanceData &I = c->inst[b];
-    if (tau) HIP_TRY(hipMemcpy2DAsync(tau, (size_t)I.n * 4, I.ds.tau, (size_t)I.P * 4, (size_t)I.n * 4, I.n,
-                                      hipMemcpyDeviceToHost, c->stream));
-    if (ti) HIP_TRY(hipMemcpy2DAsync(ti, (size_t)I.n * 4, I.ds.tinfo, (size_t)I.P * 4, (size_t)I.n * 4, I.n,
-                                     hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return ACO_OK;
+    return read_back(c, [&](Readback &rb, hipStream_t st) {
+        const size_t w = (size_t)I.n * 4, pitch = (size_t)I.P * 4;
+        hipError_t e = tau ? rb.get2d(tau, w, I.ds.tau, pitch, w, I.n, st) : hipSuccess;
+        if (e == hipSuccess && ti) e = rb.get2d(ti, w, I.ds.tinfo, pitch, w, I.n, st);
+        return e;
+    });
 }
 
 int aco_get_pheromone(aco_ctx *c, float *tau, float *ti) { return aco_get_pheromone_at(c, 0, tau, ti); }
@@ -1049,10 +1169,10 @@ int aco_set_pheromone_at(aco_ctx *c, int32_t b, const float *tau, const float *t
     if (rc) return rc;
     if (!tau || !ti) return set_error(ACO_ERR_ARG, "null argument");
     const InstanceData &I = c->inst[b];
-    HIP_TRY(hipMemcpy2DAsync(I.ds.tau, (size_t)I.P * 4, tau, (size_t)I.n * 4, (size_t)I.n * 4, I.n,
-                             hipMemcpyHostToDevice, c->stream));
-    HIP_TRY(hipMemcpy2DAsync(I.ds.tinfo, (size_t)I.P * 4, ti, (size_t)I.n * 4, (size_t)I.n * 4, I.n,
-                             hipMemcpyHostToDevice, c->stream));
+    PinnedStager up;
+    HIP_TRY(up.init(c->stream, Readback::kBytes));
+    HIP_TRY(up.put2d(I.ds.tau, (size_t)I.P * 4, tau, (size_t)I.n * 4, I.n));
+    HIP_TRY(up.put2d(I.ds.tinfo, (size_t)I.P * 4, ti, (size_t)I.n * 4, I.n));
     if ((rc = run_gather(c))) return rc;
     HIP_TRY(hipStreamSynchronize(c->stream));
     return ACO_OK;
@@ -1078,24 +1198,21 @@ int aco_get_setup_at(aco_ctx *c, int32_t b, float *heur, float *d0, int32_t *nnk
     const InstanceData &I = c->inst[b];
     const DevProblem &dp = I.dp;
     const int n = I.n, k = c->prm.k, nl = dp.nn_ls;
-    if (heur)
-        HIP_TRY(hipMemcpy2DAsync(heur, (size_t)n * 4, dp.heur, (size_t)I.P * 4, (size_t)n * 4, n, hipMemcpyDeviceToHost,
-                                 c->stream));
-    if (d0) HIP_TRY(hipMemcpyAsync(d0, dp.d0, (size_t)n * 4, hipMemcpyDeviceToHost, c->stream));
-    if (nnk && k > 0) HIP_TRY(hipMemcpyAsync(nnk, dp.nnk, (size_t)n * k * 4, hipMemcpyDeviceToHost, c->stream));
-    if (nnkd && k > 0) HIP_TRY(hipMemcpyAsync(nnkd, dp.nnkd, (size_t)n * k * 4, hipMemcpyDeviceToHost, c->stream));
-    if (nnls)
-        HIP_TRY(hipMemcpy2DAsync(nnls, (size_t)nl * 4, dp.nnls, (size_t)dp.nnP * 4, (size_t)nl * 4, n,
-                                 hipMemcpyDeviceToHost, c->stream));
-    if (nnd)
-        HIP_TRY(hipMemcpy2DAsync(nnd, (size_t)nl * 4, dp.nnd, (size_t)dp.nnP * 4, (size_t)nl * 4, n,
-                                 hipMemcpyDeviceToHost, c->stream));
-    if (nnpos) HIP_TRY(hipMemcpyAsync(nnpos, dp.nnpos, (size_t)n * n * 2, hipMemcpyDeviceToHost, c->stream));
-    if (dist16 && c->int16_rows)
-        HIP_TRY(hipMemcpy2DAsync(dist16, (size_t)n * 2, dp.dist16, (size_t)I.P * 2, (size_t)n * 2, n,
-                                 hipMemcpyDeviceToHost, c->stream));
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    return ACO_OK;
+    return read_back(c, [&](Readback &rb, hipStream_t st) {
+        hipError_t e = hipSuccess;
+        auto rows = [&](void *dst, const void *src, size_t pitch, size_t width) {
+            if (e == hipSuccess && dst) e = rb.get2d(dst, width, src, pitch, width, n, st);
+        };
+        rows(heur, dp.heur, (size_t)I.P * 4, (size_t)n * 4);
+        if (e == hipSuccess && d0) e = rb.get(d0, dp.d0, (size_t)n * 4, st);
+        rows(nnk, dp.nnk, (size_t)k * 4, (size_t)k * 4);
+        rows(nnkd, dp.nnkd, (size_t)k * 4, (size_t)k * 4);
+        rows(nnls, dp.nnls, (size_t)dp.nnP * 4, (size_t)nl * 4);
+        rows(nnd, dp.nnd, (size_t)dp.nnP * 4, (size_t)nl * 4);
+        rows(nnpos, dp.nnpos, (size_t)n * 2, (size_t)n * 2);
+        if (c->int16_rows) rows(dist16, dp.dist16, (size_t)I.P * 2, (size_t)n * 2);
+        return e;
+    });
 }
 
 int aco_set_candidates_at(aco_ctx *c, int32_t b, const int32_t *cand, int32_t width)
