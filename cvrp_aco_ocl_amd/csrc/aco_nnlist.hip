@@ -1,7 +1,7 @@
 // Candidate (nearest-neighbour) lists of many instances on the GPU:
-// compute_nn_lists (vrpHelper.cpp:188-236), one thread per row, the row
-// sorted in LDS (k_nn_lists; at most 60 KB and 64 rows per block) or,
-// for the entry point that allocates nothing, in a global scratch array.
+// compute_nn_lists (vrpHelper.cpp:188-236), one wave per row, the row
+// sorted in LDS (k_nn_lists), or, for the entry point that allocates
+// nothing, one thread per row in a global scratch array.
 //
 // Each row is sorted with the reference's own steps, sort2
 // (utilities.cpp:246-267): the middle element is swapped to the front as
@@ -85,14 +85,86 @@ __device__ void nn_sort_row(float *v, I *ix, int n, int tie)
     }
 }
 
-// One row per thread, sorted in LDS: keys as floats, node ids as 16-bit
-// values (n <= 4096), row r of the block at r * nmax.  The rows of a block
-// may belong to different instances.
-__global__ __launch_bounds__(64) void k_nn_lists(const NnJob *jobs, int njobs, int rows, int tie, int nmax)
+// ---- one row per wave, in LDS ----
+//
+// A pass over [l, r] with its pivot in front swaps the j-th smaller element
+// (position s_j) with position l + j.  All its swaps are made at once:
+// smaller element j ends at l + j, and what stands at l + j moves to s_j, so
+// another element at p moves to s_(p-l) for as long as p <= l + m (m smaller
+// elements), each hop further right.  The hops of all elements together are
+// at most m, and about log(r - l) for one element unless nearly all are
+// smaller.  Every element lands where the sequential swaps put it, equal
+// distances included.
+//
+// Parts of more than kNnSmall elements are split this way, 64 elements at a
+// time; smaller ones are handed to the lanes, which sort 64 of them side by
+// side with the sequential steps.  One thread per row, as before, is a chain
+// of n log2(n) LDS round trips: 1001 rows of 1001 nodes 3.58 ms, now 0.28 ms,
+// bound by the latency of about 2n/kNnSmall passes per wave.
+constexpr int kNnSmall = 32;
+constexpr int kNnRowBytes = 4 + 2 + 4 + 2 + 2;   // keys, ids, a second copy of both, s_j
+
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// sort2 on at most kNnSmall elements; parts waiting are packed in a word, 10
+// bits each (at most log2(kNnSmall) + 1 = 6 of them).
+__device__ __forceinline__ void nn_sort_small(float *v, unsigned short *ix, int n, int tie)
+{
+    static_assert(kNnSmall == 32, "two 5-bit bounds per waiting part");
+    unsigned long long waiting = 0;
+    int count = 0, l = 0, r = n - 1;
+    for (;;) {
+        if (l >= r) {
+            if (count == 0) return;
+            --count;
+            l = (int)(waiting >> 5) & 31;
+            r = (int)waiting & 31;
+            waiting >>= 10;
+            continue;
+        }
+        const int mid = (l + r) / 2;
+        const float pv = v[mid];
+        const unsigned short pi = ix[mid];
+        v[mid] = v[l];
+        ix[mid] = ix[l];
+        int last = l;
+        for (int k = l + 1; k <= r; ++k) {
+            const float vk = v[k];
+            const unsigned short ik = ix[k];
+            if (nn_less(vk, ik, pv, pi, tie)) {
+                ++last;
+                v[k] = v[last];
+                ix[k] = ix[last];
+                v[last] = vk;
+                ix[last] = ik;
+            }
+        }
+        v[l] = v[last];
+        ix[l] = ix[last];
+        v[last] = pv;
+        ix[last] = pi;
+        int wl = l, wr = last;
+        if (last - l + 1 < r - last) {
+            wl = last + 1;
+            wr = r;
+            r = last;
+        } else {
+            l = last + 1;
+        }
+        waiting = waiting << 10 | (unsigned long long)(wl << 5 | wr);
+        ++count;
+    }
+}
+
+__global__ __launch_bounds__(64) void k_nn_lists(const NnJob *jobs, int njobs, int tie, int nmax)
 {
     extern __shared__ __align__(16) unsigned char smem[];
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= rows) return;
+    __shared__ int stack[2 * kNnStack];
+    const int row = blockIdx.x, lane = threadIdx.x;
     int lo = 0, hi = njobs - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) / 2;
@@ -102,42 +174,109 @@ __global__ __launch_bounds__(64) void k_nn_lists(const NnJob *jobs, int njobs, i
     const NnJob J = jobs[lo];
     const int node = row - J.first_row, n = J.n;
     const float *d = J.dist + (size_t)node * J.dpitch;
-    float *v = reinterpret_cast<float *>(smem) + (size_t)threadIdx.x * nmax;
-    unsigned short *ix = reinterpret_cast<unsigned short *>(smem + (size_t)blockDim.x * nmax * 4) +
-                         (size_t)threadIdx.x * nmax;
-    for (int i = 0; i < n; ++i) {
-        v[i] = d[i];
+    float *v = reinterpret_cast<float *>(smem), *v2 = v + nmax;
+    unsigned short *ix = reinterpret_cast<unsigned short *>(v2 + nmax), *ix2 = ix + nmax, *sp = ix2 + nmax;
+    for (int i = lane; i < n; i += 64) {
+        // a node is not its own neighbour, nor is the depot anyone's
+        v[i] = i == node || i == 0 ? INFINITY : d[i];
         ix[i] = (unsigned short)i;
     }
-    v[node] = INFINITY;   // a node is not its own neighbour
-    v[0] = INFINITY;      // nor is the depot anyone's
-    nn_sort_row(v, ix, n, tie);
-    for (int h = 0; h < J.width; ++h) J.out[(size_t)node * J.width + h] = ix[h];
-}
-
-// Rows per block of k_nn_lists for `rows` rows of at most nmax nodes: the
-// rows of a wave run their sorts side by side (divergent), so a row gets a
-// wave of its own while there are fewer rows than SIMDs (4 per CU), and
-// rows are packed up to 64 per wave beyond that, within 60 KB of LDS per
-// block (6 bytes per row element).
-static int nn_rows_per_block(int rows, int nmax, int cus)
-{
-    const int simds = 4 * (cus > 0 ? cus : 1);
-    int r = (rows + simds - 1) / simds;
-    const int cap = (60 << 10) / (6 * nmax);
-    r = r > cap ? cap : r;
-    return r < 1 ? 1 : (r > 64 ? 64 : r);
+    wave_lds_sync();
+    int waiting = 0, l = 0, r = n - 1;   // uniform
+    int small = 0, sl = 0, sn = 0;       // lane q < small: the part of sn elements at sl
+    for (;;) {
+        if (r - l + 1 <= kNnSmall) {
+            if (r > l) {
+                if (lane == small) {
+                    sl = l;
+                    sn = r - l + 1;
+                }
+                ++small;
+            }
+            if (small == 64 || waiting == 0) {
+                if (lane < small) nn_sort_small(v + sl, ix + sl, sn, tie);
+                wave_lds_sync();
+                small = 0;
+            }
+            if (waiting == 0) break;
+            --waiting;
+            l = __builtin_amdgcn_readfirstlane(stack[2 * waiting]);
+            r = __builtin_amdgcn_readfirstlane(stack[2 * waiting + 1]);
+            continue;
+        }
+        const int mid = (l + r) / 2;
+        const float pv = v[mid], fv = v[l];
+        const unsigned short pi = ix[mid], fi = ix[l];
+        wave_lds_sync();
+        if (lane == 0) {
+            v[mid] = fv;
+            ix[mid] = fi;
+        }
+        wave_lds_sync();
+        // s_1 .. s_m, relative to l
+        int m = 0;
+        for (int k0 = l + 1; k0 <= r; k0 += 64) {
+            const int k = k0 + lane;
+            const bool less = k <= r && nn_less(v[k <= r ? k : r], ix[k <= r ? k : r], pv, pi, tie);
+            const unsigned long long b = __ballot(less);
+            if (less) sp[m + __popcll(b & ((1ull << lane) - 1ull)) + 1] = (unsigned short)(k - l);
+            m += __popcll(b);
+        }
+        wave_lds_sync();
+        // every element but the pivot to its place (the m-th smaller one and
+        // the pivot change places at the end: l and l + m)
+        int before = 0;
+        for (int k0 = l + 1; k0 <= r; k0 += 64) {
+            const int k = k0 + lane, kk = k <= r ? k : r;
+            const float vk = v[kk];
+            const unsigned short ik = ix[kk];
+            const bool less = k <= r && nn_less(vk, ik, pv, pi, tie);
+            const unsigned long long b = __ballot(less);
+            if (k <= r) {
+                int q = k - l;
+                if (less) {
+                    q = before + __popcll(b & ((1ull << lane) - 1ull)) + 1;
+                    if (q == m) q = 0;
+                } else {
+                    while (q <= m) q = sp[q];
+                }
+                v2[l + q] = vk;
+                ix2[l + q] = ik;
+            }
+            before += __popcll(b);
+        }
+        if (lane == 0) {
+            v2[l + m] = pv;
+            ix2[l + m] = pi;
+        }
+        wave_lds_sync();
+        for (int k = l + lane; k <= r; k += 64) {
+            v[k] = v2[k];
+            ix[k] = ix2[k];
+        }
+        const int last = l + m;
+        int wl = l, wr = last;
+        if (last - l + 1 < r - last) {
+            wl = last + 1;
+            wr = r;
+            r = last;
+        } else {
+            l = last + 1;
+        }
+        if (lane == 0) {
+            stack[2 * waiting] = wl;
+            stack[2 * waiting + 1] = wr;
+        }
+        ++waiting;
+        wave_lds_sync();
+    }
+    for (int h = lane; h < J.width; h += 64) J.out[(size_t)node * J.width + h] = ix[h];
 }
 
 static hipError_t launch_nn_lists(const NnJob *djobs, int nj, int rows, int tie, int nmax, hipStream_t st)
 {
-    int dev = 0, cus = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess) return e;
-    const int rpb = nn_rows_per_block(rows, nmax, cus);
-    const size_t lds = (size_t)rpb * nmax * 6;
-    hipLaunchKernelGGL(k_nn_lists, dim3((rows + rpb - 1) / rpb), dim3(rpb), lds, st, djobs, nj, rows, tie, nmax);
+    static_assert(kMaxNodes * kNnRowBytes + 8 * kNnStack <= (64 << 10), "a row fits a block's LDS");
+    hipLaunchKernelGGL(k_nn_lists, dim3(rows), dim3(64), (size_t)nmax * kNnRowBytes, st, djobs, nj, tie, nmax);
     return hipGetLastError();
 }
 
