@@ -11,10 +11,13 @@ size_t local_search_lds_bytes(int n, int ring, int row16, int flags)
 }
 
 // With 4 or 8 waves per ant several ants share a CU: registers are held to
-// 128 per lane so that four waves fit each SIMD (not for the random-order
-// 2-opt instantiations, which would spill).
+// 96 (4 waves) or 128 per lane, so that five or four waves fit each SIMD (not
+// for the random-order 2-opt instantiations, which would spill).  Five ants
+// of 4 waves per CU instead of four: 20 instances of 64 ants at 151 nodes
+// 0.76 -> 0.55 ms (1280 ants, one round instead of two), 256 instances 9.4 ->
+// 8.8 ms.  Six (80 registers) spill: 0.56 and 8.9 ms.
 template <int W, typename RT, bool R2>
-__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(W <= 8 && !R2 ? 4 : 1)))
+__global__ __launch_bounds__(W * 64) __attribute__((amdgpu_waves_per_eu(R2 || W > 8 ? 1 : W == 4 ? 5 : 4)))
 void k_local_search(DevBatch bt, int first, int flags, int ring, int prefetch)
 {
     extern __shared__ __align__(16) unsigned char smem[];

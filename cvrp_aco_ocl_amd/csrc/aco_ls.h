@@ -177,18 +177,15 @@ __device__ __forceinline__ int ls_routes(const DevProblem &p, LsLds &L, int S, i
 // with the reversals split over the lanes.
 constexpr int kOptGroup = 8;
 
-// Minimum over the aligned group of 8 lanes (lane ^ 1, ^ 2, ^ 4 stay inside
-// the group, all of whose lanes are active).
-__device__ __forceinline__ u64 group_min_u64(u64 v)
+// Minimum over the aligned group of 8 lanes, all of them active (within
+// pairs, within quads, then with the mirrored lane of the other quad).
+__device__ __forceinline__ unsigned group_min_u32(unsigned v)
 {
     static_assert(kOptGroup == 8, "the DPP exchanges cover groups of 8 lanes");
-    const int lane = (int)(threadIdx.x & 63);
-    u64 w = dpp_u64<kDppXor1>(v);
-    v = w < v ? w : v;
-    w = dpp_u64<kDppXor2>(v);
-    v = w < v ? w : v;
-    w = dpp_xor4_u64(v, lane);
-    return w < v ? w : v;
+    auto low = [](unsigned a, int b) { return a < (unsigned)b ? a : (unsigned)b; };
+    v = low(v, __builtin_amdgcn_mov_dpp((int)v, kDppXor1, 0xF, 0xF, true));
+    v = low(v, __builtin_amdgcn_mov_dpp((int)v, kDppXor2, 0xF, 0xF, true));
+    return low(v, __builtin_amdgcn_mov_dpp((int)v, kDppHalfMirror, 0xF, 0xF, true));
 }
 
 __device__ __forceinline__ void group_sync()
@@ -223,8 +220,9 @@ __device__ __forceinline__ void group_sync()
 // position only where a candidate improves measured slower (12.9 ms, 64
 // us): it puts a second latency behind the first.
 // ok*: in the row (rp < nn_ls), inside the radius and, for the predecessor
-// scan, not adjacent; gains as the reference computes them; xs = s2,
-// xp = p2.
+// scan, not adjacent; gains as the reference computes them.  Nodes are not
+// kept past the requests (the accepted candidate's are read again from its
+// position): the scan is where the kernel needs most registers.
 template <typename RT>
 __device__ __forceinline__ float opt_dist(const DevProblem &p, int a, int b)
 {
@@ -235,7 +233,7 @@ __device__ __forceinline__ float opt_dist(const DevProblem &p, int a, int b)
 template <int U> struct OptCands {
     bool oks[U], okp[U];
     float gs[U], gp[U];
-    int rp[U], n2[U], xs[U], xp[U];
+    int rp[U];
 };
 
 // Rows of n1, its successor and its predecessor in the distance matrix, and
@@ -270,39 +268,45 @@ template <typename RT> __device__ __forceinline__ const RT *opt_matrix(const Dev
 }
 
 template <typename RT, int U>
-__device__ __forceinline__ void two_opt_cands(const DevProblem &p, const LsLds &L, int rend, int pos1, int q0, int n1,
-                                              int p1, float rads, float radp, const OptRows<RT> &row,
-                                              OptCands<U> &c)
+__device__ __forceinline__ void two_opt_cands(const DevProblem &p, const LsLds &L, int rbeg, int rend, int pos1, int q0,
+                                              float rads, float radp, const OptRows<RT> &row, OptCands<U> &c)
 {
     RT dn[U], dxs[U], dxp[U];
     float ews[U], ewp[U];
+    int n2[U], xs[U], xp[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int q = q0 + u * kOptGroup, qq = q <= rend ? q : rend;
-        c.xp[u] = L.tour[qq - 1];
-        c.n2[u] = L.tour[qq];
-        c.xs[u] = L.tour[qq + 1];   // past the route's end: the next depot
-        ewp[u] = L.dtw[qq - 1];
-        ews[u] = L.dtw[qq];
+        xp[u] = L.tour[qq - 1];
+        n2[u] = L.tour[qq];
+        xs[u] = L.tour[qq + 1];   // past the route's end: the next depot
     }
     loads_issued();
     const RT *m = opt_matrix<RT>(p);
     constexpr int sz = sizeof(RT);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        dn[u] = gload_at(m, row.d1 + (unsigned)c.n2[u] * sz);
-        dxs[u] = gload_at(m, row.ds + (unsigned)c.xs[u] * sz);
-        dxp[u] = gload_at(m, row.dp + (unsigned)c.xp[u] * sz);
-        c.rp[u] = gload_at(p.nnpos, row.pos + (unsigned)c.n2[u] * 2);
+        dn[u] = gload_at(m, row.d1 + (unsigned)n2[u] * sz);
+        dxs[u] = gload_at(m, row.ds + (unsigned)xs[u] * sz);
+        dxp[u] = gload_at(m, row.dp + (unsigned)xp[u] * sz);
+        c.rp[u] = gload_at(p.nnpos, row.pos + (unsigned)n2[u] * 2);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int q = q0 + u * kOptGroup, qq = q <= rend ? q : rend;
+        ewp[u] = L.dtw[qq - 1];
+        ews[u] = L.dtw[qq];
     }
     loads_issued();
+    // the predecessor scan's adjacent positions: n1's successor and p1
+    const int ps = pos1 + 1, pp = pos1 == rbeg ? rend : pos1 - 1;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int q = q0 + u * kOptGroup;
         const float d = (float)dn[u];
         const bool base = (q <= rend) & (q != pos1) & (c.rp[u] < p.nn_ls);
         c.oks[u] = base & (rads - d > kEps);
-        c.okp[u] = base & (radp - d > kEps) & !(c.xp[u] == n1 || p1 == c.n2[u]);
+        c.okp[u] = base & (radp - d > kEps) & (q != ps) & (q != pp);
         c.gs[u] = -rads + d + (float)dxs[u] - ews[u];
         c.gp[u] = -radp + d + (float)dxp[u] - ewp[u];
     }
@@ -324,7 +328,8 @@ __device__ __forceinline__ int two_opt_scans(const DevProblem &p, const LsLds &L
 {
     constexpr int U = kOptUnroll;
     const OptRows<RT> row(p, n1, s1, p1);
-    u64 bs = ~0ull, bp = ~0ull;
+    // best improving candidates: row position, then position
+    unsigned bs = ~0u, bp = ~0u;
     int cs = 0, cp = 0;
     // the first trip's candidates, kept for the evaluated-move count (one
     // trip covers most routes)
@@ -332,18 +337,16 @@ __device__ __forceinline__ int two_opt_scans(const DevProblem &p, const LsLds &L
     int rp_k[U] = {};
     for (int q0 = rbeg + 1 + gl; q0 <= rend; q0 += U * kOptGroup) {
         OptCands<U> c;
-        two_opt_cands<RT, U>(p, L, rend, pos1, q0, n1, p1, rads, radp, row, c);
+        two_opt_cands<RT, U>(p, L, rbeg, rend, pos1, q0, rads, radp, row, c);
         unsigned oks = 0, okp = 0;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             oks |= (unsigned)c.oks[u] << u;
             okp |= (unsigned)c.okp[u] << u;
             const bool is = c.oks[u] && c.gs[u] < -kEps, ip = c.okp[u] && c.gp[u] < -kEps;
-            if (is || ip) {
-                const u64 kr = ((u64)c.rp[u] << 32) | ((u64)c.n2[u] << 16);
-                if (is) bs = (kr | (u64)c.xs[u]) < bs ? (kr | (u64)c.xs[u]) : bs;
-                if (ip) bp = (kr | (u64)c.xp[u]) < bp ? (kr | (u64)c.xp[u]) : bp;
-            }
+            const unsigned key = (unsigned)c.rp[u] << 16 | (unsigned)(q0 + u * kOptGroup);
+            bs = is && key < bs ? key : bs;
+            bp = ip && key < bp ? key : bp;
         }
         cs += __builtin_popcount(oks);
         cp += __builtin_popcount(okp);
@@ -355,12 +358,12 @@ __device__ __forceinline__ int two_opt_scans(const DevProblem &p, const LsLds &L
         }
     }
     int kind = 0;
-    u64 best = group_min_u64(bs);
-    if (best != ~0ull) {
+    unsigned best = group_min_u32(bs);
+    if (best != ~0u) {
         kind = 1;
     } else {
-        best = group_min_u64(bp);
-        if (best != ~0ull) kind = 2;
+        best = group_min_u32(bp);
+        if (best != ~0u) kind = 2;
     }
     if (kind == 0) {
         evals += cs + cp;
@@ -368,7 +371,7 @@ __device__ __forceinline__ int two_opt_scans(const DevProblem &p, const LsLds &L
     }
     // the reference's walk stops at the accepted candidate: it evaluated
     // the candidates up to that row position
-    const int rps = (int)(best >> 32);
+    const int rps = (int)(best >> 16);
     int cnt = 0;
     if (rend - rbeg <= U * kOptGroup) {
         const unsigned ok = kind == 1 ? oks_k : okp_k;
@@ -377,14 +380,14 @@ __device__ __forceinline__ int two_opt_scans(const DevProblem &p, const LsLds &L
     } else {
         for (int q0 = rbeg + 1 + gl; q0 <= rend; q0 += U * kOptGroup) {
             OptCands<U> c;
-            two_opt_cands<RT, U>(p, L, rend, pos1, q0, n1, p1, rads, radp, row, c);
+            two_opt_cands<RT, U>(p, L, rbeg, rend, pos1, q0, rads, radp, row, c);
 #pragma unroll
             for (int u = 0; u < U; ++u) cnt += (kind == 1 ? c.oks[u] : c.okp[u]) && c.rp[u] <= rps;
         }
     }
     // the predecessor scan runs after the whole successor scan
     evals += cnt + (kind == 2 ? cs : 0);
-    const int b2 = (int)((best >> 16) & 0xFFFF), bx = (int)(best & 0xFFFF);
+    const int q2 = (int)(best & 0xFFFF), b2 = L.tour[q2], bx = L.tour[kind == 1 ? q2 + 1 : q2 - 1];
     if (kind == 1) { h1 = n1; h2 = s1; h3 = b2; h4 = bx; }
     else { h1 = p1; h2 = n1; h3 = bx; h4 = b2; }
     return kind;
