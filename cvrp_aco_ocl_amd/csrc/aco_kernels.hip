@@ -145,11 +145,25 @@ size_t construct_lds_bytes(int n, int selection)
     return (size_t)n * (4 + 4 + (selection == kSelIRoulette ? 4 : 0) + 1) + 16;
 }
 
-// The four-wave I-Roulette kernel's exchange of wave maxima (2 x 4 u64) after
-// the per-ant arrays, 8-byte aligned.
-__host__ __device__ __forceinline__ size_t iroulette4_exchange_offset(int n)
+// Best candidate of a wave of the several-wave I-Roulette kernel: key (prob
+// bits, then 4095 - rank and node), demand and distance.
+struct __align__(16) IrSlot {
+    u32 prob, low;
+    int dem;
+    float dc;
+};
+
+// The kernel's LDS after demands, depot distances and visited flags: two
+// rounds of IrSlot, one per wave, then (staged) the instance's total_info
+// and, with a route-length limit, distance matrices.
+__host__ __device__ __forceinline__ size_t iroulette_slots_offset(int n)
 {
-    return ((size_t)n * 13 + 16 + 7) & ~size_t(7);
+    return ((size_t)n * 9 + 16 + 15) & ~size_t(15);
+}
+static size_t iroulette_waves_lds(int n, int P, int waves, bool staged, bool has_d)
+{
+    return iroulette_slots_offset(n) + 2 * (size_t)waves * sizeof(IrSlot) +
+           (staged ? (size_t)n * P * 4 * (has_d ? 2 : 1) : 0);
 }
 
 // kernel.cl:445-452 mask: not visited, load + d_i <= Q and, with a route
@@ -410,112 +424,185 @@ __global__ __launch_bounds__(64) void k_construct_iroulette(DevBatch bt)
     s.pm[a * kLanes + lane] = z;
 }
 
-// The same construction with W = 4 or 8 waves per ant, for launches with at
-// most one ant per CU (otherwise the single-wave kernel keeps the CU's other
-// SIMDs busy with other ants).  A lane's draws stay its own Park-Miller
-// stream: node l + 64u uses the stream's (u+1)-th draw of the step,
-// z * 16807^(u+1) mod (2^31 - 1), so wave w takes u = w, w+W, ... starting
-// from the jump 16807^(w+1) and stepping by 16807^W; after the step every
-// wave advances the lane's state by the lane's node count.  The same keys as the
-// single-wave kernel; the waves' maxima meet in LDS (one barrier per step,
-// two buffers by step parity), and every wave sets the visited flag itself,
-// so it reads its own write in the next step.
+// z * a mod (2^31 - 1) for z, a in [1, 2^31 - 2]: 2^31 = 1 (mod 2^31 - 1),
+// and the product is never 0 mod the prime, so one subtraction suffices.
 __device__ __forceinline__ int pm_mulmod(int z, unsigned a)
 {
-    // z * a mod (2^31 - 1) for z, a in [1, 2^31 - 2]: 2^31 = 1 (mod 2^31 - 1),
-    // and the product is never 0 mod the prime, so one subtraction suffices
     const u64 prod = (u64)(u32)z * (u64)a;
     u32 r = (u32)(prod & 0x7FFFFFFFull) + (u32)(prod >> 31);
     r = r >= 0x7FFFFFFFu ? r - 0x7FFFFFFFu : r;
     return (int)r;
 }
 
-// Waves per ant: 4, or 8 when the instance has more than 512 nodes (two
-// waves per SIMD hide more of each step's latency; on smaller rows most of
-// an eighth-wave's lanes would have no node).
-constexpr int kIrWavesMax = 8;
-__host__ __device__ constexpr int iroulette_waves(int n) { return n > 512 ? 8 : 4; }
+// Largest value over the wave (uniform), and over lanes 0 .. N-1 where every
+// run of N lanes holds the same values.
+__device__ __forceinline__ u32 dpp_max_u32(u32 v, int o) { return v > (u32)o ? v : (u32)o; }
+template <int N> __device__ __forceinline__ u32 lanes_max_u32(u32 v)
+{
+    if (N >= 2) v = dpp_max_u32(v, __builtin_amdgcn_mov_dpp((int)v, kDppXor1, 0xF, 0xF, true));
+    if (N >= 4) v = dpp_max_u32(v, __builtin_amdgcn_mov_dpp((int)v, kDppXor2, 0xF, 0xF, true));
+    if (N >= 8) v = dpp_max_u32(v, __builtin_amdgcn_mov_dpp((int)v, kDppHalfMirror, 0xF, 0xF, true));
+    if (N >= 16) v = dpp_max_u32(v, __builtin_amdgcn_mov_dpp((int)v, kDppMirror, 0xF, 0xF, true));
+    if (N < 64) return (u32)uniform((int)v);
+    const u32 r0 = lane_i32((int)v, 0), r1 = lane_i32((int)v, 16), r2 = lane_i32((int)v, 32), r3 = lane_i32((int)v, 48);
+    const u32 a = r0 > r1 ? r0 : r1, b = r2 > r3 ? r2 : r3;
+    return a > b ? a : b;
+}
+// Lane (below N) of the largest (prob, low), whose prob is returned in top.
+template <int N> __device__ __forceinline__ int lanes_best(u32 prob, u32 low, u32 &top)
+{
+    constexpr u64 in = N < 64 ? (1ull << (N & 63)) - 1ull : ~0ull;
+    top = lanes_max_u32<N>(prob);
+    u64 tie = __ballot(prob == top) & in;
+    if (tie & (tie - 1)) {
+        const u32 l = lanes_max_u32<N>(prob == top ? low : 0u);
+        tie = __ballot(prob == top && low == l) & in;
+    }
+    return __builtin_ctzll(tie);
+}
 
-template <bool HAS_D, int kIrWaves>
-__global__ __launch_bounds__(kIrWaves * 64) void k_construct_iroulette4(DevBatch bt)
+// The same construction with NW waves per ant, for launches with at most
+// one ant per CU (otherwise the single-wave kernel keeps the CU's other
+// SIMDs busy with other ants).  A lane's draws stay its own Park-Miller
+// stream: node l + 64u uses the stream's (u+1)-th draw of the step,
+// z * 16807^(u+1) mod (2^31 - 1), so wave w takes u = w, w+NW, ... starting
+// from the jump 16807^(w+1) and stepping by 16807^NW; after the step every
+// wave advances the lane's state by the lane's node count.
+//
+// A step is a chain: row values, wave maximum, exchange of the waves' maxima
+// (one barrier, two buffers by step parity), next row.  So a lane keeps
+// everything that is fixed about its C nodes (demand, rank, depot distance,
+// visited bits) in registers, the maximum is taken over the 32-bit
+// probabilities (ties are resolved apart), the winner's demand and distance
+// travel with its key, and an instance whose matrices fit LDS has its rows
+// there (STAGED).  Per step, with keys of 64 bits, all fields in LDS and 4 or
+// 8 waves before: 51 nodes with a length limit 0.94 -> 0.41 us, 101 nodes
+// 0.88 -> 0.47 us (staged), 400 nodes 0.92 -> 0.63 us, 1001 nodes 1.15 ->
+// 0.70 us.  Unstaged it is bound by the row's L2 latency, staged by the
+// reduction.
+template <bool HAS_D, int NW, int C, bool STAGED>
+__global__ __launch_bounds__(NW * 64) void k_construct_iroulette_waves(DevBatch bt)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     ANT_PROLOGUE
-    const int n = p.n, tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    AntLds L = ant_lds(smem, n, true);
-    u64 *sh = reinterpret_cast<u64 *>(smem + iroulette4_exchange_offset(n));   // [2][kIrWaves]
-    for (int i = tid; i < n; i += kIrWaves * kLanes) {
+    const int n = p.n, P = p.P, tid = threadIdx.x, lane = tid & 63;
+    const int w = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 6);
+    AntLds L = ant_lds(smem, n, false);
+    IrSlot *slots = reinterpret_cast<IrSlot *>(smem + iroulette_slots_offset(n));   // [2][NW]
+    float *mt = reinterpret_cast<float *>(slots + 2 * NW), *md = mt + (STAGED ? n * P : 0);
+    for (int i = tid; i < n; i += NW * kLanes) {
         L.dem[i] = p.dem[i];
         L.d0[i] = p.d0[i];
-        L.rank[i] = p.rank[i];
         L.vis[i] = i == 0;
     }
-    __syncthreads();
+    if (STAGED) {
+        const float4 *gt = reinterpret_cast<const float4 *>(s.tinfo), *gd = reinterpret_cast<const float4 *>(p.dist);
+#pragma unroll 4
+        for (int e = tid; e < n * P / 4; e += NW * kLanes) {
+            reinterpret_cast<float4 *>(mt)[e] = gt[e];
+            if (HAS_D) reinterpret_cast<float4 *>(md)[e] = gd[e];
+        }
+    }
+    int node[C], dem[C];
+    u32 low[C];
+    float d0[C];
+    unsigned open = 0;   // the lane's nodes not visited yet
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+        const int i = lane + kLanes * (w + NW * j), ic = i < n ? i : n - 1;
+        node[j] = ic;
+        dem[j] = p.dem[ic];
+        d0[j] = HAS_D ? p.d0[ic] : 0.0f;
+        low[j] = (u32)(4095 - p.rank[ic]) << 12 | (u32)ic;
+        open |= i > 0 && i < n ? 1u << j : 0u;
+    }
     int z = s.pm[a * kLanes + lane];
-    const unsigned a4 = (unsigned)pm_jump(1, kIrWaves), aw = (unsigned)pm_jump(1, (unsigned long long)w + 1);
+    const unsigned anw = (unsigned)pm_jump(1, NW), aw = (unsigned)pm_jump(1, (unsigned long long)w + 1);
     const int cnt = lane < n ? (n - lane + kLanes - 1) / kLanes : 0;   // the lane's nodes (draws) per step
     const unsigned acnt = (unsigned)pm_jump(1, (unsigned long long)cnt);
     int *tour = s.tours + (size_t)a * p.T;
     int cur = 0, load = 0, vcnt = 1, step = 0, fb = 0, tbuf = 0;
     float rdist = 0.0f, tdist = 0.0f;
-    constexpr int C = kIrChunk / kIrWaves;   // a wave's nodes per lane per pass
+    __syncthreads();
     while (vcnt < n) {
-        const float *tirow = s.tinfo + (size_t)cur * p.P;
-        const float *drow = p.dist + (size_t)cur * p.P;
-        u64 best = 0;
-        int zz = pm_mulmod(z, aw);
-        // pass over u = base + w + Wj (node lane + 64u), j < C
-        for (int ub = 0; ub * kLanes < n; ub += kIrChunk) {
-            IrNodes<HAS_D, C> F;
+        const float *tirow = s.tinfo + (size_t)cur * P;
+        const float *drow = p.dist + (size_t)cur * P;
+        float tv[C], dv[C];
 #pragma unroll
-            for (int j = 0; j < C; ++j) F.load(p, L, tirow, drow, j, lane + kLanes * (ub + w + kIrWaves * j));
-#pragma unroll
-            for (int j = 0; j < C; ++j) {
-                const int i = lane + kLanes * (ub + w + kIrWaves * j);
-                if (i < n) {
-                    const float r = (float)zz * 0x1p-31f + 0.001f;
-                    zz = pm_mulmod(zz, a4);
-                    best = F.key(p, j, i, r, load, rdist, best);
-                }
-            }
+        for (int j = 0; j < C; ++j) {
+            tv[j] = STAGED ? mt[cur * P + node[j]] : gload(tirow + node[j]);
+            dv[j] = !HAS_D ? 0.0f : STAGED ? md[cur * P + node[j]] : gload(drow + node[j]);
         }
-        best = wave_max_u64(best);
-        u64 *ex = sh + (step & 1) * kIrWaves;
-        if (lane == 0) ex[w] = best;
-        __syncthreads();
+        float r[C];
+        int zz = pm_mulmod(z, aw);
 #pragma unroll
-        for (int v = 0; v < kIrWaves; ++v) {
-            const u64 o = ex[v];
-            best = o > best ? o : best;
+        for (int j = 0; j < C; ++j) {
+            r[j] = (float)zz * 0x1p-31f + 0.001f;
+            if (j + 1 < C) zz = pm_mulmod(zz, anw);
         }
         z = pm_mulmod(z, acnt);
+        // the lane's largest key of kernel.cl's reduction, (prob, 4095 -
+        // rank, node), with the mask of kernel.cl:445-452
+        IrSlot best = {0u, 0u, 0, 0.0f};
+#pragma unroll
+        for (int j = 0; j < C; ++j) {
+            const float pp = tv[j] * 100.0f;
+            bool c = ((open >> j) & 1u) & (load + dem[j] <= p.Q);
+            if (HAS_D) {
+                float t = rdist + (dv[j] + p.svc);
+                t = t + d0[j];
+                c = c & (t <= p.D);
+            }
+            const u32 prob = f2u(c ? r[j] * pp : 0.0f);
+            const bool more = prob > best.prob || (prob == best.prob && low[j] > best.low);
+            best.prob = more ? prob : best.prob;
+            best.low = more ? low[j] : best.low;
+            best.dem = more ? dem[j] : best.dem;
+            if (HAS_D) best.dc = more ? dv[j] : best.dc;
+        }
+        u32 top;
+        int l = lanes_best<kLanes>(best.prob, best.low, top);
+        u32 lo = (u32)lane_i32((int)best.low, l);
+        int dw = lane_i32(best.dem, l);
+        float dcw = HAS_D ? lane_f32(best.dc, l) : 0.0f;
+        if (NW > 1) {
+            IrSlot *ex = slots + (step & 1) * NW;
+            if (lane == 0) ex[w] = IrSlot{top, lo, dw, dcw};
+            __syncthreads();
+            const IrSlot o = ex[lane & (NW - 1)];
+            l = lanes_best<NW>(o.prob, o.low, top);
+            lo = (u32)lane_i32((int)o.low, l);
+            dw = lane_i32(o.dem, l);
+            if (HAS_D) dcw = lane_f32(o.dc, l);
+        }
         step++;
         int wn;
-        if ((best >> 32) == 0) {
+        if (top == 0) {
+            wn = 0;
             if (cur == 0) {
-                wn = greedy_pick<HAS_D>(p, L, tirow, drow, load, rdist, lane);
+                wn = uniform(greedy_pick<HAS_D>(p, L, tirow, drow, load, rdist, lane));
                 fb++;
-            } else {
-                wn = 0;
             }
+            dw = uniform(L.dem[wn]);
+            dcw = HAS_D ? drow[wn] : 0.0f;
         } else {
-            wn = (int)(best & 0xFFFull);
+            wn = (int)(lo & 0xFFFu);
         }
-        wn = uniform(wn);
-        const float dcw = HAS_D ? drow[wn] : 0.0f;   // without a limit: summed afterwards
         if (wn == 0) {
             load = 0;
             rdist = 0.0f;
         } else {
-            load += L.dem[wn];
+            load += dw;
             rdist = rdist + (dcw + p.svc);
             vcnt++;
         }
-        if (lane == 0) L.vis[wn] = 1;
-        tdist = tdist + dcw;
+#pragma unroll
+        for (int j = 0; j < C; ++j) open &= node[j] == wn ? ~(1u << j) : ~0u;
+        if (lane == 0) L.vis[wn] = 1;   // each wave for itself (greedy_pick)
+        tdist = tdist + dcw;            // without a limit: summed afterwards
         if (w == 0) tour_put(tour, tbuf, step, wn, lane);
         cur = wn;
+        if (NW == 1) __builtin_amdgcn_wave_barrier();
     }
     tdist = tdist + L.d0[cur];
     step++;
@@ -531,6 +618,27 @@ __global__ __launch_bounds__(kIrWaves * 64) void k_construct_iroulette4(DevBatch
         }
         s.pm[a * kLanes + lane] = z;
     }
+}
+
+// Waves and nodes per lane by instance size.  The exchange between waves
+// costs more than a second node per lane (one wave up to 128 nodes: 0.47
+// against 0.54 us a step with two); four waves and two nodes beat eight and
+// one at 400 nodes (0.63, 0.68 us), eight and two beat four and four or
+// sixteen and one at 1001 (0.70; 0.79, 0.75 us).
+struct IrChoice {
+    const void *fn;
+    int waves;
+};
+template <bool HAS_D> static IrChoice iroulette_choice(int n, bool staged)
+{
+#define IR(NW, C, S) IrChoice{(const void *)k_construct_iroulette_waves<HAS_D, NW, C, S>, NW}
+    if (staged) return n <= 64 ? IR(1, 1, true) : n <= 128 ? IR(1, 2, true) : IR(4, 1, true);
+    if (n <= 256) return IR(4, 1, false);
+    if (n <= 512) return IR(4, 2, false);
+    if (n <= 1024) return IR(8, 2, false);
+    if (n <= 2048) return IR(8, 4, false);
+    return IR(8, 8, false);
+#undef IR
 }
 
 // Roulette over the k-nearest candidate row: lane c holds candidate c's
@@ -825,8 +933,6 @@ static hipError_t max_static_lds(const void *const *fns, int count, size_t &byte
 hipError_t construct_static_lds(size_t &bytes)
 {
     const void *fns[] = {(const void *)k_construct_iroulette<false>, (const void *)k_construct_iroulette<true>,
-                         (const void *)k_construct_iroulette4<false, 4>, (const void *)k_construct_iroulette4<true, 4>,
-                         (const void *)k_construct_iroulette4<false, 8>, (const void *)k_construct_iroulette4<true, 8>,
                          (const void *)k_construct_knn<false, kRngPhilox, true>,
                          (const void *)k_construct_knn<true, kRngPhilox, true>,
                          (const void *)k_construct_knn<false, kRngParkMiller, true>,
@@ -863,17 +969,16 @@ hipError_t launch_construct(const DevBatch &b, int selection, int rng, int apb, 
     const dim3 grid(b.ants), block(kLanes);
     if (selection == kSelIRoulette) {
         if (b.ants <= b.cus) {
-            // at most one ant per CU: four waves per ant
-            const size_t lds4 = iroulette4_exchange_offset(b.max_n) + 2 * kIrWavesMax * sizeof(u64);
-            const int nw = iroulette_waves(b.max_n);
-            const dim3 block4(nw * kLanes);
-            if (nw == 8) {
-                if (b.has_d) hipLaunchKernelGGL((k_construct_iroulette4<true, 8>), grid, block4, lds4, st, b);
-                else hipLaunchKernelGGL((k_construct_iroulette4<false, 8>), grid, block4, lds4, st, b);
-            } else {
-                if (b.has_d) hipLaunchKernelGGL((k_construct_iroulette4<true, 4>), grid, block4, lds4, st, b);
-                else hipLaunchKernelGGL((k_construct_iroulette4<false, 4>), grid, block4, lds4, st, b);
-            }
+            // at most one ant per CU: several waves per ant, the matrices in
+            // LDS where they fit (an instance of up to about 190 nodes, 135
+            // with a length limit): reading them once costs a step or two
+            const bool staged = b.max_n <= 256 &&
+                                iroulette_waves_lds(b.max_n, b.max_P, 4, true, b.has_d) <= b.cons_lds_budget;
+            const IrChoice c = b.has_d ? iroulette_choice<true>(b.max_n, staged) : iroulette_choice<false>(b.max_n, staged);
+            DevBatch bt = b;
+            void *args[] = {&bt};
+            return hipLaunchKernel(c.fn, grid, dim3(c.waves * kLanes), args,
+                                   iroulette_waves_lds(b.max_n, b.max_P, c.waves, staged, b.has_d), st);
         } else if (b.has_d) {
             hipLaunchKernelGGL(k_construct_iroulette<true>, grid, block, lds, st, b);
         } else {
