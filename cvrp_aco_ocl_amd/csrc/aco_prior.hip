@@ -31,6 +31,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -278,7 +279,8 @@ __global__ __launch_bounds__(kThreads) void k_forward(const unsigned short *xb, 
 }
 
 // Fused forward + backward over kTilesPerWave tiles of the batch
-// (positions [0, Eb) of idx); writes one partial row per wave.
+// (positions [0, Eb) of idx, or of the data in order without one); writes
+// one partial row per wave.
 __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, const float *label,
                                                     const int *idx, int Eb,
                                                     const unsigned short *wb, const float *pf,
@@ -304,7 +306,7 @@ __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, co
         if (tile >= tiles) break;
         const int pos = tile * 16 + r;
         const bool valid = pos < Eb;
-        const int e = valid ? idx[pos] : 0;
+        const int e = !valid ? 0 : idx ? idx[pos] : pos;
         const v4s x = load_x(xb, e, valid, g);
         const float y = valid ? label[e] : 0.0f;
         Fwd F;
@@ -457,18 +459,42 @@ __global__ void k_to_bf16(const float *pf, unsigned short *wb, int count)
     if (p < count) wb[p] = f2bf(pf[p]);
 }
 
-// Features -> bf16 rows of 16 (features 12..15 zero).
-__global__ void k_pack_features(const float *feat, long long E, unsigned short *xb)
+// Features -> bf16 rows of 16 (features 12..15 zero), labels copied along:
+// four threads per edge, 16 bytes each.  The inputs may lie in pinned host
+// memory (read once, in order, over the link).
+__global__ void k_pack_features(const float *feat, const float *label, long long E, unsigned short *xb, float *lab)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= E * NFP) return;
-    const long long e = t / NFP;
-    const int f = (int)(t % NFP);
-    xb[t] = f < NF ? f2bf(feat[e * NF + f]) : (unsigned short)0;
+    const long long e = t >> 2;
+    const int q = (int)(t & 3);
+    if (e >= E) return;
+    ushort4 o = {0, 0, 0, 0};
+    if (q < 3) {
+        const float4 f = *reinterpret_cast<const float4 *>(feat + e * NF + 4 * q);
+        o = ushort4{f2bf(f.x), f2bf(f.y), f2bf(f.z), f2bf(f.w)};
+    } else if (label) {
+        lab[e] = label[e];
+    }
+    *reinterpret_cast<ushort4 *>(xb + e * NFP + 4 * q) = o;
 }
 
-// dist rows have pitch P (>= n)
-__global__ void k_node_stats(int n, int P, const float *x, const float *y, const float *dist,
+// Distances of one instance: the whole matrix with row pitch P (>= n), or
+// its depot row and candidate edges only.
+struct DistMatrix {
+    const float *d;
+    int P;
+    __device__ __forceinline__ float edge(int i, int, int j) const { return d[(size_t)i * P + j]; }
+    __device__ __forceinline__ float depot(int i) const { return d[i]; }
+};
+struct DistEdges {
+    const float *d0, *e;   // n, n x k
+    int k;
+    __device__ __forceinline__ float edge(int i, int r, int) const { return e[(size_t)i * k + r]; }
+    __device__ __forceinline__ float depot(int i) const { return d0[i]; }
+};
+
+template <class D>
+__global__ void k_node_stats(int n, const float *x, const float *y, D dist,
                              const int *nn, int nnw, int k, float *rad, float *ang, float *kd)
 {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
@@ -476,7 +502,7 @@ __global__ void k_node_stats(int n, int P, const float *x, const float *y, const
     const float dx = x[v] - x[0], dy = y[v] - y[0];
     rad[v] = sqrtf(dx * dx + dy * dy);
     ang[v] = atan2f(dy, dx) / 3.14159265358979323846f;
-    kd[v] = dist[(size_t)v * P + nn[(size_t)v * nnw + k - 1]];
+    kd[v] = dist.edge(v, k - 1, nn[(size_t)v * nnw + k - 1]);
 }
 
 // One block: R = max radius (1 if 0), mkd = mean k-th candidate distance
@@ -510,7 +536,8 @@ __global__ void k_node_reduce(int n, const float *rad, const float *kd, float *o
     }
 }
 
-__global__ void k_edge_features(int n, int P, int k, const float *dist, const int *nn, int nnw,
+template <class D>
+__global__ void k_edge_features(int n, int k, D dist, const int *nn, int nnw,
                                 const int *dem, float Q, const float *rad, const float *ang,
                                 const float *kd, const float *Rm, float *feat, unsigned short *xb)
 {
@@ -519,7 +546,7 @@ __global__ void k_edge_features(int n, int P, int k, const float *dist, const in
     const int i = (int)(t / k), r = (int)(t % k);
     const int j = nn[(size_t)i * nnw + r];
     const float R = Rm[0], mkd = Rm[1];
-    const float dij = dist[(size_t)i * P + j];
+    const float dij = dist.edge(i, r, j);
     float f[NF];
     f[0] = dij / mkd;
     f[1] = (float)r / (float)k;
@@ -531,7 +558,7 @@ __global__ void k_edge_features(int n, int P, int k, const float *dist, const in
     f[7] = rad[j] / R;
     f[8] = kd[i] / mkd;
     f[9] = kd[j] / mkd;
-    f[10] = ((dist[i] + dist[j]) - dij) / R;
+    f[10] = ((dist.depot(i) + dist.depot(j)) - dij) / R;
     bool mutual = false;
     for (int q = 0; q < k; ++q) mutual |= nn[(size_t)j * nnw + q] == i;
     f[11] = mutual ? 1.0f : 0.0f;
@@ -565,6 +592,43 @@ __global__ void k_prior_scatter(int n, int k, const int *nn, int nnw, const floa
     out[(size_t)i * n + j] = prior_pow(p, ex);
 }
 
+// Rows row0 .. row0 + gridDim.x of the dense multiplier, one block each,
+// written once and in order (out may be pinned host memory): `val` except at
+// the row's candidates.  LDS: n floats where they fit (staged), otherwise
+// the candidates are written after the fill.
+template <bool STAGED>
+__global__ __launch_bounds__(256) void k_prior_rows(int n, int row0, int k, const int *nn, int nnw, const float *logits,
+                                                    float ex, float val, float *out)
+{
+    extern __shared__ float row[];
+    const int i = row0 + blockIdx.x;
+    float *o = out + (size_t)blockIdx.x * n, *w = STAGED ? row : o;
+    for (int j = threadIdx.x; j < n; j += 256) w[j] = val;
+    if (!STAGED) __threadfence_system();   // another thread writes the candidate's entry again
+    __syncthreads();
+    for (int r = threadIdx.x; r < k; r += 256) {
+        const float p = 1.0f / (1.0f + expf(-logits[(size_t)i * k + r]));
+        w[nn[(size_t)i * nnw + r]] = prior_pow(p, ex);
+    }
+    if (!STAGED) return;
+    __syncthreads();
+    for (int j = threadIdx.x; j < n; j += 256) o[j] = row[j];
+}
+constexpr int kPriorRowLds = 4096;   // floats: 16 KB, several rows per CU
+
+// Fisher-Yates swap targets of draws draw0 .. draw0 + count of a SplitMix64
+// stream: draw d swaps index i = last - (d - draw0) with out = x % (i + 1).
+__global__ void k_swap_targets(unsigned long long seed, unsigned long long draw0, int last, int count, int *out)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= count) return;
+    unsigned long long z = seed + 0x9E3779B97F4A7C15ull * (draw0 + (unsigned long long)t + 1ull);
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    z ^= z >> 31;
+    out[t] = (int)(z % (unsigned long long)(last - t + 1));
+}
+
 // heur[i][j] (pitch P) *= prior[i][j] (pitch n), j < n
 __global__ void k_heur_mul(int n, int P, const float *prior, float *heur)
 {
@@ -594,8 +658,99 @@ static hipError_t dalloc(DevBuf &b, size_t bytes)
 using namespace cvrp;
 using namespace cvrp::prior;
 
+// Working memory of a network's calls, kept between them (one call at a
+// time): one device allocation, given back after a call that needed more
+// than kKeep, and four pinned buffers of 512 KB.  Pageable copies of this
+// size cost 25 to 60 us each whatever they hold, allocations of 2 MB and more
+// 25 us; a gradient made six of the first and two of the second.  Gradient
+// over 16384 edges 202 -> 99 us, multiplier of 501 nodes 200 -> 117 us, eight
+// training steps of 16384 edges 945 -> 700 us; what is left is the copy into
+// the buffers, the launches and the kernels (50 us of the gradient).
+struct PriorSpace {
+    static constexpr size_t kPin = size_t(512) << 10, kKeep = size_t(64) << 20;
+    std::mutex mutex;
+    unsigned char *dev = nullptr;
+    size_t dev_bytes = 0;
+    unsigned char *pin[4] = {nullptr, nullptr, nullptr, nullptr};   // 0, 1: inputs and matrices; 2, 3: small results
+    hipEvent_t done[2] = {nullptr, nullptr};
+    bool busy[2] = {false, false};
+    int cur = 0;
+    hipStream_t side = nullptr;   // swap targets, beside the training stream
+
+    hipError_t init(size_t bytes)
+    {
+        if (bytes <= dev_bytes) return hipSuccess;
+        release();
+        const hipError_t e = hipMalloc((void **)&dev, bytes);
+        if (e == hipSuccess) dev_bytes = bytes;
+        return e;
+    }
+    hipError_t pinned(int i)   // buffer i exists
+    {
+        return pin[i] ? hipSuccess : hipHostMalloc((void **)&pin[i], kPin, hipHostMallocDefault);
+    }
+    void release()
+    {
+        if (dev) (void)hipFree(dev);
+        dev = nullptr;
+        dev_bytes = 0;
+    }
+    ~PriorSpace()
+    {
+        release();
+        for (unsigned char *p : pin)
+            if (p) (void)hipHostFree(p);
+        for (hipEvent_t e : done)
+            if (e) (void)hipEventDestroy(e);
+        if (side) (void)hipStreamDestroy(side);
+    }
+    // input buffer to fill next, once its last reader on the device is done
+    hipError_t take(unsigned char *&p)
+    {
+        hipError_t e = pinned(cur);
+        if (e == hipSuccess && !done[cur]) e = hipEventCreateWithFlags(&done[cur], hipEventDisableTiming);
+        if (e == hipSuccess && busy[cur]) e = hipEventSynchronize(done[cur]);
+        busy[cur] = false;
+        p = pin[cur];
+        return e;
+    }
+    hipError_t used(hipStream_t st)
+    {
+        const hipError_t e = hipEventRecord(done[cur], st);
+        busy[cur] = true;
+        cur ^= 1;
+        return e;
+    }
+};
+
+// One call's use of a PriorSpace: pieces of the device allocation, and at the
+// end nothing of the call in flight.
+struct SpaceUse {
+    PriorSpace &s;
+    hipStream_t st;
+    std::lock_guard<std::mutex> lock;
+    size_t off = 0;
+    SpaceUse(PriorSpace &sp, hipStream_t stream) : s(sp), st(stream), lock(sp.mutex) {}
+    ~SpaceUse()
+    {
+        (void)hipStreamSynchronize(st);
+        if (s.side) (void)hipStreamSynchronize(s.side);
+        s.busy[0] = s.busy[1] = false;
+        s.cur = 0;
+        if (s.dev_bytes > PriorSpace::kKeep) s.release();
+    }
+    static size_t round(size_t bytes) { return (bytes + 255) & ~size_t(255); }
+    template <class T> T *take(size_t count)
+    {
+        T *p = reinterpret_cast<T *>(s.dev + off);
+        off += round(count * sizeof(T));
+        return p;
+    }
+};
+
 struct aco_prior {
     hipStream_t stream = nullptr;
+    PriorSpace space;
     float *pf = nullptr, *m = nullptr, *v = nullptr;
     unsigned short *wb = nullptr;
     int step = 0;
@@ -664,20 +819,63 @@ static AdamArgs adam_args(int step, float lr, float b1, float b2, float eps)
     return a;
 }
 
-// bf16 features of `count` edges (host fp32, count x 12) into xb.
-static int stage_features(aco_prior *net, const float *feat, long long count, DevBuf &xb)
+// bf16 features (and labels) of `count` edges into device arrays: rows pass
+// through the pinned input buffers, from which the packing kernel reads them
+// while the next buffer is filled.
+static int stage_features(aco_prior *net, const float *feat, const float *label, long long count, unsigned short *xb,
+                          float *lab)
 {
-    DevBuf f32;
-    PCHK(dalloc(f32, (size_t)count * NF * sizeof(float)));
-    PCHK(dalloc(xb, (size_t)count * NFP * sizeof(unsigned short)));
-    PCHK(hipMemcpyAsync(f32.p, feat, (size_t)count * NF * sizeof(float), hipMemcpyHostToDevice, net->stream));
-    const long long tot = count * NFP;
-    hipLaunchKernelGGL(k_pack_features, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, net->stream,
-                       f32.as<float>(), count, xb.as<unsigned short>());
-    PCHK(hipGetLastError());
-    PCHK(hipStreamSynchronize(net->stream));
+    PriorSpace &sp = net->space;
+    const long long per = (long long)(PriorSpace::kPin / ((NF + 1) * sizeof(float)));
+    for (long long e = 0; e < count; e += per) {
+        const long long c = std::min(per, count - e);
+        unsigned char *b = nullptr;
+        PCHK(sp.take(b));
+        float *f = reinterpret_cast<float *>(b), *l = f + c * NF;
+        memcpy(f, feat + e * NF, (size_t)c * NF * sizeof(float));
+        if (label) memcpy(l, label + e, (size_t)c * sizeof(float));
+        hipLaunchKernelGGL(k_pack_features, dim3((unsigned)((4 * c + 255) / 256)), dim3(256), 0, net->stream, f,
+                           label ? l : nullptr, c, xb + e * NFP, label ? lab + e : nullptr);
+        PCHK(hipGetLastError());
+        PCHK(sp.used(net->stream));
+    }
     return ACO_OK;
 }
+
+// Bytes put one after another, sent to the device through the pinned input
+// buffers.
+struct PinnedStream {
+    aco_prior *net;
+    unsigned char *dst, *buf = nullptr;
+    size_t fill = 0;
+    int flush()
+    {
+        if (!fill) return ACO_OK;
+        PCHK(hipMemcpyAsync(dst, buf, fill, hipMemcpyHostToDevice, net->stream));
+        PCHK(net->space.used(net->stream));
+        dst += fill;
+        fill = 0;
+        buf = nullptr;
+        return ACO_OK;
+    }
+    int put(const void *src, size_t bytes)
+    {
+        const unsigned char *s = static_cast<const unsigned char *>(src);
+        while (bytes) {
+            if (fill == PriorSpace::kPin) {
+                const int rc = flush();
+                if (rc != ACO_OK) return rc;
+            }
+            if (!buf) PCHK(net->space.take(buf));
+            const size_t c = std::min(bytes, PriorSpace::kPin - fill);
+            memcpy(buf + fill, s, c);
+            fill += c;
+            s += c;
+            bytes -= c;
+        }
+        return ACO_OK;
+    }
+};
 
 static int launch_forward(aco_prior *net, const unsigned short *xb, long long count, float *logits,
                           hipStream_t st = nullptr)
@@ -810,13 +1008,12 @@ static int check_instance_args(int32_t n, const float *x, const float *y, const 
     return ACO_OK;
 }
 
-// Device features of one instance: fp32 (optional) and bf16 rows.
+// Device features of one instance, fp32 rows.
 static int device_features(hipStream_t st, int32_t n, const float *x, const float *y,
                            const int32_t *demand, int32_t capacity, const float *dist,
-                           const int32_t *nn, int32_t nnw, int32_t k, DevBuf &feat_d, DevBuf &xb,
-                           DevBuf &nn_d, bool want_f32)
+                           const int32_t *nn, int32_t nnw, int32_t k, DevBuf &feat_d)
 {
-    DevBuf xd, yd, dd, demd, rad, ang, kd, Rm;
+    DevBuf xd, yd, dd, demd, nn_d, rad, ang, kd, Rm;
     const size_t N = (size_t)n, E = N * (size_t)k;
     PCHK(dalloc(xd, N * 4));
     PCHK(dalloc(yd, N * 4));
@@ -827,24 +1024,23 @@ static int device_features(hipStream_t st, int32_t n, const float *x, const floa
     PCHK(dalloc(ang, N * 4));
     PCHK(dalloc(kd, N * 4));
     PCHK(dalloc(Rm, 16));
-    PCHK(dalloc(xb, E * NFP * 2));
-    if (want_f32) PCHK(dalloc(feat_d, E * NF * 4));
+    PCHK(dalloc(feat_d, E * NF * 4));
     PCHK(hipMemcpyAsync(xd.p, x, N * 4, hipMemcpyHostToDevice, st));
     PCHK(hipMemcpyAsync(yd.p, y, N * 4, hipMemcpyHostToDevice, st));
     PCHK(hipMemcpyAsync(dd.p, dist, N * N * 4, hipMemcpyHostToDevice, st));
     PCHK(hipMemcpyAsync(demd.p, demand, N * 4, hipMemcpyHostToDevice, st));
     PCHK(hipMemcpyAsync(nn_d.p, nn, N * nnw * 4, hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_node_stats, dim3((n + 255) / 256), dim3(256), 0, st, n, n, xd.as<float>(),
-                       yd.as<float>(), dd.as<float>(), nn_d.as<int>(), nnw, k, rad.as<float>(),
-                       ang.as<float>(), kd.as<float>());
+    const DistMatrix D = {dd.as<float>(), n};
+    hipLaunchKernelGGL(k_node_stats<DistMatrix>, dim3((n + 255) / 256), dim3(256), 0, st, n, xd.as<float>(),
+                       yd.as<float>(), D, nn_d.as<int>(), nnw, k, rad.as<float>(), ang.as<float>(),
+                       kd.as<float>());
     PCHK(hipGetLastError());
     hipLaunchKernelGGL(k_node_reduce, dim3(1), dim3(256), 0, st, n, rad.as<float>(), kd.as<float>(),
                        Rm.as<float>());
     PCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_edge_features, dim3((unsigned)((E + 255) / 256)), dim3(256), 0, st, n, n, k,
-                       dd.as<float>(), nn_d.as<int>(), nnw, demd.as<int>(), (float)capacity,
-                       rad.as<float>(), ang.as<float>(), kd.as<float>(), Rm.as<float>(),
-                       want_f32 ? feat_d.as<float>() : nullptr, xb.as<unsigned short>());
+    hipLaunchKernelGGL(k_edge_features<DistMatrix>, dim3((unsigned)((E + 255) / 256)), dim3(256), 0, st, n, k, D,
+                       nn_d.as<int>(), nnw, demd.as<int>(), (float)capacity, rad.as<float>(), ang.as<float>(),
+                       kd.as<float>(), Rm.as<float>(), feat_d.as<float>(), (unsigned short *)nullptr);
     PCHK(hipGetLastError());
     PCHK(hipStreamSynchronize(st));
     return ACO_OK;
@@ -862,8 +1058,8 @@ int aco_prior_features(int32_t n, const float *x, const float *y, const int32_t 
     hipStream_t st;
     PCHK(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
     {
-        DevBuf fd, xb, nnd;
-        rc = device_features(st, n, x, y, demand, capacity, dist, nn, nn_width, k, fd, xb, nnd, true);
+        DevBuf fd;
+        rc = device_features(st, n, x, y, demand, capacity, dist, nn, nn_width, k, fd);
         if (rc == ACO_OK) {
             const hipError_t e = hipMemcpy(feat, fd.p, (size_t)n * k * NF * 4, hipMemcpyDeviceToHost);
             if (e != hipSuccess) rc = set_error(ACO_ERR_HIP, std::string("feature readback: ") + hipGetErrorString(e));
@@ -877,13 +1073,15 @@ int aco_prior_forward(aco_prior *net, const float *feat, int64_t count, float *l
 {
     if (!net || !feat || !logits) return set_error(ACO_ERR_ARG, "null argument");
     if (count < 1 || count > (1ll << 31)) return set_error(ACO_ERR_ARG, "count out of range");
-    DevBuf xb, out;
-    int rc = stage_features(net, feat, count, xb);
+    SpaceUse use(net->space, net->stream);
+    PCHK(net->space.init(SpaceUse::round((size_t)count * NFP * 2) + SpaceUse::round((size_t)count * 4)));
+    unsigned short *xb = use.take<unsigned short>((size_t)count * NFP);
+    float *out = use.take<float>((size_t)count);
+    int rc = stage_features(net, feat, nullptr, count, xb, nullptr);
     if (rc != ACO_OK) return rc;
-    PCHK(dalloc(out, (size_t)count * 4));
-    rc = launch_forward(net, xb.as<unsigned short>(), count, out.as<float>());
+    rc = launch_forward(net, xb, count, out);
     if (rc != ACO_OK) return rc;
-    PCHK(hipMemcpyAsync(logits, out.p, (size_t)count * 4, hipMemcpyDeviceToHost, net->stream));
+    PCHK(hipMemcpyAsync(logits, out, (size_t)count * 4, hipMemcpyDeviceToHost, net->stream));
     PCHK(hipStreamSynchronize(net->stream));
     return ACO_OK;
 }
@@ -894,26 +1092,23 @@ int aco_prior_gradient(aco_prior *net, const float *feat, const float *label, in
     if (!net || !feat || !label || !grad) return set_error(ACO_ERR_ARG, "null argument");
     if (count < 1 || count > kMaxBatch) return set_error(ACO_ERR_ARG, "count must be in [1, 65536]");
     if (!(pos_weight > 0.0f) || !std::isfinite(pos_weight)) return set_error(ACO_ERR_ARG, "pos_weight must be positive");
-    DevBuf xb, lab, idx, part, g, l;
-    int rc = stage_features(net, feat, count, xb);
+    SpaceUse use(net->space, net->stream);
+    const size_t E = (size_t)count;
+    PCHK(net->space.init(SpaceUse::round(E * NFP * 2) + SpaceUse::round(E * 4) + partial_bytes((int)count)));
+    unsigned short *xb = use.take<unsigned short>(E * NFP);
+    float *lab = use.take<float>(E), *part = use.take<float>(partial_bytes((int)count) / 4);
+    int rc = stage_features(net, feat, label, count, xb, lab);
     if (rc != ACO_OK) return rc;
-    std::vector<int> id((size_t)count);
-    for (int i = 0; i < (int)count; ++i) id[i] = i;
-    PCHK(dalloc(lab, (size_t)count * 4));
-    PCHK(dalloc(idx, (size_t)count * 4));
-    PCHK(dalloc(part, partial_bytes((int)count)));
-    PCHK(dalloc(g, NP * 4));
-    PCHK(dalloc(l, 16));
-    PCHK(hipMemcpyAsync(lab.p, label, (size_t)count * 4, hipMemcpyHostToDevice, net->stream));
-    PCHK(hipMemcpyAsync(idx.p, id.data(), (size_t)count * 4, hipMemcpyHostToDevice, net->stream));
-    rc = launch_batch(net, xb.as<unsigned short>(), lab.as<float>(), idx.as<int>(), (int)count, pos_weight,
-                      part.as<float>(), g.as<float>(), l.as<float>(), false, adam_args(1, 0, 0.9f, 0.999f, 1e-8f));
+    // the reduction writes the gradient and the loss to host memory
+    PCHK(net->space.pinned(2));
+    float *g = reinterpret_cast<float *>(net->space.pin[2]);
+    static_assert(NPL * sizeof(float) <= PriorSpace::kPin, "gradient and loss fit");
+    rc = launch_batch(net, xb, lab, nullptr, (int)count, pos_weight, part, g, g + NP, false,
+                      adam_args(1, 0, 0.9f, 0.999f, 1e-8f));
     if (rc != ACO_OK) return rc;
-    PCHK(hipMemcpyAsync(grad, g.p, NP * 4, hipMemcpyDeviceToHost, net->stream));
-    float lv = 0.0f;
-    PCHK(hipMemcpyAsync(&lv, l.p, 4, hipMemcpyDeviceToHost, net->stream));
     PCHK(hipStreamSynchronize(net->stream));
-    if (loss) *loss = lv;
+    memcpy(grad, g, NP * sizeof(float));
+    if (loss) *loss = g[NP];
     return ACO_OK;
 }
 
@@ -944,41 +1139,87 @@ int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64
         return set_error(ACO_ERR_ARG, "epochs >= 1 and batch in [16, 65536] required");
     if (!(tp->lr > 0.0f) || !(tp->lr_final >= 0.0f) || !(tp->pos_weight > 0.0f))
         return set_error(ACO_ERR_ARG, "lr, lr_final, pos_weight must be positive");
-    DevBuf xb, lab, idx, part, losses;
-    int rc = stage_features(net, feat, count, xb);
-    if (rc != ACO_OK) return rc;
     const long long nb = (count + tp->batch - 1) / tp->batch;
     const long long total = nb * tp->epochs;
-    PCHK(dalloc(lab, (size_t)count * 4));
-    PCHK(dalloc(idx, (size_t)count * 4));
-    PCHK(dalloc(part, partial_bytes(tp->batch)));
-    PCHK(dalloc(losses, (size_t)total * 4));
-    PCHK(hipMemcpyAsync(lab.p, label, (size_t)count * 4, hipMemcpyHostToDevice, net->stream));
+    SpaceUse use(net->space, net->stream);
+    PriorSpace &sp = net->space;
+    const size_t E = (size_t)count;
+    PCHK(sp.init(SpaceUse::round(E * NFP * 2) + 2 * SpaceUse::round(E * 4) + SpaceUse::round(partial_bytes(tp->batch)) +
+                 SpaceUse::round((size_t)total * 4)));
+    unsigned short *xb = use.take<unsigned short>(E * NFP);
+    float *lab = use.take<float>(E);
+    int *idx = use.take<int>(E);
+    float *part = use.take<float>(partial_bytes(tp->batch) / 4), *losses = use.take<float>((size_t)total);
+    // The order of an epoch is a Fisher-Yates shuffle, which only the host can
+    // make (65536 swaps: 0.1 ms), but the swap targets are one 64-bit remainder
+    // each (0.3 ms) of a counter-based stream, so the device draws them, on a
+    // stream of its own, two buffers ahead of the swaps.
+    const int chunk = (int)(PriorSpace::kPin / sizeof(int));
+    const long long per_epoch = count - 1, draws = per_epoch * tp->epochs;
+    long long drawn = 0;   // draws requested so far
+    int at = 0;            // pinned buffer the next request fills (2 or 3)
+    hipEvent_t ready[2] = {nullptr, nullptr};
+    struct Events {
+        hipEvent_t *e;
+        ~Events()
+        {
+            for (int i = 0; i < 2; ++i)
+                if (e[i]) (void)hipEventDestroy(e[i]);
+        }
+    } events{ready};
+    for (hipEvent_t &e : ready) PCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    PCHK(sp.pinned(2));
+    PCHK(sp.pinned(3));
+    if (!sp.side) PCHK(hipStreamCreateWithFlags(&sp.side, hipStreamNonBlocking));
+    auto request = [&]() -> int {   // never across an epoch's end
+        if (drawn == draws) return ACO_OK;
+        const long long in = drawn % per_epoch;
+        const int c = (int)std::min<long long>(chunk, per_epoch - in);
+        hipLaunchKernelGGL(k_swap_targets, dim3((c + 255) / 256), dim3(256), 0, sp.side, tp->shuffle_seed,
+                           (unsigned long long)drawn, (int)(per_epoch - in), c, reinterpret_cast<int *>(sp.pin[2 + at]));
+        PCHK(hipGetLastError());
+        PCHK(hipEventRecord(ready[at], sp.side));
+        drawn += c;
+        at ^= 1;
+        return ACO_OK;
+    };
+    int rc = request();
+    if (rc == ACO_OK) rc = request();
+    if (rc != ACO_OK) return rc;
+    rc = stage_features(net, feat, label, count, xb, lab);
+    if (rc != ACO_OK) return rc;
     std::vector<int> perm((size_t)count);
-    uint64_t s = tp->shuffle_seed;
     long long step = 0;
+    int from = 0;   // buffer the next targets come from
     for (int ep = 0; ep < tp->epochs; ++ep) {
         for (long long i = 0; i < count; ++i) perm[(size_t)i] = (int)i;
-        for (long long i = count - 1; i > 0; --i) {
-            const long long j = (long long)(sm_next(s) % (uint64_t)(i + 1));
-            std::swap(perm[(size_t)i], perm[(size_t)j]);
+        for (long long i = count - 1; i > 0;) {
+            PCHK(hipEventSynchronize(ready[from]));
+            const int *j = reinterpret_cast<const int *>(sp.pin[2 + from]);
+            const long long c = std::min<long long>(chunk, i);
+            for (long long t = 0; t < c; ++t) std::swap(perm[(size_t)(i - t)], perm[(size_t)j[t]]);
+            i -= c;
+            rc = request();   // refills this buffer
+            if (rc != ACO_OK) return rc;
+            from ^= 1;
         }
-        PCHK(hipStreamSynchronize(net->stream));  // previous epoch done with idx
-        PCHK(hipMemcpyAsync(idx.p, perm.data(), (size_t)count * 4, hipMemcpyHostToDevice, net->stream));
+        PinnedStream up = {net, reinterpret_cast<unsigned char *>(idx)};   // behind the epoch that reads idx now
+        rc = up.put(perm.data(), E * sizeof(int));
+        if (rc == ACO_OK) rc = up.flush();
+        if (rc != ACO_OK) return rc;
         for (long long b = 0; b < nb; ++b, ++step) {
             const long long lo = b * tp->batch;
             const int Eb = (int)std::min<long long>(tp->batch, count - lo);
             const double frac = total > 1 ? (double)step / (double)(total - 1) : 0.0;
             const float lr = (float)(tp->lr_final + 0.5 * (tp->lr - tp->lr_final) * (1.0 + cos(M_PI * frac)));
             net->step += 1;
-            rc = launch_batch(net, xb.as<unsigned short>(), lab.as<float>(), idx.as<int>() + lo, Eb,
-                              tp->pos_weight, part.as<float>(), nullptr, losses.as<float>() + step, true,
+            rc = launch_batch(net, xb, lab, idx + lo, Eb, tp->pos_weight, part, nullptr, losses + step, true,
                               adam_args(net->step, lr, tp->beta1, tp->beta2, tp->eps));
             if (rc != ACO_OK) return rc;
         }
     }
     std::vector<float> lh((size_t)total);
-    PCHK(hipMemcpyAsync(lh.data(), losses.p, (size_t)total * 4, hipMemcpyDeviceToHost, net->stream));
+    PCHK(hipMemcpyAsync(lh.data(), losses, (size_t)total * 4, hipMemcpyDeviceToHost, net->stream));
     PCHK(hipStreamSynchronize(net->stream));
     if (epoch_loss)
         for (int ep = 0; ep < tp->epochs; ++ep) {
@@ -998,24 +1239,72 @@ int aco_prior_build(aco_prior *net, int32_t n, const float *x, const float *y,
     if (rc != ACO_OK) return rc;
     if (!(exponent >= 0.0f) || !std::isfinite(exponent)) return set_error(ACO_ERR_ARG, "exponent must be >= 0");
     if (!(floor > 0.0f && floor <= 1.0f)) return set_error(ACO_ERR_ARG, "floor must be in (0, 1]");
-    DevBuf fd, xb, nnd, lg, out;
-    rc = device_features(net->stream, n, x, y, demand, capacity, dist, nn, nn_width, k, fd, xb, nnd, false);
-    if (rc != ACO_OK) return rc;
-    const long long E = (long long)n * k, NN = (long long)n * n;
-    PCHK(dalloc(lg, (size_t)E * 4));
-    PCHK(dalloc(out, (size_t)NN * 4));
-    rc = launch_forward(net, xb.as<unsigned short>(), E, lg.as<float>());
+    // The device needs the depot row and the candidate edges of the distance
+    // matrix, not the matrix, and returns the multiplier row by row into the
+    // pinned buffers, each copied out while the next is written.
+    SpaceUse use(net->space, net->stream);
+    PriorSpace &sp = net->space;
+    hipStream_t st = net->stream;
+    const size_t N = (size_t)n, E = N * (size_t)k;
+    // x, y, demand, depot row, lists and edges in one block, in this order
+    const size_t block = 4 * N + 2 * E;
+    PCHK(sp.init(SpaceUse::round(block * 4) + 3 * SpaceUse::round(N * 4) + 256 + SpaceUse::round(E * NFP * 2) +
+                 SpaceUse::round(E * 4)));
+    float *xd = use.take<float>(block), *yd = xd + N, *d0 = yd + 2 * N, *de = d0 + N + E;
+    const int *demd = reinterpret_cast<int *>(yd + N), *nnd = reinterpret_cast<int *>(d0 + N);
+    float *rad = use.take<float>(N), *ang = use.take<float>(N), *kd = use.take<float>(N), *Rm = use.take<float>(64);
+    unsigned short *xb = use.take<unsigned short>(E * NFP);
+    float *lg = use.take<float>(E);
+    PinnedStream up = {net, reinterpret_cast<unsigned char *>(xd)};
+    const struct { const void *p; } heads[4] = {{x}, {y}, {demand}, {dist}};   // dist: its first row
+    for (const auto &h : heads)
+        if ((rc = up.put(h.p, N * 4)) != ACO_OK) return rc;
+    for (size_t i = 0; i < N; ++i)
+        if ((rc = up.put(nn + i * nn_width, (size_t)k * 4)) != ACO_OK) return rc;
+    std::vector<float> edges((size_t)k);
+    for (size_t i = 0; i < N; ++i) {
+        for (int r = 0; r < k; ++r) edges[r] = dist[i * N + (size_t)nn[i * nn_width + r]];
+        if ((rc = up.put(edges.data(), (size_t)k * 4)) != ACO_OK) return rc;
+    }
+    if ((rc = up.flush()) != ACO_OK) return rc;
+    const DistEdges D = {d0, de, k};
+    hipLaunchKernelGGL(k_node_stats<DistEdges>, dim3((n + 255) / 256), dim3(256), 0, st, n, xd, yd, D, nnd, k, k, rad,
+                       ang, kd);
+    PCHK(hipGetLastError());
+    hipLaunchKernelGGL(k_node_reduce, dim3(1), dim3(256), 0, st, n, rad, kd, Rm);
+    PCHK(hipGetLastError());
+    hipLaunchKernelGGL(k_edge_features<DistEdges>, dim3((unsigned)((E + 255) / 256)), dim3(256), 0, st, n, k, D, nnd, k,
+                       demd, (float)capacity, rad, ang, kd, Rm, (float *)nullptr, xb);
+    PCHK(hipGetLastError());
+    rc = launch_forward(net, xb, (long long)E, lg);
     if (rc != ACO_OK) return rc;
     const float fl = floor_pow(floor, exponent);
-    hipLaunchKernelGGL(k_prior_fill, dim3((unsigned)((NN + 255) / 256)), dim3(256), 0, net->stream, NN, fl,
-                       out.as<float>());
-    PCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_prior_scatter, dim3((unsigned)((E + 255) / 256)), dim3(256), 0, net->stream, n, k,
-                       nnd.as<int>(), nn_width, lg.as<float>(), exponent, out.as<float>());
-    PCHK(hipGetLastError());
-    PCHK(hipMemcpyAsync(prior, out.p, (size_t)NN * 4, hipMemcpyDeviceToHost, net->stream));
-    PCHK(hipStreamSynchronize(net->stream));
-    return ACO_OK;
+    const int per = (int)std::min<size_t>(N, PriorSpace::kPin / (N * 4));
+    static_assert(65536 * 4 <= PriorSpace::kPin, "a row fits a buffer");
+    struct { int row, rows, buf; } out = {0, 0, 0};   // rows on their way
+    auto collect = [&]() -> int {
+        if (!out.rows) return ACO_OK;
+        PCHK(hipEventSynchronize(sp.done[out.buf]));
+        sp.busy[out.buf] = false;
+        memcpy(prior + (size_t)out.row * N, sp.pin[out.buf], (size_t)out.rows * N * 4);
+        return ACO_OK;
+    };
+    for (int row = 0; row < n; row += per) {
+        const int rows = std::min(per, n - row), buf = sp.cur;
+        unsigned char *b = nullptr;
+        PCHK(sp.take(b));
+        if (n <= kPriorRowLds)
+            hipLaunchKernelGGL(k_prior_rows<true>, dim3(rows), dim3(256), N * 4, st, n, row, k, nnd, k, lg, exponent, fl,
+                               reinterpret_cast<float *>(b));
+        else
+            hipLaunchKernelGGL(k_prior_rows<false>, dim3(rows), dim3(256), 0, st, n, row, k, nnd, k, lg, exponent, fl,
+                               reinterpret_cast<float *>(b));
+        PCHK(hipGetLastError());
+        PCHK(sp.used(st));
+        if ((rc = collect()) != ACO_OK) return rc;
+        out = {row, rows, buf};
+    }
+    return collect();
 }
 
 int aco_prior_apply(aco_ctx *ctx, aco_prior *net, const float *const *x, const float *const *y,
@@ -1059,15 +1348,16 @@ int aco_prior_apply(aco_ctx *ctx, aco_prior *net, const float *const *x, const f
         const long long En = (long long)n * k, NN = (long long)n * n;
         PCHK(hipMemcpyAsync(xd.p, x[b], (size_t)n * 4, hipMemcpyHostToDevice, st));
         PCHK(hipMemcpyAsync(yd.p, y[b], (size_t)n * 4, hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_node_stats, dim3((n + 255) / 256), dim3(256), 0, st, n, v.P, xd.as<float>(),
-                           yd.as<float>(), v.dist, nn, nnw, k, rad.as<float>(), ang.as<float>(), kd.as<float>());
+        const DistMatrix D = {v.dist, v.P};
+        hipLaunchKernelGGL(k_node_stats<DistMatrix>, dim3((n + 255) / 256), dim3(256), 0, st, n, xd.as<float>(),
+                           yd.as<float>(), D, nn, nnw, k, rad.as<float>(), ang.as<float>(), kd.as<float>());
         PCHK(hipGetLastError());
         hipLaunchKernelGGL(k_node_reduce, dim3(1), dim3(256), 0, st, n, rad.as<float>(), kd.as<float>(),
                            Rm.as<float>());
         PCHK(hipGetLastError());
-        hipLaunchKernelGGL(k_edge_features, dim3((unsigned)((En + 255) / 256)), dim3(256), 0, st, n, v.P, k,
-                           v.dist, nn, nnw, v.dem, (float)v.Q, rad.as<float>(), ang.as<float>(),
-                           kd.as<float>(), Rm.as<float>(), nullptr, xb.as<unsigned short>());
+        hipLaunchKernelGGL(k_edge_features<DistMatrix>, dim3((unsigned)((En + 255) / 256)), dim3(256), 0, st, n, k,
+                           D, nn, nnw, v.dem, (float)v.Q, rad.as<float>(), ang.as<float>(), kd.as<float>(),
+                           Rm.as<float>(), (float *)nullptr, xb.as<unsigned short>());
         PCHK(hipGetLastError());
         rc = launch_forward(net, xb.as<unsigned short>(), En, lg.as<float>(), st);
         if (rc != ACO_OK) return rc;
