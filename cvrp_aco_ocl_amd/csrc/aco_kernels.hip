@@ -258,7 +258,7 @@ __device__ __forceinline__ int greedy_pick(const DevProblem &p, const AntLds &L,
 __device__ __forceinline__ void tour_put(int *tour, int &tbuf, int step, int w, int lane)
 {
     if (lane == (step & 63)) tbuf = w;
-    if ((step & 63) == 63) tour[step - 63 + lane] = tbuf;
+    if (__builtin_expect((step & 63) == 63, 0)) tour[step - 63 + lane] = tbuf;
 }
 
 __device__ __forceinline__ void tour_close(int *tour, int &tbuf, int step, int lane)
@@ -577,7 +577,7 @@ __global__ __launch_bounds__(NW * 64) void k_construct_iroulette_waves(DevBatch 
         }
         step++;
         int wn;
-        if (top == 0) {
+        if (__builtin_expect(top == 0, 0)) {
             wn = 0;
             if (cur == 0) {
                 wn = uniform(greedy_pick<HAS_D>(p, L, tirow, drow, load, rdist, lane));
@@ -641,6 +641,87 @@ template <bool HAS_D> static IrChoice iroulette_choice(int n, bool staged)
 #undef IR
 }
 
+// The full-row greedy pick (greedy_pick: same choice) for instances of up to
+// 64 NODES nodes: lane l keeps the demands of nodes l, l + 64, ... and their
+// visited bits in registers, so what is feasible is known without an LDS
+// read and the largest total_info is found on 32-bit values, the lowest
+// index among equals afterwards.  A candidate roulette falls back to it in a
+// quarter of its steps at 1001 nodes (every route ends with one), a step of
+// about 1200 cycles of which the row's load is 300 and the scan 110.  With
+// this and a pick that runs straight through: 256 ants at 1001 nodes 687 ->
+// 582 us, 480 at 481 nodes 319 -> 248 us (284 -> 245 us staged), 242 at 242
+// nodes with a length limit 206 -> 147 us, 256 instances of 64 ants 1327 ->
+// 1158 us.  It is bound by the chain of a step's instructions.
+// WIDE as in greedy_pass: every load issued, or a chunk of 64 nodes with
+// nothing feasible reads the row's first element instead.
+template <int NODES> struct OwnNodes {
+    int dem[NODES > 0 ? NODES : 1];
+    unsigned open;
+    __device__ __forceinline__ void init(const int *demand, int n, int lane)
+    {
+        open = 0;
+#pragma unroll
+        for (int u = 0; u < NODES; ++u) {
+            const int i = lane + u * kLanes;
+            dem[u] = demand[i < n ? i : n - 1];
+            open |= i > 0 && i < n ? 1u << u : 0u;
+        }
+    }
+    __device__ __forceinline__ void visit(int w, int lane)
+    {
+        if (NODES > 0) open &= lane == (w & (kLanes - 1)) ? ~(1u << (w >> 6)) : ~0u;
+    }
+};
+
+template <bool HAS_D, bool WIDE, int NODES>
+__device__ __forceinline__ int greedy_own(const DevProblem &p, const AntLds &L, const OwnNodes<NODES> &own,
+                                          const float *tirow, const float *drow, int load, float rdist, int lane)
+{
+    static_assert(NODES > 0 && NODES <= 32, "one visited bit per node of a lane");
+    const int room = p.Q - load;
+    bool f[NODES], any = false;
+    u64 chunk[NODES];
+#pragma unroll
+    for (int u = 0; u < NODES; ++u) {
+        f[u] = ((own.open >> u) & 1u) & (own.dem[u] <= room);
+        any |= f[u];
+        if (!WIDE) chunk[u] = __ballot(f[u]);
+    }
+    if (!__ballot(any)) return 0;
+    float tv[NODES], dv[NODES], d0[NODES];
+#pragma unroll
+    for (int u = 0; u < NODES; ++u) {
+        const int i = lane + u * kLanes, ic = i < p.n ? i : p.n - 1;
+        const int ia = WIDE || chunk[u] ? ic : 0;
+        tv[u] = gload(tirow + ia);
+        dv[u] = HAS_D ? gload(drow + ia) : 0.0f;
+        d0[u] = HAS_D ? L.d0[ic] : 0.0f;
+    }
+    u32 val[NODES], best = 0;
+#pragma unroll
+    for (int u = 0; u < NODES; ++u) {
+        if (HAS_D) {
+            float t = rdist + (dv[u] + p.svc);
+            t = t + d0[u];
+            f[u] = f[u] & (t <= p.D);
+        }
+        val[u] = f[u] ? f2u(tv[u]) + 1u : 0u;
+        best = val[u] > best ? val[u] : best;
+    }
+    const u32 top = lanes_max_u32<kLanes>(best);
+    if (HAS_D && top == 0) return 0;
+    // the lowest node with that value
+    u32 low = 0;
+#pragma unroll
+    for (int u = 0; u < NODES; ++u) {
+        const u32 key = 0xFFFFu - (u32)(lane + u * kLanes);
+        low = val[u] == top && key > low ? key : low;
+    }
+    u64 tie = __ballot(best == top);
+    const u32 l = tie & (tie - 1) ? lanes_max_u32<kLanes>(low) : (u32)lane_i32((int)low, __builtin_ctzll(tie));
+    return (int)(0xFFFFu - l);
+}
+
 // Roulette over the k-nearest candidate row: lane c holds candidate c's
 // total_info masked by feasibility, a wavefront scan gives the wheel,
 // r = u * wheel[k-1] and the first lane whose prefix exceeds r wins (the
@@ -650,7 +731,8 @@ template <bool HAS_D> static IrChoice iroulette_choice(int n, bool staged)
 // demands and depot distances and this ant's visited flags (depot set).
 // The step loop synchronises the wave only, so the waves of a block may
 // build different ants.
-template <bool HAS_D, int RNG, bool WIDE = false>
+// NODES > 0: the fallback from registers (n <= 64 NODES), 0: greedy_pick.
+template <bool HAS_D, int RNG, bool WIDE = false, int NODES = 0>
 __device__ void construct_knn_ant(const DevProblem &p, const DevState &s, int a, const AntLds &L, int lane)
 {
     const int n = p.n, k = p.k;
@@ -661,9 +743,11 @@ __device__ void construct_knn_ant(const DevProblem &p, const DevState &s, int a,
     int cur = 0, load = 0, vcnt = 1, step = 0, fb = 0, tbuf = 0;
     float rdist = 0.0f, tdist = 0.0f;
     float ublk = 0.0f;   // Philox draws of steps step+1 .. step+64, refreshed every 64 steps
+    OwnNodes<NODES> own;
+    own.init(L.dem, n, lane);
     while (vcnt < n) {
         step++;
-        if (RNG == kRngPhilox && ((step - 1) & 63) == 0) ublk = philox_block(seed, iter, (u32)a, (u32)step, lane);
+        if (RNG == kRngPhilox && __builtin_expect(((step - 1) & 63) == 0, 0)) ublk = philox_block(seed, iter, (u32)a, (u32)step, lane);
         // candidate id, its total_info and (with a length limit) d(cur, id):
         // one contiguous read each, issued together; lanes >= k read the row's
         // last entry and are masked.  total_info is finite and >= 0, so the
@@ -677,36 +761,32 @@ __device__ void construct_knn_ant(const DevProblem &p, const DevState &s, int a,
         const float pj = tj * (ok ? 1.0f : 0.0f);
         const float x = wave_scan_f32(pj, lane);
         const float total = lane_f32(x, k - 1);
-        int w, dw;
-        float dcw;
-        if (total > 0.0f) {
-            const float u = RNG == kRngPhilox ? lane_f32(ublk, (step - 1) & 63) : pm_ran01(z);
-            const float r = u * total;
-            // only lanes with mass: the scan's additions are grouped by the DPP
-            // tree, so a lane without mass can round above its left
-            // neighbour's prefix and must not be taken
-            const u64 m1 = __ballot(pj > 0.0f && x > r);
-            int wc;
-            if (m1) {
-                wc = __ffsll((unsigned long long)m1) - 1;
-            } else {
-                const u64 m2 = __ballot(pj > 0.0f);
-                wc = 63 - __clzll((long long)m2);
-            }
-            w = lane_i32(j, wc);
-            dw = lane_i32(dj, wc);
-            dcw = HAS_D ? lane_f32(dcj, wc) : 0.0f;
-        } else {
+        // Picked before it is known that there is mass, so that the common
+        // step runs straight through (a jump costs as much as the scan).
+        // Only lanes with mass: the scan's additions are grouped by the DPP
+        // tree, so a lane without mass can round above its left neighbour's
+        // prefix and must not be taken.
+        const u64 mass = __ballot(pj > 0.0f);
+        int zn = z;
+        const float r = (RNG == kRngPhilox ? lane_f32(ublk, (step - 1) & 63) : pm_ran01(zn)) * total;
+        const u64 over = __ballot(x > r) & mass;
+        const int wc = over ? __builtin_ctzll(over) : 63 - __builtin_clzll(mass | 1ull);
+        int w = lane_i32(j, wc), dw = lane_i32(dj, wc);
+        float dcw = HAS_D ? lane_f32(dcj, wc) : 0.0f;
+        if (__builtin_expect(mass == 0, 0)) {
             const float *drow = p.dist + (size_t)cur * p.P;
-            w = greedy_pick<HAS_D, WIDE>(p, L, s.tinfo + (size_t)cur * p.P, drow, load, rdist, lane);
+            const float *tirow = s.tinfo + (size_t)cur * p.P;
+            if constexpr (NODES > 0) w = greedy_own<HAS_D, WIDE, NODES>(p, L, own, tirow, drow, load, rdist, lane);
+            else w = greedy_pick<HAS_D, WIDE>(p, L, tirow, drow, load, rdist, lane);
             fb++;
             w = uniform(w);
             // scalar reads keep their waits on this path (see the staged
             // kernel)
             dw = uniform(L.dem[w]);
             dcw = HAS_D ? drow[w] : 0.0f;
+        } else {
+            z = zn;
         }
-        w = uniform(w);
         if (w == 0) {
             load = 0;
             rdist = 0.0f;
@@ -716,6 +796,7 @@ __device__ void construct_knn_ant(const DevProblem &p, const DevState &s, int a,
             vcnt++;
         }
         if (lane == 0) L.vis[w] = 1;
+        own.visit(w, lane);
         tdist = tdist + dcw;
         tour_put(tour, tbuf, step, w, lane);
         cur = w;
@@ -739,7 +820,7 @@ __device__ void construct_knn_ant(const DevProblem &p, const DevState &s, int a,
     }
 }
 
-template <bool HAS_D, int RNG, bool WIDE>
+template <bool HAS_D, int RNG, bool WIDE, int NODES>
 __global__ __launch_bounds__(64) void k_construct_knn(DevBatch bt)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -748,7 +829,7 @@ __global__ __launch_bounds__(64) void k_construct_knn(DevBatch bt)
     AntLds L = ant_lds(smem, n, false);
     ant_lds_fill<false>(p, L, n, lane);
     __syncthreads();
-    construct_knn_ant<HAS_D, RNG, WIDE>(p, s, a, L, lane);
+    construct_knn_ant<HAS_D, RNG, WIDE, NODES>(p, s, a, L, lane);
 }
 
 // The same roulette with the instance's candidate table staged in LDS, for
@@ -765,7 +846,7 @@ __global__ __launch_bounds__(64) void k_construct_knn(DevBatch bt)
 // LDS: dem[n] | vis[A][pitch] | ent[rows * k].
 __device__ __forceinline__ int construct_vis_pitch(int n) { return (n + 15) & ~15; }
 
-template <int RNG, int A>
+template <int RNG, int A, int NODES>
 __global__ __launch_bounds__(64 * A) void k_construct_knn_lds(DevBatch bt, int rows_cap)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -813,9 +894,11 @@ __global__ __launch_bounds__(64 * A) void k_construct_knn_lds(DevBatch bt, int r
     int cur = 0, load = 0, vcnt = 1, step = 0, fb = 0, tbuf = 0;
     float ublk = 0.0f;   // Philox draws of steps step+1 .. step+64, refreshed every 64 steps
     const int c = lane < k ? lane : k - 1;   // lanes >= k read the row's last entry and are masked
+    OwnNodes<NODES> own;
+    own.init(dem, n, lane);
     while (vcnt < n) {
         step++;
-        if (RNG == kRngPhilox && ((step - 1) & 63) == 0) ublk = philox_block(seed, iter, (u32)a, (u32)step, lane);
+        if (RNG == kRngPhilox && __builtin_expect(((step - 1) & 63) == 0, 0)) ublk = philox_block(seed, iter, (u32)a, (u32)step, lane);
         int j, dj;
         float tj;
         if (cur < rows) {
@@ -835,33 +918,30 @@ __global__ __launch_bounds__(64 * A) void k_construct_knn_lds(DevBatch bt, int r
         const float pj = tj * (ok ? 1.0f : 0.0f);
         const float x = wave_scan_f32(pj, lane);
         const float total = lane_f32(x, k - 1);
-        int w, dw;
-        if (total > 0.0f) {
-            const float u = RNG == kRngPhilox ? lane_f32(ublk, (step - 1) & 63) : pm_ran01(z);
-            const float r = u * total;
-            // only lanes with mass: the scan's additions are grouped by the DPP
-            // tree, so a lane without mass can round above its left
-            // neighbour's prefix and must not be taken
-            const u64 m1 = __ballot(pj > 0.0f && x > r);
-            int wc;
-            if (m1) {
-                wc = __ffsll((unsigned long long)m1) - 1;
-            } else {
-                const u64 m2 = __ballot(pj > 0.0f);
-                wc = 63 - __clzll((long long)m2);
-            }
-            w = lane_i32(j, wc);
-            dw = lane_i32(dj, wc);
-        } else {
-            w = greedy_pick<false, false, true>(p, L, s.tinfo + (size_t)cur * p.P, nullptr, load, 0.0f, lane);
+        // Picked before it is known that there is mass, so that the common
+        // step runs straight through (a jump costs as much as the scan).
+        // Only lanes with mass: the scan's additions are grouped by the DPP
+        // tree, so a lane without mass can round above its left neighbour's
+        // prefix and must not be taken.
+        const u64 mass = __ballot(pj > 0.0f);
+        int zn = z;
+        const float r = (RNG == kRngPhilox ? lane_f32(ublk, (step - 1) & 63) : pm_ran01(zn)) * total;
+        const u64 over = __ballot(x > r) & mass;
+        const int wc = over ? __builtin_ctzll(over) : 63 - __builtin_clzll(mass | 1ull);
+        int w = lane_i32(j, wc), dw = lane_i32(dj, wc);
+        if (__builtin_expect(mass == 0, 0)) {
+            const float *tirow = s.tinfo + (size_t)cur * p.P;
+            if constexpr (NODES > 0) w = greedy_own<false, false, NODES>(p, L, own, tirow, nullptr, load, 0.0f, lane);
+            else w = greedy_pick<false, false, true>(p, L, tirow, nullptr, load, 0.0f, lane);
             fb++;
             w = uniform(w);
             // scalar, so the wait for this read stays on this path: a vector
             // result would place it where the paths join, where every step
             // would also wait for the visited-flag store
             dw = uniform(dem[w]);
+        } else {
+            z = zn;
         }
-        w = uniform(w);
         if (w == 0) {
             load = 0;
         } else {
@@ -872,6 +952,7 @@ __global__ __launch_bounds__(64 * A) void k_construct_knn_lds(DevBatch bt, int r
         // one wave complete in order, and the store and the loads use the
         // same array, so the compiler keeps their order
         if (lane == 0) vis[w] = 1;
+        own.visit(w, lane);
         tour_put(tour, tbuf, step, w, lane);
         cur = w;
         __builtin_amdgcn_wave_barrier();
@@ -933,34 +1014,44 @@ static hipError_t max_static_lds(const void *const *fns, int count, size_t &byte
 hipError_t construct_static_lds(size_t &bytes)
 {
     const void *fns[] = {(const void *)k_construct_iroulette<false>, (const void *)k_construct_iroulette<true>,
-                         (const void *)k_construct_knn<false, kRngPhilox, true>,
-                         (const void *)k_construct_knn<true, kRngPhilox, true>,
-                         (const void *)k_construct_knn<false, kRngParkMiller, true>,
-                         (const void *)k_construct_knn<true, kRngParkMiller, true>,
-                         (const void *)k_construct_knn<false, kRngPhilox, false>,
-                         (const void *)k_construct_knn<true, kRngPhilox, false>,
-                         (const void *)k_construct_knn<false, kRngParkMiller, false>,
-                         (const void *)k_construct_knn<true, kRngParkMiller, false>,
-                         (const void *)k_construct_knn_lds<kRngPhilox, 1>, (const void *)k_construct_knn_lds<kRngPhilox, 2>,
-                         (const void *)k_construct_knn_lds<kRngPhilox, 4>,
-                         (const void *)k_construct_knn_lds<kRngParkMiller, 1>,
-                         (const void *)k_construct_knn_lds<kRngParkMiller, 2>,
-                         (const void *)k_construct_knn_lds<kRngParkMiller, 4>};
+#define KN(D, R, S) (const void *)k_construct_knn<D, R, S, 0>, (const void *)k_construct_knn<D, R, S, 8>, \
+                    (const void *)k_construct_knn<D, R, S, 16>
+#define KL(R, A) (const void *)k_construct_knn_lds<R, A, 0>, (const void *)k_construct_knn_lds<R, A, 8>, \
+                 (const void *)k_construct_knn_lds<R, A, 16>
+                         KN(false, kRngPhilox, true), KN(true, kRngPhilox, true),
+                         KN(false, kRngParkMiller, true), KN(true, kRngParkMiller, true),
+                         KN(false, kRngPhilox, false), KN(true, kRngPhilox, false),
+                         KN(false, kRngParkMiller, false), KN(true, kRngParkMiller, false),
+                         KL(kRngPhilox, 1), KL(kRngPhilox, 2), KL(kRngPhilox, 4),
+                         KL(kRngParkMiller, 1), KL(kRngParkMiller, 2), KL(kRngParkMiller, 4)};
+#undef KN
+#undef KL
     return max_static_lds(fns, (int)(sizeof(fns) / sizeof(fns[0])), bytes);
 }
 
 hipError_t launch_construct(const DevBatch &b, int selection, int rng, int apb, int k, hipStream_t st)
 {
+    // nodes per lane of the roulette's fallback (0: instances past 1024 nodes)
+    const int nodes = b.max_n <= 512 ? 8 : b.max_n <= 1024 ? 16 : 0;
     if (apb > 0) {
         const int rows = construct_staged_rows(b.max_n, k, apb, b.cons_lds_budget);
         if (rows < 0) return hipErrorInvalidValue;
         const size_t lds = construct_lds_staged_bytes(b.max_n, k, apb, b.cons_lds_budget);
         const dim3 grid(b.ants / apb), block(kLanes * apb);
-#define CKL(R, A) hipLaunchKernelGGL((k_construct_knn_lds<R, A>), grid, block, lds, st, b, rows)
+#define CKL(R, A)                                                                                            \
+    do {                                                                                                     \
+        if (nodes == 8) hipLaunchKernelGGL((k_construct_knn_lds<R, A, 8>), grid, block, lds, st, b, rows);        \
+        else if (nodes == 16) hipLaunchKernelGGL((k_construct_knn_lds<R, A, 16>), grid, block, lds, st, b, rows); \
+        else hipLaunchKernelGGL((k_construct_knn_lds<R, A, 0>), grid, block, lds, st, b, rows);                   \
+    } while (0)
         if (rng == kRngPhilox) {
-            if (apb == 1) CKL(kRngPhilox, 1); else if (apb == 2) CKL(kRngPhilox, 2); else CKL(kRngPhilox, 4);
+            if (apb == 1) CKL(kRngPhilox, 1);
+            else if (apb == 2) CKL(kRngPhilox, 2);
+            else CKL(kRngPhilox, 4);
         } else {
-            if (apb == 1) CKL(kRngParkMiller, 1); else if (apb == 2) CKL(kRngParkMiller, 2); else CKL(kRngParkMiller, 4);
+            if (apb == 1) CKL(kRngParkMiller, 1);
+            else if (apb == 2) CKL(kRngParkMiller, 2);
+            else CKL(kRngParkMiller, 4);
         }
 #undef CKL
         return hipGetLastError();
@@ -989,14 +1080,25 @@ hipError_t launch_construct(const DevBatch &b, int selection, int rng, int apb, 
         // latency (at most one ant's wave per SIMD); with more ants the
         // device is busy and the narrow pass's fewer bytes win
         const bool spec = b.ants <= 4 * b.cus;
-#define CK(D, R, S) hipLaunchKernelGGL((k_construct_knn<D, R, S>), grid, block, lds, st, b)
+#define CKN(D, R, S)                                                                              \
+    do {                                                                                          \
+        if (nodes == 8) hipLaunchKernelGGL((k_construct_knn<D, R, S, 8>), grid, block, lds, st, b);        \
+        else if (nodes == 16) hipLaunchKernelGGL((k_construct_knn<D, R, S, 16>), grid, block, lds, st, b); \
+        else hipLaunchKernelGGL((k_construct_knn<D, R, S, 0>), grid, block, lds, st, b);                   \
+    } while (0)
+#define CK(D, R)                   \
+    do {                           \
+        if (spec) CKN(D, R, true); \
+        else CKN(D, R, false);     \
+    } while (0)
         if (rng == kRngPhilox) {
-            if (b.has_d) { if (spec) CK(true, kRngPhilox, true); else CK(true, kRngPhilox, false); }
-            else { if (spec) CK(false, kRngPhilox, true); else CK(false, kRngPhilox, false); }
+            if (b.has_d) CK(true, kRngPhilox);
+            else CK(false, kRngPhilox);
         } else {
-            if (b.has_d) { if (spec) CK(true, kRngParkMiller, true); else CK(true, kRngParkMiller, false); }
-            else { if (spec) CK(false, kRngParkMiller, true); else CK(false, kRngParkMiller, false); }
+            if (b.has_d) CK(true, kRngParkMiller);
+            else CK(false, kRngParkMiller);
         }
+#undef CKN
 #undef CK
     }
     return hipGetLastError();
