@@ -248,7 +248,7 @@ __host__ __device__ inline int pm_jump(int z, unsigned long long t)
     return (int)(r * (unsigned long long)(unsigned)z % M);
 }
 // compute_nn_lists for `count` instances on the device (host arrays in and
-// out, one thread per row, the reference's sort steps); ACO_OK or an error.
+// out, one wave per row, the reference's sort steps); ACO_OK or an error.
 int gpu_nn_lists(hipStream_t st, int count, const int *n, const float *const *dist, const int *width,
                  int tie, int *const *out);
 // the same from device distances (rows of pitch pitch[b]) into device arrays

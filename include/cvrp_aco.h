@@ -270,7 +270,7 @@ int aco_compute_distances_batch(int32_t count, const int32_t *n, const double *c
  * tie 0 = the reference's quicksort order, tie 1 = (distance, index) */
 int aco_compute_nn_lists(int32_t n, const float *dist, int32_t nn, int32_t tie, int32_t *out);
 /* The same lists for `count` instances at once on the current HIP device
- * (compute_nn_lists, vrpHelper.cpp:188-236; one thread per row, the same
+ * (compute_nn_lists, vrpHelper.cpp:188-236; one wave per row, the same
  * sort steps, so the result equals aco_compute_nn_lists instance by
  * instance).  n[b], dist[b] (n[b] x n[b] host array), nn[b] (1..n[b]-2)
  * entries per row into out[b] (n[b] x nn[b] host array).  aco_create uses
