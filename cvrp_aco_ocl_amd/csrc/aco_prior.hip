@@ -48,7 +48,6 @@ constexpr int OFF_W1 = 0, OFF_B1 = H * NF, OFF_W2 = OFF_B1 + H, OFF_B2 = OFF_W2 
 static_assert(NP == ACO_PRIOR_PARAMS, "parameter layout");
 constexpr int NPL = NP + 1;         // partial row: gradient, then the loss sum
 constexpr int kThreads = 256, kWaves = kThreads / 64;
-constexpr int kTilesPerWave = 4;    // training: 64 edges per wave per launch
 constexpr int kMaxBatch = 65536;
 
 typedef short v4s __attribute__((ext_vector_type(4)));
@@ -97,25 +96,35 @@ struct NetLds {
     alignas(16) unsigned short tr[kWaves][9][16][16];
 };
 
+// Every global read is requested before the first LDS write (8 or 16 bytes
+// each): an element at a time, a block waited for twenty of them in turn.
 __device__ void load_net(NetLds &S, const unsigned short *wb, const float *pf)
 {
+    typedef unsigned short v8u __attribute__((ext_vector_type(8)));
+    static_assert(H == 64 && NF == 12 && NFP == 16 && kThreads == 256, "one pass of the block");
+    static_assert(OFF_W1 % 8 == 0 && OFF_W2 % 8 == 0, "aligned vector reads");
     const int t = threadIdx.x;
-    for (int e = t; e < H * NFP; e += kThreads) {
-        const int o = e / NFP, f = e % NFP;
-        S.w1[o][f] = f < NF ? wb[OFF_W1 + o * NF + f] : (unsigned short)0;
-    }
-    for (int e = t; e < H * H; e += kThreads) {
-        const int o = e / H, i = e % H;
-        const unsigned short w = wb[OFF_W2 + e];
-        S.w2[o][i] = w;
-        S.w2t[i][o] = w;
-    }
-    for (int e = t; e < H; e += kThreads) {
-        S.b1[e] = pf[OFF_B1 + e];
-        S.b2[e] = pf[OFF_B2 + e];
-        S.w3[e] = bf2f(wb[OFF_W3 + e]);
-    }
-    if (t == 0) S.b3 = pf[OFF_B3];
+    const v8u *w2 = reinterpret_cast<const v8u *>(wb + OFF_W2);
+    const v8u a0 = w2[t], a1 = w2[t + kThreads];
+    const v4s c = reinterpret_cast<const v4s *>(wb + OFF_W1)[t < H * NF / 4 ? t : 0];
+    const int q = t & (H - 1), part = t / H;
+    const float b = part < 2 ? pf[(part == 0 ? OFF_B1 : OFF_B2) + q] : 0.0f;
+    const unsigned short w3 = wb[OFF_W3 + q];
+    const float b3 = pf[OFF_B3];
+    auto put = [&](int e, v8u a) {   // elements 8e .. 8e + 7
+        const int o = e / (H / 8), i0 = 8 * (e % (H / 8));
+        *reinterpret_cast<v8u *>(&S.w2[o][i0]) = a;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) S.w2t[i0 + k][o] = a[k];
+    };
+    put(t, a0);
+    put(t + kThreads, a1);
+    if (t < H * NF / 4) *reinterpret_cast<v4s *>(&S.w1[t / 3][4 * (t % 3)]) = c;
+    if (part == 0) S.b1[q] = b;
+    else if (part == 1) S.b2[q] = b;
+    else if (part == 2) S.w3[q] = bf2f(w3);
+    else *reinterpret_cast<v4s *>(&S.w1[q][NF]) = v4s{0, 0, 0, 0};
+    if (t == 0) S.b3 = b3;
     __syncthreads();
 }
 
@@ -278,9 +287,13 @@ __global__ __launch_bounds__(kThreads) void k_forward(const unsigned short *xb, 
     }
 }
 
-// Fused forward + backward over kTilesPerWave tiles of the batch
-// (positions [0, Eb) of idx, or of the data in order without one); writes
-// one partial row per wave.
+// Fused forward + backward over one tile of 16 edges per wave (positions
+// [0, Eb) of idx, or of the data in order without one); the block's waves add
+// their gradients in LDS in wave order and write one partial row.  A wave's
+// chain of products, conversions and transposes is the launch's length, so a
+// batch is spread over as many waves as it has tiles: 16384 edges on 64
+// blocks of four tiles per wave took 36 us, on 256 blocks of one 19.5 us, with
+// as many partial rows.
 __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, const float *label,
                                                     const int *idx, int Eb,
                                                     const unsigned short *wb, const float *pf,
@@ -289,8 +302,7 @@ __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, co
     __shared__ NetLds S;
     load_net(S, wb, pf);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
-    const int gw = blockIdx.x * kWaves + w;
-    const int tiles = (Eb + 15) / 16;
+    const int tile = blockIdx.x * kWaves + w, tiles = (Eb + 15) / 16;
     unsigned short(*T)[16][16] = S.tr[w];
     const v4f zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
     v4f dW2[4][4], dW1[4], db1[4], db2[4], dw3[4];
@@ -301,9 +313,7 @@ __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, co
         for (int b = 0; b < 4; ++b) dW2[a][b] = zero4;
     }
     float db3 = 0.0f, loss = 0.0f;
-    for (int tt = 0; tt < kTilesPerWave; ++tt) {
-        const int tile = gw * kTilesPerWave + tt;
-        if (tile >= tiles) break;
+    if (tile < tiles) {
         const int pos = tile * 16 + r;
         const bool valid = pos < Eb;
         const int e = !valid ? 0 : idx ? idx[pos] : pos;
@@ -366,46 +376,69 @@ __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, co
             dW1[ot] = mfma(a1, xT, dW1[ot]);
         }
     }
-    // per-wave partial row
-    float *P = partials + (size_t)gw * NPL;
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int it = 0; it < 4; ++it)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) P[OFF_W2 + (16 * mt + 4 * g + j) * H + 16 * it + r] = dW2[mt][it][j];
-#pragma unroll
-    for (int ot = 0; ot < 4; ++ot)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (r < NF) P[OFF_W1 + (16 * ot + 4 * g + j) * NF + r] = dW1[ot][j];
     // bias / w3 gradients: sum over the 16 edge lanes of each row group
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float a = db1[t][j], b = db2[t][j], c = dw3[t][j];
+        for (int j = 0; j < 4; ++j)
 #pragma unroll
             for (int o = 1; o < 16; o <<= 1) {
-                a += __shfl_xor(a, o);
-                b += __shfl_xor(b, o);
-                c += __shfl_xor(c, o);
+                db1[t][j] += __shfl_xor(db1[t][j], o);
+                db2[t][j] += __shfl_xor(db2[t][j], o);
+                dw3[t][j] += __shfl_xor(dw3[t][j], o);
             }
-            if (r == 0) {
-                P[OFF_B1 + 16 * t + 4 * g + j] = a;
-                P[OFF_B2 + 16 * t + 4 * g + j] = b;
-                P[OFF_W3 + 16 * t + 4 * g + j] = c;
-            }
-        }
 #pragma unroll
     for (int o = 1; o < 16; o <<= 1) {
         db3 += __shfl_xor(db3, o);
         loss += __shfl_xor(loss, o);
     }
-    if (lane == 0) {
-        P[OFF_B3] = db3;
-        P[NP] = loss * invE;
+    // the block's partial row, wave after wave: a wave reads its 80 sums
+    // together before it writes any (an add at a time is a chain of LDS round
+    // trips)
+    __shared__ float sum[NPL];
+    for (int turn = 0; turn < kWaves; ++turn) {
+        if (turn == w) {
+            const bool more = turn > 0;
+            const int o2 = OFF_W2 + 4 * g * H + r, o1 = OFF_W1 + 4 * g * NF + (r < NF ? r : 0), ob = 4 * g;
+            float s2[4][4][4], s1[4][4], sb[3][4][4], s3 = 0.0f, sl = 0.0f;
+            if (more) {
+#pragma unroll
+                for (int a = 0; a < 4; ++a)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) s2[a][b][j] = sum[o2 + (16 * a + j) * H + 16 * b];
+                        s1[a][j] = sum[o1 + (16 * a + j) * NF];
+                        sb[0][a][j] = sum[OFF_B1 + ob + 16 * a + j];
+                        sb[1][a][j] = sum[OFF_B2 + ob + 16 * a + j];
+                        sb[2][a][j] = sum[OFF_W3 + ob + 16 * a + j];
+                    }
+                s3 = sum[OFF_B3];
+                sl = sum[NP];
+            }
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+                        sum[o2 + (16 * a + j) * H + 16 * b] = more ? s2[a][b][j] + dW2[a][b][j] : dW2[a][b][j];
+                    if (r < NF) sum[o1 + (16 * a + j) * NF] = more ? s1[a][j] + dW1[a][j] : dW1[a][j];
+                    if (r == 0) {
+                        sum[OFF_B1 + ob + 16 * a + j] = more ? sb[0][a][j] + db1[a][j] : db1[a][j];
+                        sum[OFF_B2 + ob + 16 * a + j] = more ? sb[1][a][j] + db2[a][j] : db2[a][j];
+                        sum[OFF_W3 + ob + 16 * a + j] = more ? sb[2][a][j] + dw3[a][j] : dw3[a][j];
+                    }
+                }
+            if (lane == 0) {
+                sum[OFF_B3] = more ? s3 + db3 : db3;
+                sum[NP] = more ? sl + loss * invE : loss * invE;
+            }
+        }
+        __syncthreads();
     }
+    float *P = partials + (size_t)blockIdx.x * NPL;
+    for (int i = threadIdx.x; i < NPL; i += kThreads) P[i] = sum[i];
 }
 
 // Per parameter: the sum of the partial rows in a fixed order (runs of
@@ -663,9 +696,9 @@ using namespace cvrp::prior;
 // than kKeep, and four pinned buffers of 512 KB.  Pageable copies of this
 // size cost 25 to 60 us each whatever they hold, allocations of 2 MB and more
 // 25 us; a gradient made six of the first and two of the second.  Gradient
-// over 16384 edges 202 -> 99 us, multiplier of 501 nodes 200 -> 117 us, eight
-// training steps of 16384 edges 945 -> 700 us; what is left is the copy into
-// the buffers, the launches and the kernels (50 us of the gradient).
+// over 16384 edges 202 -> 82 us, multiplier of 501 nodes 200 -> 117 us, eight
+// training steps of 16384 edges 945 -> 556 us; what is left is the copy into
+// the buffers, the launches and the kernels (30 us of the gradient).
 struct PriorSpace {
     static constexpr size_t kPin = size_t(512) << 10, kKeep = size_t(64) << 20;
     std::mutex mutex;
@@ -900,15 +933,13 @@ static int launch_batch(aco_prior *net, const unsigned short *xb, const float *l
                         int Eb, float pos_weight, float *partials, float *grad_out, float *loss_out,
                         bool update, const AdamArgs &aa)
 {
-    const int tiles = (Eb + 15) / 16;
-    const int waves = (tiles + kTilesPerWave - 1) / kTilesPerWave;
-    const int blocks = (waves + kWaves - 1) / kWaves;
+    const int blocks = ((Eb + 15) / 16 + kWaves - 1) / kWaves;
     hipLaunchKernelGGL(k_train, dim3(blocks), dim3(kThreads), 0, net->stream, xb, label, idx, Eb,
                        net->wb, net->pf, pos_weight, 1.0f / (float)Eb, partials);
     PCHK(hipGetLastError());
     hipLaunchKernelGGL(k_reduce_adam, dim3((NPL + kReduceParams - 1) / kReduceParams),
                        dim3(kReduceParams * kReduceGroups), 0, net->stream, partials,
-                       blocks * kWaves, net->pf, net->m, net->v, net->wb, grad_out, loss_out,
+                       blocks, net->pf, net->m, net->v, net->wb, grad_out, loss_out,
                        update ? 1 : 0, aa);
     PCHK(hipGetLastError());
     return ACO_OK;
@@ -916,10 +947,8 @@ static int launch_batch(aco_prior *net, const unsigned short *xb, const float *l
 
 static size_t partial_bytes(int Eb)
 {
-    const int tiles = (Eb + 15) / 16;
-    const int waves = (tiles + kTilesPerWave - 1) / kTilesPerWave;
-    const int blocks = (waves + kWaves - 1) / kWaves;
-    return (size_t)blocks * kWaves * NPL * sizeof(float);
+    const int blocks = ((Eb + 15) / 16 + kWaves - 1) / kWaves;
+    return (size_t)blocks * NPL * sizeof(float);
 }
 
 extern "C" {
