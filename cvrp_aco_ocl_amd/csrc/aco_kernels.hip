@@ -581,6 +581,10 @@ __global__ __launch_bounds__(NW * 64) void k_construct_iroulette_waves(DevBatch 
             wn = 0;
             if (cur == 0) {
                 wn = uniform(greedy_pick<HAS_D>(p, L, tirow, drow, load, rdist, lane));
+                // every wave picks from the block's visited flags: none may
+                // mark the node below while another still reads them (top
+                // and cur are the block's, so all waves are here)
+                if (NW > 1) __syncthreads();
                 fb++;
             }
             dw = uniform(L.dem[wn]);
@@ -598,7 +602,8 @@ __global__ __launch_bounds__(NW * 64) void k_construct_iroulette_waves(DevBatch 
         }
 #pragma unroll
         for (int j = 0; j < C; ++j) open &= node[j] == wn ? ~(1u << j) : ~0u;
-        if (lane == 0) L.vis[wn] = 1;   // each wave for itself (greedy_pick)
+        // the same flag from every wave, so a wave's next pick sees its own write
+        if (lane == 0) L.vis[wn] = 1;
         tdist = tdist + dcw;            // without a limit: summed afterwards
         if (w == 0) tour_put(tour, tbuf, step, wn, lane);
         cur = wn;
