@@ -727,6 +727,10 @@ __device__ __forceinline__ int greedy_own(const DevProblem &p, const AntLds &L, 
     return (int)(0xFFFFu - l);
 }
 
+// v > 0 for a uniform v, in scalar integer arithmetic (false for NaN): the
+// bit patterns of the smallest denormal to infinity.
+__device__ __forceinline__ bool positive(float v) { return (u32)uniform((int)f2u(v)) - 1u < 0x7f800000u; }
+
 // Roulette over the k-nearest candidate row: lane c holds candidate c's
 // total_info masked by feasibility, a wavefront scan gives the wheel,
 // r = u * wheel[k-1] and the first lane whose prefix exceeds r wins (the
@@ -755,8 +759,9 @@ __device__ void construct_knn_ant(const DevProblem &p, const DevState &s, int a,
         if (RNG == kRngPhilox && __builtin_expect(((step - 1) & 63) == 0, 0)) ublk = philox_block(seed, iter, (u32)a, (u32)step, lane);
         // candidate id, its total_info and (with a length limit) d(cur, id):
         // one contiguous read each, issued together; lanes >= k read the row's
-        // last entry and are masked.  total_info is finite and >= 0, so the
-        // product by 1 or 0 is exact and keeps its load unconditional.
+        // last entry and are masked.  The product by 1 or 0 is exact for finite
+        // total_info >= 0 and keeps its load unconditional (a masked infinity
+        // makes the total NaN: no wheel).
         const int e = cur * k + (lane < k ? lane : k - 1);
         const int j = gload(p.nnk + e);
         const float tj = gload(s.tiknn + e);
@@ -766,7 +771,7 @@ __device__ void construct_knn_ant(const DevProblem &p, const DevState &s, int a,
         const float pj = tj * (ok ? 1.0f : 0.0f);
         const float x = wave_scan_f32(pj, lane);
         const float total = lane_f32(x, k - 1);
-        // Picked before it is known that there is mass, so that the common
+        // Picked before it is known that there is a wheel, so that the common
         // step runs straight through (a jump costs as much as the scan).
         // Only lanes with mass: the scan's additions are grouped by the DPP
         // tree, so a lane without mass can round above its left neighbour's
@@ -778,7 +783,7 @@ __device__ void construct_knn_ant(const DevProblem &p, const DevState &s, int a,
         const int wc = over ? __builtin_ctzll(over) : 63 - __builtin_clzll(mass | 1ull);
         int w = lane_i32(j, wc), dw = lane_i32(dj, wc);
         float dcw = HAS_D ? lane_f32(dcj, wc) : 0.0f;
-        if (__builtin_expect(mass == 0, 0)) {
+        if (__builtin_expect(!positive(total), 0)) {
             const float *drow = p.dist + (size_t)cur * p.P;
             const float *tirow = s.tinfo + (size_t)cur * p.P;
             if constexpr (NODES > 0) w = greedy_own<HAS_D, WIDE, NODES>(p, L, own, tirow, drow, load, rdist, lane);
@@ -918,12 +923,13 @@ __global__ __launch_bounds__(64 * A) void k_construct_knn_lds(DevBatch bt, int r
             dj = dem[j];
         }
         const bool ok = (lane < k) & (vis[j] == 0) & (load + dj <= p.Q);   // feasible_mask<false>
-        // total_info is finite and >= 0, so x * 1 = x and x * 0 = 0 exactly; the
+        // x * 1 = x and x * 0 = 0 exactly for finite total_info >= 0 (a masked
+        // infinity makes the total NaN: no wheel); the
         // product keeps its load unconditional (one 8-byte LDS read with the id)
         const float pj = tj * (ok ? 1.0f : 0.0f);
         const float x = wave_scan_f32(pj, lane);
         const float total = lane_f32(x, k - 1);
-        // Picked before it is known that there is mass, so that the common
+        // Picked before it is known that there is a wheel, so that the common
         // step runs straight through (a jump costs as much as the scan).
         // Only lanes with mass: the scan's additions are grouped by the DPP
         // tree, so a lane without mass can round above its left neighbour's
@@ -934,7 +940,7 @@ __global__ __launch_bounds__(64 * A) void k_construct_knn_lds(DevBatch bt, int r
         const u64 over = __ballot(x > r) & mass;
         const int wc = over ? __builtin_ctzll(over) : 63 - __builtin_clzll(mass | 1ull);
         int w = lane_i32(j, wc), dw = lane_i32(dj, wc);
-        if (__builtin_expect(mass == 0, 0)) {
+        if (__builtin_expect(!positive(total), 0)) {
             const float *tirow = s.tinfo + (size_t)cur * p.P;
             if constexpr (NODES > 0) w = greedy_own<false, false, NODES>(p, L, own, tirow, nullptr, load, 0.0f, lane);
             else w = greedy_pick<false, false, true>(p, L, tirow, nullptr, load, 0.0f, lane);
