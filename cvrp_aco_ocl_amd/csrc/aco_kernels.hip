@@ -830,8 +830,14 @@ __device__ void construct_knn_ant(const DevProblem &p, const DevState &s, int a,
     }
 }
 
+// With a length limit and sixteen nodes per lane the narrow shape, which is
+// for more ants than SIMDs, is held to 128 registers, so that four ants share
+// a SIMD: with the 142 it would take, three do, and 4096 ants at 1001 nodes
+// take 1716 us instead of 1285 (513 nodes: 873, 631).  One round of ants is
+// not changed by it (1500 ants at 1001 nodes: 932, 945).
 template <bool HAS_D, int RNG, bool WIDE, int NODES>
-__global__ __launch_bounds__(64) void k_construct_knn(DevBatch bt)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(HAS_D && !WIDE && NODES > 8 ? 4 : 1)))
+void k_construct_knn(DevBatch bt)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     ANT_PROLOGUE
