@@ -1317,19 +1317,39 @@ __device__ __forceinline__ void ls_relocate(const DevProblem &p, LsLds &L, const
 
 // ----------------------------------------------------- packed relocate ----
 
-// Instances whose distances are integers up to kPackedMax (and demands up to
-// kPackedDemand; DevProblem::packed) take this relocate.  Same rounds, rows
-// and order as ls_relocate; the difference is the arithmetic: eight
-// consecutive edges per lane (512 per trip), gains as packed 16-bit
-// integers, exact because no intermediate leaves 16 bits, and the capacity
-// test of each edge's route beside them, so only candidates that fit leave
-// the trip (70% of the scans at 1001 nodes meet an improving insertion, 15
+// The relocate of searches on 16-bit rows (a launch shape, row16, that a
+// context has from its autotuning or by request) for instances whose
+// distances are integers up to kPackedMax and whose demands are at most
+// kPackedDemand (DevProblem::packed).  Same rounds, rows and order as
+// ls_relocate; the difference is the arithmetic: eight consecutive edges per
+// lane (512 per trip), gains as packed 16-bit integers, exact because no
+// intermediate leaves 16 bits, and the capacity test of each edge's route
+// beside them, so only candidates that fit leave the trip (70% of the scans at 1001 nodes meet an improving insertion, 15
 // to 27% one that fits).  A trip costs about 110 instructions for 512
 // edges, one of relocate_scan about 100 for 128.
 // Measured with 256 ants at 1001 nodes: relocate 1.18 -> 0.93 ms of a search
-// of 2.24 -> 2.00 ms; 480 ants at 481 nodes 0.38 -> 0.36 ms; 256 instances of
-// 64 ants 10.7 -> 10.2 ms.  What bounds it there is the round around the
-// scans: two barriers, the row ring's upkeep and the move itself.
+// of 2.24 -> 2.00 ms.  What bounds it there is the round around the scans:
+// two barriers, the row ring's upkeep and the move itself.
+//
+// Tours of at least packed_positions() positions take it.  A trip covers 512
+// edges whether the tour has them or not, and a move's shift is done by the
+// whole block, whose barriers cost the more the more waves meet there; with a
+// limit, candidates that fit are taken one by one.  Packed / general, in us,
+// 256 ants with about 12 customers per route (1.085 n positions):
+//   nodes             351          651          851         1001
+//   relocate alone
+//    4 waves       649/655    1280/1371    1585/2255    2281/2932
+//      limit       809/763    1450/1613    1813/2290    2680/3035
+//    8 waves       671/637    1311/1279    1596/2042    1929/2575
+//      limit       848/749    1496/1511    1863/2101    2337/2714
+//    12 waves      756/646    1455/1343    1765/2030    2057/2516
+//      limit       949/747    1658/1509    2064/2100    2575/2660
+//    16 waves      815/699    1584/1437    1905/2142    2239/2605
+//      limit      1034/789    1819/1605    2284/2212    2843/2814
+//   full search
+//    4 waves       673/700    1246/1363    1722/2238    2374/2934
+//    12 waves      605/569    1031/1016    1357/1579    1747/2030
+//      limit       672/616    1087/1126    1465/1626    1910/2117
 //
 // A swap has four row reads per candidate instead of one, which no packing
 // saves: the same scheme measured slower there (1001 nodes 0.86 -> 1.00 ms),
@@ -1425,6 +1445,14 @@ __device__ __forceinline__ unsigned bits_below(int lim, int q0)
 }
 
 __device__ __forceinline__ int room16(int q) { return q > kRoomMax ? kRoomMax : q < -kRoomMax ? -kRoomMax : q; }
+
+// Fewest tour positions that take the packed relocate (figures above): the
+// lines lie where neither the search nor relocate alone gets slower.
+template <int W> __device__ __forceinline__ int packed_positions(bool has_d)
+{
+    return W == 4 ? (has_d ? 480 : 400) : W == 8 ? (has_d ? 704 : 768) : W == 12 ? (has_d ? 900 : 832)
+                                                                                 : (has_d ? 1024 : 880);
+}
 
 struct PackedTour {
     unsigned short *t2, *w, *rx, *room;
@@ -1829,7 +1857,7 @@ __device__ void local_search_ant(const DevProblem &p, const DevState &s, int a, 
     if (flags & kLsRelocate) {
         bool packed = false;
         if constexpr (sizeof(RT) == 2) {
-            if (p.packed) {
+            if (p.packed && S >= packed_positions<W>(p.has_d)) {
                 packed = true;
                 // a swap keeps the depots' positions and the route indices
                 if (!(flags & kLsSwap)) ls_routes<W>(p, L, S, tid, false);
