@@ -1711,6 +1711,14 @@ __global__ __launch_bounds__(W * 64, W == 4 ? 3 : 4) void k_iteration_fused(DevB
                                                            float tick_to_s)
 {
     constexpr int NT = W * 64;
+    // The packed relocate only with 8 waves.  With 4 it pushes the kernel's
+    // registers into scratch (480 instead of 300 bytes a lane), which every
+    // phase pays for: five iterations of 256 ants at 1001 nodes, 2-opt alone
+    // 28.7 ms with it and 23.7 without, 2-opt and swap 51.0 and 45.1, the
+    // full search 75.1 and 79.4; at 301 nodes 6.0 and 5.1, 9.9 and 9.0, 15.4
+    // and 14.4 (8 waves: 24.0 and 23.6, 56.6 and 53.6, 91.8 and 102.6 at
+    // 1001 nodes).
+    constexpr bool PACKED = W == 8 && sizeof(RT) == 2;
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int sh_item, sh_last;
     const int tid = threadIdx.x, lane = tid & 63, wv = wave_id();
@@ -1745,7 +1753,7 @@ __global__ __launch_bounds__(W * 64, W == 4 ? 3 : 4) void k_iteration_fused(DevB
         }
 #pragma unroll 1
         for (int q = 0; q < W; ++q) {
-            local_search_ant<W, RT>(p, s, a0 + q, flags, ring, prefetch, smem);
+            local_search_ant<W, RT, false, PACKED>(p, s, a0 + q, flags, ring, prefetch, smem);
             __syncthreads();
         }
         __threadfence();   // this item's tours, lengths and counters, device-wide

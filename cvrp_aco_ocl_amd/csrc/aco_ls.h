@@ -1790,7 +1790,8 @@ __device__ __forceinline__ void scan_priority(int w, int W)
     else __builtin_amdgcn_s_setprio(0);
 }
 
-template <int W, typename RT, bool R2 = false>
+// PACKED: with the packed relocate (searches on 16-bit rows).
+template <int W, typename RT, bool R2 = false, bool PACKED = sizeof(RT) == 2>
 __device__ void local_search_ant(const DevProblem &p, const DevState &s, int a, int flags, int ring,
                                  int prefetch, unsigned char *smem)
 {
@@ -1856,7 +1857,7 @@ __device__ void local_search_ant(const DevProblem &p, const DevState &s, int a, 
     }
     if (flags & kLsRelocate) {
         bool packed = false;
-        if constexpr (sizeof(RT) == 2) {
+        if constexpr (PACKED) {
             if (p.packed && S >= packed_positions<W>(p.has_d)) {
                 packed = true;
                 // a swap keeps the depots' positions and the route indices
