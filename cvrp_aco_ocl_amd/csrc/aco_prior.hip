@@ -287,13 +287,19 @@ __global__ __launch_bounds__(kThreads) void k_forward(const unsigned short *xb, 
     }
 }
 
-// Fused forward + backward over one tile of 16 edges per wave (positions
-// [0, Eb) of idx, or of the data in order without one); the block's waves add
-// their gradients in LDS in wave order and write one partial row.  A wave's
-// chain of products, conversions and transposes is the launch's length, so a
-// batch is spread over as many waves as it has tiles: 16384 edges on 64
-// blocks of four tiles per wave took 36 us, on 256 blocks of one 19.5 us, with
-// as many partial rows.
+// Fused forward + backward (positions [0, Eb) of idx, or of the data in order
+// without one): wave w of block b takes the tiles of 16 edges 4b + w, + 4
+// blocks, ...; the block's waves add their gradients in LDS in wave order and
+// write one partial row.  A wave's chain of products, conversions and
+// transposes is the launch's length, and a CU holds one block (the
+// accumulators), so a batch gets a block per four tiles up to kTrainBlocks,
+// one per CU, and more tiles per wave beyond: 16384 edges on 64 blocks of four
+// tiles per wave take 36 us, on 256 blocks of one 19.5 us; 65536 edges on 1024
+// blocks of one tile 70 us, on 256 blocks of four 37 us (30000: 37, 25).  A constant, so the
+// order of the sums does not depend on the device.
+constexpr int kTrainBlocks = 256;
+static int train_blocks(int Eb) { return std::min((Eb + 16 * kWaves - 1) / (16 * kWaves), kTrainBlocks); }
+
 __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, const float *label,
                                                     const int *idx, int Eb,
                                                     const unsigned short *wb, const float *pf,
@@ -302,7 +308,7 @@ __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, co
     __shared__ NetLds S;
     load_net(S, wb, pf);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
-    const int tile = blockIdx.x * kWaves + w, tiles = (Eb + 15) / 16;
+    const int tiles = (Eb + 15) / 16;
     unsigned short(*T)[16][16] = S.tr[w];
     const v4f zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
     v4f dW2[4][4], dW1[4], db1[4], db2[4], dw3[4];
@@ -313,7 +319,7 @@ __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, co
         for (int b = 0; b < 4; ++b) dW2[a][b] = zero4;
     }
     float db3 = 0.0f, loss = 0.0f;
-    if (tile < tiles) {
+    for (int tile = blockIdx.x * kWaves + w; tile < tiles; tile += gridDim.x * kWaves) {
         const int pos = tile * 16 + r;
         const bool valid = pos < Eb;
         const int e = !valid ? 0 : idx ? idx[pos] : pos;
@@ -936,7 +942,7 @@ static int launch_batch(aco_prior *net, const unsigned short *xb, const float *l
                         int Eb, float pos_weight, float *partials, float *grad_out, float *loss_out,
                         bool update, const AdamArgs &aa)
 {
-    const int blocks = ((Eb + 15) / 16 + kWaves - 1) / kWaves;
+    const int blocks = train_blocks(Eb);
     hipLaunchKernelGGL(k_train, dim3(blocks), dim3(kThreads), 0, net->stream, xb, label, idx, Eb,
                        net->wb, net->pf, pos_weight, 1.0f / (float)Eb, partials);
     PCHK(hipGetLastError());
@@ -950,8 +956,7 @@ static int launch_batch(aco_prior *net, const unsigned short *xb, const float *l
 
 static size_t partial_bytes(int Eb)
 {
-    const int blocks = ((Eb + 15) / 16 + kWaves - 1) / kWaves;
-    return (size_t)blocks * NPL * sizeof(float);
+    return (size_t)train_blocks(Eb) * NPL * sizeof(float);
 }
 
 extern "C" {
