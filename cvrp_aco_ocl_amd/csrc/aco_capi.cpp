@@ -53,44 +53,59 @@ struct InstanceData {
     void *arena = nullptr;
 };
 
-// Device-to-host copies through two pinned buffers in turn.  The pieces of
-// one readback are packed into a buffer; when it is full it is copied out
-// while the other one is being filled.  A pitched matrix travels with its
-// padding, as one run of bytes, and loses it on the way out: the runtime's
-// 2-D copies go row by row (7 us each: 14 ms for two matrices of 1001 rows)
-// into pageable memory, and into any memory where the rows are not whole
-// words; this takes 0.4 ms.  Several small arrays need one wait.
-// 512 KB a buffer: the runtime keeps freed pinned blocks of this size, so
-// neither this context nor the next one pays for pinning (with 1 or 2 MB
-// aco_create of a 242-node instance after another context's end took 1.56
-// instead of 0.88 ms), and a chunk's transfer still covers its launch.
-// Reading 243 tours of 242 nodes: 2.1 -> 0.08 ms.
-// One context, one readback at a time (the mutex); the buffers are made by
-// the first readback and live as long as the context.
+// Copies between host arrays and the device through two pinned buffers in
+// turn.  The pieces of one readback are packed into a buffer; when it is full
+// it is copied out while the other one is being filled.  A pitched matrix
+// travels with its padding, as one run of bytes, and loses it on the way out:
+// the runtime's 2-D copies go row by row (7 us each: 14 ms for two matrices of
+// 1001 rows) into pageable memory, and into any memory where the rows are not
+// whole words; this takes 0.4 ms.  Several small arrays need one wait.
+// A buffer holds what the context's tours or its two trail matrices need,
+// from 64 KB to 512 KB, and the second one is made when the first is full:
+// pinning costs 12 us while the runtime has a freed block for it and 100 to
+// 300 us when not, which it is the likelier to have the less is asked for.
+// Creating a context of 20 nodes and reading its best tour: 410 to 450 us with
+// pageable copies, 445 to 1060 us with two buffers of 512 KB, 390 to 430 us
+// so.  1 or 2 MB buffers cost the next context's creation 0.7 ms.  At 512 KB a
+// chunk's transfer covers its launch.  Reading 243 tours of 242 nodes: 2.1 ->
+// 0.05 ms.
+// One context, one transfer at a time (the mutex); the buffers are made by
+// the first one and live as long as the context.
 struct Readback {
-    static constexpr size_t kBytes = size_t(512) << 10;
+    static constexpr size_t kMost = size_t(512) << 10, kLeast = size_t(64) << 10;
+    static constexpr int kPieces = 16;
     struct Piece {
         unsigned char *dst;
         size_t dpitch, pitch, width, rows, off;
     };
     std::mutex mutex;
+    size_t size = kLeast;   // of a buffer
     unsigned char *buf[2] = {nullptr, nullptr};
     hipEvent_t done[2] = {nullptr, nullptr};
-    std::vector<Piece> pieces[2];
+    Piece pieces[2][kPieces];
+    int count[2] = {0, 0};
     size_t used = 0;
     int cur = 0;
 
+    // before the first transfer: the most bytes that one is likely to move
+    void fit(size_t bytes)
+    {
+        while (size < bytes && size < kMost) size *= 2;
+    }
+    // start of a transfer
     hipError_t init()
     {
-        for (int i = 0; i < 2; ++i) {
-            hipError_t e = hipSuccess;
-            if (!buf[i]) e = hipHostMalloc((void **)&buf[i], kBytes, hipHostMallocDefault);
-            if (e == hipSuccess && !done[i]) e = hipEventCreateWithFlags(&done[i], hipEventDisableTiming);
-            if (e != hipSuccess) return e;
-            pieces[i].clear();
-        }
+        count[0] = count[1] = 0;
         used = 0;
-        return hipSuccess;
+        cur = 0;
+        return make(0);
+    }
+    hipError_t make(int i)
+    {
+        hipError_t e = hipSuccess;
+        if (!buf[i]) e = hipHostMalloc((void **)&buf[i], size, hipHostMallocDefault);
+        if (e == hipSuccess && !done[i]) e = hipEventCreateWithFlags(&done[i], hipEventDisableTiming);
+        return e;
     }
     ~Readback()
     {
@@ -102,28 +117,30 @@ struct Readback {
     // waits for buffer i's transfers and copies its pieces out
     hipError_t drain(int i)
     {
-        if (pieces[i].empty()) return hipSuccess;
+        if (!count[i]) return hipSuccess;
         const hipError_t e = hipEventSynchronize(done[i]);
         if (e != hipSuccess) return e;
-        for (const Piece &p : pieces[i]) {
+        for (int q = 0; q < count[i]; ++q) {
+            const Piece &p = pieces[i][q];
             if (p.dpitch == p.width && p.pitch == p.width) memcpy(p.dst, buf[i] + p.off, p.width * p.rows);
             else
                 for (size_t r = 0; r < p.rows; ++r)
                     memcpy(p.dst + r * p.dpitch, buf[i] + p.off + r * p.pitch, p.width);
         }
-        pieces[i].clear();
+        count[i] = 0;
         return hipSuccess;
     }
     // the current buffer is full: copy the other one out, then fill it
     hipError_t turn(hipStream_t st)
     {
         hipError_t e = hipEventRecord(done[cur], st);
+        if (e == hipSuccess) e = make(cur ^ 1);
         if (e != hipSuccess) return e;
         cur ^= 1;
         used = 0;
         return drain(cur);
     }
-    // `rows` rows of `width` bytes, device pitch spitch (at most kBytes, and
+    // `rows` rows of `width` bytes, device pitch spitch (at most kLeast, and
     // the last row's padding is allocated too), to host rows of pitch dpitch
     hipError_t get2d(void *dst, size_t dpitch, const void *src, size_t spitch, size_t width, size_t rows, hipStream_t st)
     {
@@ -132,11 +149,11 @@ struct Readback {
         if (!width) return hipSuccess;
         while (rows) {
             hipError_t e = hipSuccess;
-            if (used + spitch > kBytes && (e = turn(st)) != hipSuccess) return e;
-            const size_t nr = std::min(rows, (kBytes - used) / spitch);
+            if ((used + spitch > size || count[cur] == kPieces) && (e = turn(st)) != hipSuccess) return e;
+            const size_t nr = std::min(rows, (size - used) / spitch);
             e = hipMemcpyAsync(buf[cur] + used, s, spitch * nr, hipMemcpyDeviceToHost, st);
             if (e != hipSuccess) return e;
-            pieces[cur].push_back({d, dpitch, spitch, width, nr, used});
+            pieces[cur][count[cur]++] = {d, dpitch, spitch, width, nr, used};
             used = (used + spitch * nr + 63) & ~size_t(63);
             d += nr * dpitch;
             s += nr * spitch;
@@ -147,11 +164,38 @@ struct Readback {
     // contiguous bytes (taken as rows of at most 64 KB)
     hipError_t get(void *dst, const void *src, size_t bytes, hipStream_t st)
     {
-        const size_t w = size_t(64) << 10, rows = bytes / w, rest = bytes - rows * w;
+        const size_t w = kLeast, rows = bytes / w, rest = bytes - rows * w;
         hipError_t e = get2d(dst, w, src, w, w, rows, st);
         if (e != hipSuccess) return e;
         return get2d(static_cast<unsigned char *>(dst) + rows * w, rest, static_cast<const unsigned char *>(src) + rows * w,
                      rest, rest, 1, st);
+    }
+    // `rows` dense host rows of `width` bytes (at most kLeast) into a device
+    // array of row pitch dpitch; the buffers are free once the stream is idle
+    hipError_t put2d(void *dst, size_t dpitch, const void *src, size_t width, size_t rows, hipStream_t st)
+    {
+        unsigned char *d = static_cast<unsigned char *>(dst);
+        const unsigned char *s = static_cast<const unsigned char *>(src);
+        while (rows) {
+            hipError_t e = hipSuccess;
+            if (used + width > size) {
+                e = hipEventRecord(done[cur], st);
+                if (e == hipSuccess) e = make(cur ^ 1);
+                if (e == hipSuccess) e = hipEventSynchronize(done[cur ^ 1]);   // its transfers, if it had any
+                if (e != hipSuccess) return e;
+                cur ^= 1;
+                used = 0;
+            }
+            const size_t nr = std::min(rows, (size - used) / width);
+            memcpy(buf[cur] + used, s, nr * width);
+            e = hipMemcpy2DAsync(d, dpitch, buf[cur] + used, width, width, nr, hipMemcpyHostToDevice, st);
+            if (e != hipSuccess) return e;
+            used = (used + nr * width + 63) & ~size_t(63);
+            d += nr * dpitch;
+            s += nr * width;
+            rows -= nr;
+        }
+        return hipSuccess;
     }
     hipError_t finish(hipStream_t st)
     {
@@ -815,6 +859,8 @@ int aco_create_batch(const aco_problem *pbs, int32_t count, const aco_params *pr
     CHK(hipMemcpyAsync(dinst, ant_inst.data(), 4 * ant_inst.size(), hipMemcpyHostToDevice, c->stream));
     CHK(hipMemcpyAsync(dbase, ant_base.data(), 4 * ant_base.size(), hipMemcpyHostToDevice, c->stream));
     CHK(hipStreamSynchronize(c->stream));
+    for (const InstanceData &I : c->inst)
+        c->rb.fit(std::max((size_t)(m + 1) * I.T * 4, 2 * (size_t)I.n * I.P * 4));
     bt.cons_lds_budget = c->lds_limit - c->lds_static_cons;
     bt.cus = prop.multiProcessorCount;
     bt.probs = dprobs;
@@ -962,7 +1008,7 @@ int aco_get_best_at(aco_ctx *c, int32_t b, int32_t *tour, int32_t cap, int32_t *
     if (rc) return rc;
     const std::lock_guard<std::mutex> lock(c->rb.mutex);
     HIP_TRY(c->rb.init());
-    static_assert((2 + 2 * kMaxNodes) * 4 <= Readback::kBytes, "a tour fits one buffer");
+    static_assert((2 + 2 * kMaxNodes) * 4 <= Readback::kLeast, "a tour fits the smallest buffer");
     int32_t *best = reinterpret_cast<int32_t *>(c->rb.buf[0]);
     HIP_TRY(launch_best_pack(c->bt, b, best, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
@@ -1169,12 +1215,16 @@ int aco_set_pheromone_at(aco_ctx *c, int32_t b, const float *tau, const float *t
     if (rc) return rc;
     if (!tau || !ti) return set_error(ACO_ERR_ARG, "null argument");
     const InstanceData &I = c->inst[b];
-    PinnedStager up;
-    HIP_TRY(up.init(c->stream, Readback::kBytes));
-    HIP_TRY(up.put2d(I.ds.tau, (size_t)I.P * 4, tau, (size_t)I.n * 4, I.n));
-    HIP_TRY(up.put2d(I.ds.tinfo, (size_t)I.P * 4, ti, (size_t)I.n * 4, I.n));
-    if ((rc = run_gather(c))) return rc;
-    HIP_TRY(hipStreamSynchronize(c->stream));
+    const std::lock_guard<std::mutex> lock(c->rb.mutex);
+    HIP_TRY(c->rb.init());
+    const size_t w = (size_t)I.n * 4, pitch = (size_t)I.P * 4;
+    hipError_t e = c->rb.put2d(I.ds.tau, pitch, tau, w, I.n, c->stream);
+    if (e == hipSuccess) e = c->rb.put2d(I.ds.tinfo, pitch, ti, w, I.n, c->stream);
+    if (e == hipSuccess) rc = run_gather(c);
+    const hipError_t es = hipStreamSynchronize(c->stream);   // the buffers are free again
+    HIP_TRY(e);
+    if (rc) return rc;
+    HIP_TRY(es);
     return ACO_OK;
 }
 

@@ -295,8 +295,8 @@ __global__ __launch_bounds__(kThreads) void k_forward(const unsigned short *xb, 
 // accumulators), so a batch gets a block per four tiles up to kTrainBlocks,
 // one per CU, and more tiles per wave beyond: 16384 edges on 64 blocks of four
 // tiles per wave take 36 us, on 256 blocks of one 19.5 us; 65536 edges on 1024
-// blocks of one tile 70 us, on 256 blocks of four 37 us (30000: 37, 25).  A constant, so the
-// order of the sums does not depend on the device.
+// blocks of one tile 70 us, on 256 blocks of four 37 us (30000: 37, 25).  A
+// constant, so the order of the sums does not depend on the device.
 constexpr int kTrainBlocks = 256;
 static int train_blocks(int Eb) { return std::min((Eb + 16 * kWaves - 1) / (16 * kWaves), kTrainBlocks); }
 

@@ -183,7 +183,9 @@ int aco_set_ants(aco_ctx *ctx, const int32_t *tours, int32_t stride, const int32
                  const float *lengths);
 /* best-so-far records (g_aco.cpp:95-117); *count = records written */
 int aco_get_bsf(aco_ctx *ctx, aco_bsf_record *records, int32_t capacity, int32_t *count);
-/* n*n pheromone and total_info, row-major */
+/* n*n pheromone and total_info, row-major.  These and the transfers above
+ * (best, ants, setup arrays) go through one or two pinned host buffers of 64
+ * to 512 KB, made by a context's first transfer and kept until its end. */
 int aco_get_pheromone(aco_ctx *ctx, float *tau, float *total_info);
 int aco_set_pheromone(aco_ctx *ctx, const float *tau, const float *total_info);
 /* m*64 Park-Miller lane states of instance 0 (the per-ant draw streams,
