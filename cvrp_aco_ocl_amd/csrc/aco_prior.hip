@@ -861,7 +861,16 @@ static AdamArgs adam_args(int step, float lr, float b1, float b2, float eps)
     return a;
 }
 
-// bf16 features (and labels) of `count` edges into device arrays: rows pass
+static int pack_features(aco_prior *net, const float *feat, const float *label, long long count, unsigned short *xb,
+                         float *lab)
+{
+    hipLaunchKernelGGL(k_pack_features, dim3((unsigned)((4 * count + 255) / 256)), dim3(256), 0, net->stream, feat,
+                       label, count, xb, lab);
+    PCHK(hipGetLastError());
+    return ACO_OK;
+}
+
+// bf16 features and labels of `count` edges into device arrays: rows pass
 // through the pinned input buffers, from which the packing kernel reads them
 // while the next buffer is filled.
 static int stage_features(aco_prior *net, const float *feat, const float *label, long long count, unsigned short *xb,
@@ -875,11 +884,27 @@ static int stage_features(aco_prior *net, const float *feat, const float *label,
         PCHK(sp.take(b));
         float *f = reinterpret_cast<float *>(b), *l = f + c * NF;
         memcpy(f, feat + e * NF, (size_t)c * NF * sizeof(float));
-        if (label) memcpy(l, label + e, (size_t)c * sizeof(float));
-        hipLaunchKernelGGL(k_pack_features, dim3((unsigned)((4 * c + 255) / 256)), dim3(256), 0, net->stream, f,
-                           label ? l : nullptr, c, xb + e * NFP, label ? lab + e : nullptr);
-        PCHK(hipGetLastError());
+        memcpy(l, label + e, (size_t)c * sizeof(float));
+        const int rc = pack_features(net, f, l, c, xb + e * NFP, lab + e);
+        if (rc != ACO_OK) return rc;
         PCHK(sp.used(net->stream));
+    }
+    return ACO_OK;
+}
+
+// bf16 features alone, from pageable memory through f32, which holds
+// kForwardRows rows: one plain copy for most calls.  Without labels there is
+// one array to move, and the runtime's copy of it is faster than a memcpy into
+// pinned buffers from some 8000 edges on (forward of 16384 edges 75 against
+// 87 us, 65536: 229, 305), and for fewer a new network pins nothing.
+constexpr long long kForwardRows = 131072;   // 6 MB
+static int stage_features_only(aco_prior *net, const float *feat, long long count, unsigned short *xb, float *f32)
+{
+    for (long long e = 0; e < count; e += kForwardRows) {
+        const long long c = std::min(kForwardRows, count - e);
+        PCHK(hipMemcpyAsync(f32, feat + e * NF, (size_t)c * NF * sizeof(float), hipMemcpyHostToDevice, net->stream));
+        const int rc = pack_features(net, f32, nullptr, c, xb + e * NFP, nullptr);
+        if (rc != ACO_OK) return rc;
     }
     return ACO_OK;
 }
@@ -1111,10 +1136,12 @@ int aco_prior_forward(aco_prior *net, const float *feat, int64_t count, float *l
     if (!net || !feat || !logits) return set_error(ACO_ERR_ARG, "null argument");
     if (count < 1 || count > (1ll << 31)) return set_error(ACO_ERR_ARG, "count out of range");
     SpaceUse use(net->space, net->stream);
-    PCHK(net->space.init(SpaceUse::round((size_t)count * NFP * 2) + SpaceUse::round((size_t)count * 4)));
+    const size_t rows = (size_t)std::min<long long>(count, kForwardRows);
+    PCHK(net->space.init(SpaceUse::round((size_t)count * NFP * 2) + SpaceUse::round((size_t)count * 4) +
+                         SpaceUse::round(rows * NF * 4)));
     unsigned short *xb = use.take<unsigned short>((size_t)count * NFP);
     float *out = use.take<float>((size_t)count);
-    int rc = stage_features(net, feat, nullptr, count, xb, nullptr);
+    int rc = stage_features_only(net, feat, count, xb, use.take<float>(rows * NF));
     if (rc != ACO_OK) return rc;
     rc = launch_forward(net, xb, count, out);
     if (rc != ACO_OK) return rc;
