@@ -702,18 +702,27 @@ using namespace cvrp::prior;
 
 // Working memory of a network's calls, kept between them (one call at a
 // time): one device allocation, given back after a call that needed more
-// than kKeep, and four pinned buffers of 512 KB.  Pageable copies of this
-// size cost 25 to 60 us each whatever they hold, allocations of 2 MB and more
-// 25 us; a gradient made six of the first and two of the second.  Gradient
-// over 16384 edges 202 -> 75 us, multiplier of 501 nodes 200 -> 117 us, eight
-// training steps of 16384 edges 945 -> 502 us; what is left is the copy into
-// the buffers, the launches and the kernels (25 us of the gradient).
+// than kKeep, and one pinned one: one or two parts for inputs, then results.
+// Pageable copies of this size cost 25 to 60 us each whatever they hold,
+// allocations of 2 MB and more 25 us; a gradient made six of the first and two
+// of the second.  Gradient over 16384 edges 202 -> 75 us, multiplier of 501
+// nodes 200 -> 128 us, eight training steps of 16384 edges 932 -> 500 us; what
+// is left is the copy into the buffers, the launches and the kernels (25 us
+// of the gradient).
+// Parts are as large as the largest call so far needs, up to kPart, and a call
+// that fits one makes one: a network that is made, used once and dropped pays
+// for pinning, 25 us a block with its end while the runtime has a freed one
+// and 100 to 300 us and more when not.  A part is a chunk of the pipeline and
+// each costs about 15 us: with parts of 256, 128 and 64 KB the gradient of
+// 65536 edges takes 229, 328 and 499 us, with 512 KB 194 us.
 struct PriorSpace {
-    static constexpr size_t kPin = size_t(512) << 10, kKeep = size_t(64) << 20;
+    static constexpr size_t kPart = size_t(512) << 10, kLeast = size_t(32) << 10, kKeep = size_t(64) << 20;
     std::mutex mutex;
     unsigned char *dev = nullptr;
     size_t dev_bytes = 0;
-    unsigned char *pin[4] = {nullptr, nullptr, nullptr, nullptr};   // 0, 1: inputs and matrices; 2, 3: small results
+    unsigned char *pin = nullptr;
+    size_t part = 0, results = 0;   // bytes of a part, and behind the parts
+    int parts = 0;
     hipEvent_t done[2] = {nullptr, nullptr};
     bool busy[2] = {false, false};
     int cur = 0;
@@ -727,9 +736,30 @@ struct PriorSpace {
         if (e == hipSuccess) dev_bytes = bytes;
         return e;
     }
-    hipError_t pinned(int i)   // buffer i exists
+    // for a call that moves `bytes` through the parts, rows of `row` bytes
+    // whole, and takes `res` bytes of results; nothing is in use yet
+    hipError_t pinned(size_t bytes, size_t row, size_t res)
     {
-        return pin[i] ? hipSuccess : hipHostMalloc((void **)&pin[i], kPin, hipHostMallocDefault);
+        size_t want = std::max(part, kLeast);
+        while ((want < bytes && want < kPart) || want < row) want *= 2;
+        const int count = std::max(parts, bytes > want ? 2 : 1);
+        if (want == part && count == parts && res <= results) return hipSuccess;
+        res = std::max(res, results);
+        unpin();
+        const hipError_t e = hipHostMalloc((void **)&pin, want * count + res, hipHostMallocDefault);
+        if (e != hipSuccess) return e;
+        part = want;
+        parts = count;
+        results = res;
+        return hipSuccess;
+    }
+    unsigned char *result() const { return pin + part * parts; }
+    void unpin()
+    {
+        if (pin) (void)hipHostFree(pin);
+        pin = nullptr;
+        part = results = 0;
+        parts = 0;
     }
     void release()
     {
@@ -740,27 +770,26 @@ struct PriorSpace {
     ~PriorSpace()
     {
         release();
-        for (unsigned char *p : pin)
-            if (p) (void)hipHostFree(p);
+        unpin();
         for (hipEvent_t e : done)
             if (e) (void)hipEventDestroy(e);
         if (side) (void)hipStreamDestroy(side);
     }
-    // input buffer to fill next, once its last reader on the device is done
+    // input part to fill next, once its last reader on the device is done
     hipError_t take(unsigned char *&p)
     {
-        hipError_t e = pinned(cur);
-        if (e == hipSuccess && !done[cur]) e = hipEventCreateWithFlags(&done[cur], hipEventDisableTiming);
+        hipError_t e = hipSuccess;
+        if (!done[cur]) e = hipEventCreateWithFlags(&done[cur], hipEventDisableTiming);
         if (e == hipSuccess && busy[cur]) e = hipEventSynchronize(done[cur]);
         busy[cur] = false;
-        p = pin[cur];
+        p = pin + cur * part;
         return e;
     }
     hipError_t used(hipStream_t st)
     {
         const hipError_t e = hipEventRecord(done[cur], st);
         busy[cur] = true;
-        cur ^= 1;
+        cur = parts - 1 - cur;
         return e;
     }
 };
@@ -877,7 +906,7 @@ static int stage_features(aco_prior *net, const float *feat, const float *label,
                           float *lab)
 {
     PriorSpace &sp = net->space;
-    const long long per = (long long)(PriorSpace::kPin / ((NF + 1) * sizeof(float)));
+    const long long per = (long long)(sp.part / ((NF + 1) * sizeof(float)));
     for (long long e = 0; e < count; e += per) {
         const long long c = std::min(per, count - e);
         unsigned char *b = nullptr;
@@ -929,12 +958,12 @@ struct PinnedStream {
     {
         const unsigned char *s = static_cast<const unsigned char *>(src);
         while (bytes) {
-            if (fill == PriorSpace::kPin) {
+            if (fill == net->space.part) {
                 const int rc = flush();
                 if (rc != ACO_OK) return rc;
             }
             if (!buf) PCHK(net->space.take(buf));
-            const size_t c = std::min(bytes, PriorSpace::kPin - fill);
+            const size_t c = std::min(bytes, net->space.part - fill);
             memcpy(buf + fill, s, c);
             fill += c;
             s += c;
@@ -1159,14 +1188,13 @@ int aco_prior_gradient(aco_prior *net, const float *feat, const float *label, in
     SpaceUse use(net->space, net->stream);
     const size_t E = (size_t)count;
     PCHK(net->space.init(SpaceUse::round(E * NFP * 2) + SpaceUse::round(E * 4) + partial_bytes((int)count)));
+    PCHK(net->space.pinned(E * (NF + 1) * sizeof(float), 0, NPL * sizeof(float)));
     unsigned short *xb = use.take<unsigned short>(E * NFP);
     float *lab = use.take<float>(E), *part = use.take<float>(partial_bytes((int)count) / 4);
     int rc = stage_features(net, feat, label, count, xb, lab);
     if (rc != ACO_OK) return rc;
     // the reduction writes the gradient and the loss to host memory
-    PCHK(net->space.pinned(2));
-    float *g = reinterpret_cast<float *>(net->space.pin[2]);
-    static_assert(NPL * sizeof(float) <= PriorSpace::kPin, "gradient and loss fit");
+    float *g = reinterpret_cast<float *>(net->space.result());
     rc = launch_batch(net, xb, lab, nullptr, (int)count, pos_weight, part, g, g + NP, false,
                       adam_args(1, 0, 0.9f, 0.999f, 1e-8f));
     if (rc != ACO_OK) return rc;
@@ -1218,10 +1246,13 @@ int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64
     // make (65536 swaps: 0.1 ms), but the swap targets are one 64-bit remainder
     // each (0.3 ms) of a counter-based stream, so the device draws them, on a
     // stream of its own, two buffers ahead of the swaps.
-    const int chunk = (int)(PriorSpace::kPin / sizeof(int));
     const long long per_epoch = count - 1, draws = per_epoch * tp->epochs;
+    const int chunk = (int)std::min<long long>(std::max(per_epoch, 1ll), PriorSpace::kPart / sizeof(int));
+    const size_t span = SpaceUse::round((size_t)chunk * sizeof(int));
+    PCHK(sp.pinned(E * (NF + 1) * sizeof(float), 0, 2 * span));
+    auto targets = [&](int i) { return reinterpret_cast<int *>(sp.result() + i * span); };
     long long drawn = 0;   // draws requested so far
-    int at = 0;            // pinned buffer the next request fills (2 or 3)
+    int at = 0;            // buffer the next request fills
     hipEvent_t ready[2] = {nullptr, nullptr};
     struct Events {
         hipEvent_t *e;
@@ -1232,15 +1263,13 @@ int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64
         }
     } events{ready};
     for (hipEvent_t &e : ready) PCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    PCHK(sp.pinned(2));
-    PCHK(sp.pinned(3));
     if (!sp.side) PCHK(hipStreamCreateWithFlags(&sp.side, hipStreamNonBlocking));
     auto request = [&]() -> int {   // never across an epoch's end
         if (drawn == draws) return ACO_OK;
         const long long in = drawn % per_epoch;
         const int c = (int)std::min<long long>(chunk, per_epoch - in);
         hipLaunchKernelGGL(k_swap_targets, dim3((c + 255) / 256), dim3(256), 0, sp.side, tp->shuffle_seed,
-                           (unsigned long long)drawn, (int)(per_epoch - in), c, reinterpret_cast<int *>(sp.pin[2 + at]));
+                           (unsigned long long)drawn, (int)(per_epoch - in), c, targets(at));
         PCHK(hipGetLastError());
         PCHK(hipEventRecord(ready[at], sp.side));
         drawn += c;
@@ -1259,7 +1288,7 @@ int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64
         for (long long i = 0; i < count; ++i) perm[(size_t)i] = (int)i;
         for (long long i = count - 1; i > 0;) {
             PCHK(hipEventSynchronize(ready[from]));
-            const int *j = reinterpret_cast<const int *>(sp.pin[2 + from]);
+            const int *j = targets(from);
             const long long c = std::min<long long>(chunk, i);
             for (long long t = 0; t < c; ++t) std::swap(perm[(size_t)(i - t)], perm[(size_t)j[t]]);
             i -= c;
@@ -1319,6 +1348,7 @@ int aco_prior_build(aco_prior *net, int32_t n, const float *x, const float *y,
     float *rad = use.take<float>(N), *ang = use.take<float>(N), *kd = use.take<float>(N), *Rm = use.take<float>(64);
     unsigned short *xb = use.take<unsigned short>(E * NFP);
     float *lg = use.take<float>(E);
+    PCHK(sp.pinned(std::max(block, N * N) * 4, N * 4, 0));
     PinnedStream up = {net, reinterpret_cast<unsigned char *>(xd)};
     const struct { const void *p; } heads[4] = {{x}, {y}, {demand}, {dist}};   // dist: its first row
     for (const auto &h : heads)
@@ -1343,14 +1373,13 @@ int aco_prior_build(aco_prior *net, int32_t n, const float *x, const float *y,
     rc = launch_forward(net, xb, (long long)E, lg);
     if (rc != ACO_OK) return rc;
     const float fl = floor_pow(floor, exponent);
-    const int per = (int)std::min<size_t>(N, PriorSpace::kPin / (N * 4));
-    static_assert(65536 * 4 <= PriorSpace::kPin, "a row fits a buffer");
+    const int per = (int)std::min<size_t>(N, sp.part / (N * 4));
     struct { int row, rows, buf; } out = {0, 0, 0};   // rows on their way
     auto collect = [&]() -> int {
         if (!out.rows) return ACO_OK;
         PCHK(hipEventSynchronize(sp.done[out.buf]));
         sp.busy[out.buf] = false;
-        memcpy(prior + (size_t)out.row * N, sp.pin[out.buf], (size_t)out.rows * N * 4);
+        memcpy(prior + (size_t)out.row * N, sp.pin + out.buf * sp.part, (size_t)out.rows * N * 4);
         return ACO_OK;
     };
     for (int row = 0; row < n; row += per) {
