@@ -1222,6 +1222,8 @@ int aco_prior_adam_step(aco_prior *net, const float *grad, float lr, float beta1
     return ACO_OK;
 }
 
+constexpr long long kDeviceDraws = 4096;
+
 int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64_t count,
                     const aco_prior_train_params *tp, float *epoch_loss)
 {
@@ -1244,15 +1246,20 @@ int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64
     float *part = use.take<float>(partial_bytes(tp->batch) / 4), *losses = use.take<float>((size_t)total);
     // The order of an epoch is a Fisher-Yates shuffle, which only the host can
     // make (65536 swaps: 0.1 ms), but the swap targets are one 64-bit remainder
-    // each (0.3 ms) of a counter-based stream, so the device draws them, on a
-    // stream of its own, two buffers ahead of the swaps.
+    // each (0.3 ms) of a counter-based stream, so the device draws them, two
+    // buffers ahead of the swaps: the first two before the features go out,
+    // the others on a stream of their own, beside the training.  Epochs of
+    // fewer than kDeviceDraws draws draw on the host, where they cost less
+    // (5 ns each) than a launch and its wait (about 20 us), and a network that
+    // trains once on few edges makes no stream.
     const long long per_epoch = count - 1, draws = per_epoch * tp->epochs;
+    const bool device = per_epoch >= kDeviceDraws;
     const int chunk = (int)std::min<long long>(std::max(per_epoch, 1ll), PriorSpace::kPart / sizeof(int));
     const size_t span = SpaceUse::round((size_t)chunk * sizeof(int));
-    PCHK(sp.pinned(E * (NF + 1) * sizeof(float), 0, 2 * span));
+    PCHK(sp.pinned(E * (NF + 1) * sizeof(float), 0, device ? 2 * span : 0));
     auto targets = [&](int i) { return reinterpret_cast<int *>(sp.result() + i * span); };
     long long drawn = 0;   // draws requested so far
-    int at = 0;            // buffer the next request fills
+    int requests = 0;      // request r fills buffer r % 2
     hipEvent_t ready[2] = {nullptr, nullptr};
     struct Events {
         hipEvent_t *e;
@@ -1262,18 +1269,19 @@ int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64
                 if (e[i]) (void)hipEventDestroy(e[i]);
         }
     } events{ready};
-    for (hipEvent_t &e : ready) PCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    if (!sp.side) PCHK(hipStreamCreateWithFlags(&sp.side, hipStreamNonBlocking));
     auto request = [&]() -> int {   // never across an epoch's end
-        if (drawn == draws) return ACO_OK;
+        if (!device || drawn == draws) return ACO_OK;
         const long long in = drawn % per_epoch;
-        const int c = (int)std::min<long long>(chunk, per_epoch - in);
-        hipLaunchKernelGGL(k_swap_targets, dim3((c + 255) / 256), dim3(256), 0, sp.side, tp->shuffle_seed,
+        const int c = (int)std::min<long long>(chunk, per_epoch - in), at = requests & 1;
+        if (!ready[at]) PCHK(hipEventCreateWithFlags(&ready[at], hipEventDisableTiming));
+        if (requests >= 2 && !sp.side) PCHK(hipStreamCreateWithFlags(&sp.side, hipStreamNonBlocking));
+        const hipStream_t on = requests >= 2 ? sp.side : net->stream;
+        hipLaunchKernelGGL(k_swap_targets, dim3((c + 255) / 256), dim3(256), 0, on, tp->shuffle_seed,
                            (unsigned long long)drawn, (int)(per_epoch - in), c, targets(at));
         PCHK(hipGetLastError());
-        PCHK(hipEventRecord(ready[at], sp.side));
+        PCHK(hipEventRecord(ready[at], on));
         drawn += c;
-        at ^= 1;
+        ++requests;
         return ACO_OK;
     };
     int rc = request();
@@ -1284,9 +1292,12 @@ int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64
     std::vector<int> perm((size_t)count);
     long long step = 0;
     int from = 0;   // buffer the next targets come from
+    uint64_t seed = tp->shuffle_seed;
     for (int ep = 0; ep < tp->epochs; ++ep) {
         for (long long i = 0; i < count; ++i) perm[(size_t)i] = (int)i;
-        for (long long i = count - 1; i > 0;) {
+        for (long long i = count - 1; !device && i > 0; --i)
+            std::swap(perm[(size_t)i], perm[(size_t)(sm_next(seed) % (uint64_t)(i + 1))]);
+        for (long long i = count - 1; device && i > 0;) {
             PCHK(hipEventSynchronize(ready[from]));
             const int *j = targets(from);
             const long long c = std::min<long long>(chunk, i);
