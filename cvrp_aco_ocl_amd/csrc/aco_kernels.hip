@@ -1030,7 +1030,11 @@ static hipError_t max_static_lds(const void *const *fns, int count, size_t &byte
 
 hipError_t construct_static_lds(size_t &bytes)
 {
+#define IR(D, NW, C, S) (const void *)k_construct_iroulette_waves<D, NW, C, S>
+#define IRS(D) IR(D, 1, 1, true), IR(D, 1, 2, true), IR(D, 4, 1, true), IR(D, 4, 1, false), IR(D, 4, 2, false), \
+               IR(D, 8, 2, false), IR(D, 8, 4, false), IR(D, 8, 8, false)
     const void *fns[] = {(const void *)k_construct_iroulette<false>, (const void *)k_construct_iroulette<true>,
+                         IRS(false), IRS(true),
 #define KN(D, R, S) (const void *)k_construct_knn<D, R, S, 0>, (const void *)k_construct_knn<D, R, S, 8>, \
                     (const void *)k_construct_knn<D, R, S, 16>
 #define KL(R, A) (const void *)k_construct_knn_lds<R, A, 0>, (const void *)k_construct_knn_lds<R, A, 8>, \
@@ -1041,6 +1045,8 @@ hipError_t construct_static_lds(size_t &bytes)
                          KN(false, kRngParkMiller, false), KN(true, kRngParkMiller, false),
                          KL(kRngPhilox, 1), KL(kRngPhilox, 2), KL(kRngPhilox, 4),
                          KL(kRngParkMiller, 1), KL(kRngParkMiller, 2), KL(kRngParkMiller, 4)};
+#undef IR
+#undef IRS
 #undef KN
 #undef KL
     return max_static_lds(fns, (int)(sizeof(fns) / sizeof(fns[0])), bytes);
@@ -1827,7 +1833,6 @@ hipError_t launch_iteration_fused(const DevBatch &b, int rng, int ls_flags, cons
 }
 
 // State of a fresh colony (aco_init) of every instance in one launch: lane
-// seeds, control words, totals, an empty best-so-far slot, the scan-order
 // seeds, control words, totals, an empty best-so-far slot, the scan-order
 // seed and the context's start time.  As six uploads per instance this took
 // 5.9 ms for 256 instances of 64 ants and about 30 us for one of 51 ants; one
