@@ -511,19 +511,28 @@ static int check_instance(const aco_problem *pb, int width, std::vector<int> &nn
     if (isnan(pb->max_dist) || !(pb->service_time >= 0.0f) || !isfinite(pb->service_time))
         return set_error(ACO_ERR_ARG, "bad max_dist or service_time");
     int16 = true;
-    float longest = 0.0f;
-    for (int i = 0; i < n; ++i)
+    bool diag = true;    // every node is at distance 0 from itself
+    float top[8] = {};   // the largest distance among them
+    for (int i = 0; i < n; ++i) {
+        const float *row = pb->dist + (size_t)i * n;
         for (int j = 0; j < n; ++j) {
-            const float d = pb->dist[(size_t)i * n + j];
+            const float d = row[j];
             if (!isfinite(d) || d < 0.0f) return set_error(ACO_ERR_ARG, "distances must be finite and >= 0");
             if (d != pb->dist[(size_t)j * n + i]) return set_error(ACO_ERR_ARG, "distance matrix is not symmetric");
             int16 = int16 && d <= 65535.0f && d == floorf(d);
-            longest = d > longest ? d : longest;
         }
-    packed = int16 && longest <= (float)kPackedMax;
+        // of its own, on the row just read, eight at a time (in the loop above
+        // it cost 0.5 ns an element)
+        int j = 0;
+        for (; j + 8 <= n; j += 8)
+            for (int q = 0; q < 8; ++q) top[q] = row[j + q] > top[q] ? row[j + q] : top[q];
+        for (; j < n; ++j) top[0] = row[j] > top[0] ? row[j] : top[0];
+        diag = diag && row[i] == 0.0f;
+    }
+    packed = int16 && diag && *std::max_element(top, top + 8) <= (float)kPackedMax;
     for (int i = 0; i < n; ++i) {
         if (pb->demand[i] < 0) return set_error(ACO_ERR_ARG, "negative demand");
-        packed = packed && pb->demand[i] <= kPackedDemand && pb->dist[(size_t)i * n + i] == 0.0f;
+        packed = packed && pb->demand[i] <= kPackedDemand;
     }
     for (int i = 1; i < n; ++i) {
         if (pb->demand[i] > pb->capacity)
