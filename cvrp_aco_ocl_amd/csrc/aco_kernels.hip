@@ -1407,13 +1407,16 @@ __device__ __forceinline__ void statistics_small(const DevProblem &p, const DevS
         float elite_len = flag ? best_len : bsf_len;   // lane g: elite g's
         int elite = m, elite_size = flag ? best_size : bsf_size;
         for (int g = 1; g < ras; ++g) {
-            v = 0x7f800000u;
+            // a taken ant counts as infinite, which is less than the bits of a
+            // negative length or NaN (lengths set from outside)
+            v = ~0u;
             at = 0;
             sz = 0;
 #pragma unroll
             for (int u = 0; u < kStatOwn; ++u) {
-                const bool less = !((taken >> u) & 1u) & (len[u] < v);
-                v = less ? len[u] : v;
+                const u32 x = (taken >> u) & 1u ? 0x7f800000u : len[u];
+                const bool less = x < v;
+                v = less ? x : v;
                 at = less ? (u32)u : at;
                 sz = less ? size[u] : sz;
             }
