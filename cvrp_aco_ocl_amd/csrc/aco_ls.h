@@ -1446,12 +1446,17 @@ __device__ __forceinline__ unsigned bits_below(int lim, int q0)
 
 __device__ __forceinline__ int room16(int q) { return q > kRoomMax ? kRoomMax : q < -kRoomMax ? -kRoomMax : q; }
 
-// Fewest tour positions that take the packed relocate (figures above): the
-// lines lie where neither the search nor relocate alone gets slower.
-template <int W> __device__ __forceinline__ int packed_positions(bool has_d)
+// Fewest tour positions that take the packed relocate, by waves, without and
+// with a route-length limit: the lines lie where it stops being slower, on
+// fresh tours (figures above) and after twelve iterations.  Behind a swap few
+// moves are left and its line is lower (481 nodes, 480 ants, 8 waves: search
+// 763 against 777 us; relocate alone 1155 against 1067 us on fresh tours).
+template <int W> __device__ __forceinline__ int packed_positions(bool has_d, bool alone)
 {
-    return W == 4 ? (has_d ? 480 : 400) : W == 8 ? (has_d ? 704 : 768) : W == 12 ? (has_d ? 900 : 832)
-                                                                                 : (has_d ? 1024 : 880);
+    constexpr int behind_swap[4][2] = {{300, 360}, {480, 560}, {780, 720}, {830, 830}};
+    constexpr int by_itself[4][2] = {{400, 480}, {768, 650}, {832, 900}, {850, 1024}};
+    constexpr int w = W == 4 ? 0 : W == 8 ? 1 : W == 12 ? 2 : 3;
+    return alone ? (has_d ? by_itself[w][1] : by_itself[w][0]) : (has_d ? behind_swap[w][1] : behind_swap[w][0]);
 }
 
 struct PackedTour {
@@ -1858,7 +1863,7 @@ __device__ void local_search_ant(const DevProblem &p, const DevState &s, int a, 
     if (flags & kLsRelocate) {
         bool packed = false;
         if constexpr (PACKED) {
-            if (p.packed && S >= packed_positions<W>(p.has_d)) {
+            if (p.packed && S >= packed_positions<W>(p.has_d, !(flags & kLsSwap))) {
                 packed = true;
                 // a swap keeps the depots' positions and the route indices
                 if (!(flags & kLsSwap)) ls_routes<W>(p, L, S, tid, false);

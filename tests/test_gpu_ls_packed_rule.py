@@ -1,9 +1,10 @@
 """Which tours the 16-bit relocate takes, for every number of waves, with and
-without a route-length limit: tours one position short of the line, on it and
-past it, and past it tours at the edges of a trip (512 edges), of a lane's
-eight positions and of a block's reach in one shift (4 positions per thread).
-Against the oracle.  Whole numbers: tours and evaluated-move counts must be
-equal, and so must the lengths (sums in the same order)."""
+without a route-length limit, by itself and behind a swap: tours one position
+short of the line, on it and past it, and past it tours at the edges of a
+trip (512 edges), of a lane's eight positions and of a block's reach in one
+shift (4 positions per thread).  Against the oracle.  Whole numbers: tours
+and evaluated-move counts must be equal, and so must the lengths (sums in the
+same order)."""
 import math
 
 import numpy as np
@@ -17,15 +18,18 @@ from helpers import log, oracle_problem, pack_tours
 pytestmark = pytest.mark.gpu
 
 ANTS = 4
-LINE = {(4, False): 400, (4, True): 480, (8, False): 768, (8, True): 704, (12, False): 832, (12, True): 900,
-        (16, False): 880, (16, True): 1024}
-CASES = [(w, lim, at + d) for (w, lim), at in LINE.items() for d in (-1, 0, 1)]
-CASES += [(4, False, s) for s in (511, 512, 513, 514, 1023, 1025, 1030, 1537)] + [(4, True, s) for s in (513, 520, 1025)]
-CASES += [(8, False, s) for s in (1023, 1024, 1025)] + [(12, True, s) for s in (1025, 1029)] + [(16, False, 1031)]
+ALONE, FULL = ca.LS_RELOCATE, ca.LS_2OPT | ca.LS_SWAP | ca.LS_RELOCATE
+LINE = {(4, False, FULL): 300, (4, True, FULL): 360, (8, False, FULL): 480, (8, True, FULL): 560, (12, False, FULL): 780,
+        (12, True, FULL): 720, (16, False, FULL): 830, (16, True, FULL): 830, (4, False, ALONE): 400,
+        (4, True, ALONE): 480, (8, False, ALONE): 768, (8, True, ALONE): 650, (12, False, ALONE): 832,
+        (12, True, ALONE): 900, (16, False, ALONE): 850, (16, True, ALONE): 1024}
+CASES = [(w, lim, at + d, fl) for (w, lim, fl), at in LINE.items() for d in (-1, 0, 1)]
+PAST = [(4, False, s) for s in (511, 512, 513, 514, 1023, 1025, 1030, 1537)] + [(4, True, s) for s in (513, 520, 1025)]
+PAST += [(8, False, s) for s in (1023, 1024, 1025)] + [(12, True, s) for s in (1025, 1029)] + [(16, False, 1031)]
+CASES += [(*c, fl) for c in PAST for fl in (ALONE, FULL)]
 
 
-@pytest.mark.parametrize("waves,limited,positions", CASES)
-@pytest.mark.parametrize("flags", [ca.LS_RELOCATE, ca.LS_2OPT | ca.LS_SWAP | ca.LS_RELOCATE])
+@pytest.mark.parametrize("waves,limited,positions,flags", CASES)
 def test_relocate_at_the_line(waves, limited, positions, flags):
     log(f"relocate waves={waves} limited={limited} positions={positions} flags={flags}")
     r = np.random.default_rng(positions + waves)
