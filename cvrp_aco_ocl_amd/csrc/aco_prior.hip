@@ -1388,9 +1388,10 @@ int aco_prior_build(aco_prior *net, int32_t n, const float *x, const float *y,
     struct { int row, rows, buf; } out = {0, 0, 0};   // rows on their way
     auto collect = [&]() -> int {
         if (!out.rows) return ACO_OK;
-        // the last rows: the stream itself (a stream whose last wait was an
-        // event's costs the next one made 100 us)
-        PCHK(out.row + out.rows == n ? hipStreamSynchronize(st) : hipEventSynchronize(sp.done[out.buf]));
+        // rows that all fit one part: the stream itself (11 us less than an
+        // event's wait where it is the only one, 11 us more behind others; and
+        // a stream whose last wait was an event's costs the next one made 100 us)
+        PCHK(out.rows == n ? hipStreamSynchronize(st) : hipEventSynchronize(sp.done[out.buf]));
         sp.busy[out.buf] = false;
         memcpy(prior + (size_t)out.row * N, sp.pin + out.buf * sp.part, (size_t)out.rows * N * 4);
         return ACO_OK;
