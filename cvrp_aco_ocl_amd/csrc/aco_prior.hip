@@ -1247,17 +1247,20 @@ int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64
     // The order of an epoch is a Fisher-Yates shuffle, which only the host can
     // make (65536 swaps: 0.1 ms), but the swap targets are one 64-bit remainder
     // each (0.3 ms) of a counter-based stream, so the device draws them, two
-    // buffers ahead of the swaps: the first two before the features go out,
-    // the others on a stream of their own, beside the training.  Epochs of
-    // fewer than kDeviceDraws draws draw on the host, where they cost less
-    // (5 ns each) than a launch and its wait (about 20 us), and a network that
-    // trains once on few edges makes no stream.
+    // buffers ahead of the swaps.  On the training stream, while nothing is
+    // trained yet, and where a buffer holds an epoch (then its next one is
+    // needed an epoch later); else beside the training, on a stream of its
+    // own, which takes 0.4 to 3 ms to make (one epoch over 513024 edges on a
+    // new network: 4.1 ms with host draws, 6.7 to 7.8 with that stream, 3.4
+    // so).  Epochs of fewer than kDeviceDraws draws draw on the host, where
+    // they cost less (5 ns each) than a launch and its wait (about 20 us).
     const long long per_epoch = count - 1, draws = per_epoch * tp->epochs;
     const bool device = per_epoch >= kDeviceDraws;
     const int chunk = (int)std::min<long long>(std::max(per_epoch, 1ll), PriorSpace::kPart / sizeof(int));
     const size_t span = SpaceUse::round((size_t)chunk * sizeof(int));
     PCHK(sp.pinned(E * (NF + 1) * sizeof(float), 0, device ? 2 * span : 0));
     auto targets = [&](int i) { return reinterpret_cast<int *>(sp.result() + i * span); };
+    long long step = 0;    // batches launched
     long long drawn = 0;   // draws requested so far
     int requests = 0;      // request r fills buffer r % 2
     hipEvent_t ready[2] = {nullptr, nullptr};
@@ -1274,8 +1277,9 @@ int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64
         const long long in = drawn % per_epoch;
         const int c = (int)std::min<long long>(chunk, per_epoch - in), at = requests & 1;
         if (!ready[at]) PCHK(hipEventCreateWithFlags(&ready[at], hipEventDisableTiming));
-        if (requests >= 2 && !sp.side) PCHK(hipStreamCreateWithFlags(&sp.side, hipStreamNonBlocking));
-        const hipStream_t on = requests >= 2 ? sp.side : net->stream;
+        const bool beside = step > 0 && per_epoch > chunk;
+        if (beside && !sp.side) PCHK(hipStreamCreateWithFlags(&sp.side, hipStreamNonBlocking));
+        const hipStream_t on = beside ? sp.side : net->stream;
         hipLaunchKernelGGL(k_swap_targets, dim3((c + 255) / 256), dim3(256), 0, on, tp->shuffle_seed,
                            (unsigned long long)drawn, (int)(per_epoch - in), c, targets(at));
         PCHK(hipGetLastError());
@@ -1290,7 +1294,6 @@ int aco_prior_train(aco_prior *net, const float *feat, const float *label, int64
     rc = stage_features(net, feat, label, count, xb, lab);
     if (rc != ACO_OK) return rc;
     std::vector<int> perm((size_t)count);
-    long long step = 0;
     int from = 0;   // buffer the next targets come from
     uint64_t seed = tp->shuffle_seed;
     for (int ep = 0; ep < tp->epochs; ++ep) {

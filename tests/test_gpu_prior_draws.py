@@ -1,7 +1,7 @@
 """Training whose epochs draw their swap targets on the host (fewer than 4096
 draws) and on the device, on both sides of the line: one epoch, two (the
-requests ahead) and more (the later ones on a stream of their own), and twice
-on one network.  The order is written out here; the batches it gives, taken
+requests ahead) and more, and twice on one network; and epochs of two buffers
+(131072 draws each), whose third and later epochs draw beside the training.  The order is written out here; the batches it gives, taken
 one by one with gradient and Adam step, must give the same parameters, bit
 for bit."""
 import numpy as np
@@ -44,3 +44,18 @@ def test_order_of_small_and_large_epochs(E, epochs):
                     g, _ = step.gradient(f[at], y[at], 3.0)
                     step.adam_step(g, 1e-3)
             np.testing.assert_array_equal(net.params(), step.params())
+
+
+def test_order_of_epochs_of_two_buffers():
+    E, epochs, batch = 131074, 4, 65536
+    log(f"training draws E={E} epochs={epochs}")
+    r = np.random.default_rng(E)
+    f, y = r.normal(0, 1, (E, 12)).astype(np.float32), (r.random(E) < 0.1).astype(np.float32)
+    with pr.PriorNet(5) as net, pr.PriorNet(5) as step:
+        net.train(f, y, epochs=epochs, batch=batch, lr=1e-3, lr_final=1e-3, pos_weight=3.0, shuffle_seed=9)
+        for perm in _orders(E, epochs, 9):
+            for b in range(0, E, batch):
+                at = perm[b:b + batch]
+                g, _ = step.gradient(f[at], y[at], 3.0)
+                step.adam_step(g, 1e-3)
+        np.testing.assert_array_equal(net.params(), step.params())
