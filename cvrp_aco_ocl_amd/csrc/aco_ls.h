@@ -5,7 +5,8 @@
 //             sequential scan order, first improvement over the nn list
 //             with radius pruning, don't-look bits.  Routes are independent
 //             (the depot's don't-look bit starts clear on route 0 and set on
-//             later routes); a group of 8 lanes searches one route.
+//             later routes); a group of 8 to 64 lanes searches one route,
+//             1 to 8 of its positions at a time by 8 lanes each.
 //   swap      LocalSearch::swap (localSearch.cpp:301-410): for each position
 //             i in order, the first j > i whose swap gains more than
 //             EPSILON and keeps loads and route lengths feasible.
@@ -13,7 +14,8 @@
 //             move.cpp:32-51).
 //
 // swap and relocate run speculatively on W consecutive positions: wave w
-// scans position i0+w against the current tour (4 x 64 j per loop trip).
+// scans position i0+w against the current tour (kSwapUnroll or
+// kRelocateUnroll x 64 j per loop trip; 512 edges in the packed relocate).
 // The smallest position with a move is exactly the sequential scan's next
 // move, because no earlier position moved; results of later positions are
 // discarded.  Distance rows of the positions around i0 sit in an LDS ring

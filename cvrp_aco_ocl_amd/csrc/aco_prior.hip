@@ -21,8 +21,10 @@
 // the contraction, so the product sums exactly the slices' terms, whatever
 // order the unit adds them in.
 //
-// Determinism: per-wave partial gradients (fixed tile assignment) are summed
-// by the reduce kernel in a fixed order; there are no atomics.
+// Determinism: a wave's tiles follow from its index, a block's waves add their
+// gradients in wave order to one partial row, and the reduce kernel sums the
+// rows in a fixed order (runs of consecutive blocks, then the runs); there are
+// no atomics.
 
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -448,7 +450,7 @@ __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, co
 }
 
 // Per parameter: the sum of the partial rows in a fixed order (runs of
-// consecutive waves, then the runs in order), then (update != 0) Adam in
+// consecutive blocks, then the runs in order), then (update != 0) Adam in
 // fp32.  Parameter NP is the loss.
 struct AdamArgs {
     float lr, beta1, om_beta1, beta2, om_beta2, c1, c2, eps;
@@ -706,7 +708,7 @@ using namespace cvrp::prior;
 // Pageable copies of this size cost 25 to 60 us each whatever they hold,
 // allocations of 2 MB and more 25 us; a gradient made six of the first and two
 // of the second.  Gradient over 16384 edges 202 -> 75 us, multiplier of 501
-// nodes 200 -> 128 us, eight training steps of 16384 edges 932 -> 500 us; what
+// nodes 200 -> 115 us, eight training steps of 16384 edges 932 -> 500 us; what
 // is left is the copy into the buffers, the launches and the kernels (25 us
 // of the gradient).
 // Parts are as large as the largest call so far needs, up to kPart, and a call
