@@ -41,7 +41,9 @@ typedef struct aco_prior_train_params {
 void aco_prior_default_train_params(aco_prior_train_params *tp);
 
 /* Glorot-uniform weights from a SplitMix64 stream seeded with `seed`, zero
- * biases, zero Adam moments. */
+ * biases, zero Adam moments.  A network keeps the working memory of its
+ * calls, one call at a time: at most 64 MB on the device and 2 MB of pinned
+ * host memory, by the largest call so far, until it is destroyed. */
 int aco_prior_create(uint64_t seed, aco_prior **out);
 int aco_prior_destroy(aco_prior *net);
 int aco_prior_get_params(aco_prior *net, float *params, int32_t count);
