@@ -703,18 +703,32 @@ __device__ __forceinline__ int greedy_own(const DevProblem &p, const AntLds &L, 
         d0[u] = HAS_D ? L.d0[ic] : 0.0f;
     }
     u32 val[NODES], best = 0;
+    bool fits = !HAS_D;   // some node of the lane is feasible with the limit too
 #pragma unroll
     for (int u = 0; u < NODES; ++u) {
         if (HAS_D) {
             float t = rdist + (dv[u] + p.svc);
             t = t + d0[u];
             f[u] = f[u] & (t <= p.D);
+            fits |= f[u];
         }
         val[u] = f[u] ? f2u(tv[u]) + 1u : 0u;
         best = val[u] > best ? val[u] : best;
     }
     const u32 top = lanes_max_u32<kLanes>(best);
-    if (HAS_D && top == 0) return 0;
+    if (__builtin_expect(top == 0, 0)) {
+        if (HAS_D && !__ballot(fits)) return 0;
+        // only values whose bits are all ones (a NaN): the lowest feasible node
+#pragma unroll 1
+        for (int base = 0; base < p.n; base += kLanes) {
+            const int i = base + lane, ic = i < p.n ? i : p.n - 1;
+            const float dci = HAS_D ? gload(drow + ic) : 0.0f;
+            const bool ok = (i < p.n) & feasible_mask<HAS_D>(p, L, ic, L.dem[ic], dci, load, rdist);
+            const u64 b = __ballot(ok);
+            if (b) return base + __builtin_ctzll(b);
+        }
+        return 0;
+    }
     // the lowest node with that value
     u32 low = 0;
 #pragma unroll
@@ -833,7 +847,7 @@ __device__ void construct_knn_ant(const DevProblem &p, const DevState &s, int a,
 // With a length limit and sixteen nodes per lane the narrow shape, which is
 // for more ants than SIMDs, is held to 128 registers, so that four ants share
 // a SIMD: with the 142 it would take, three do, and 4096 ants at 1001 nodes
-// take 1716 us instead of 1285 (513 nodes: 873, 631).  One round of ants is
+// take 1716 us instead of 1300 (513 nodes: 850, 625).  One round of ants is
 // not changed by it (1500 ants at 1001 nodes: 932, 945).
 template <bool HAS_D, int RNG, bool WIDE, int NODES>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(HAS_D && !WIDE && NODES > 8 ? 4 : 1)))

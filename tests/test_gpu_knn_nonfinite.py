@@ -40,7 +40,8 @@ def tour_without_draws(inst, ti, nn):
         c = nn[cur, :K]
         bad = np.isnan(ti[cur, c]) | (np.isinf(ti[cur, c]) & ~ok[c])
         if bad.any() or not ok[c].any():
-            w = int(np.argmax(np.where(ok, bits[cur].astype(np.int64) + 1, 0))) if ok.any() else 0
+            # one more than the bits, in 32 bits: all ones come last
+            w = int(np.argmax(np.where(ok, (bits[cur].astype(np.int64) + 1) & 0xFFFFFFFF, -1))) if ok.any() else 0
             picks += 1
         else:
             w = int(c[ok[c] & (ti[cur, c] > 0)][-1])
@@ -104,6 +105,40 @@ def test_wheel_without_a_positive_total(n, limited, apb, rng, kind):
         assert sizes[a] == len(t), a
         np.testing.assert_array_equal(tours[a, : sizes[a]], t, err_msg=f"ant {a}")
     assert fallbacks == picks > 0
+
+
+@pytest.mark.parametrize("part", [1.0, 0.6])
+@pytest.mark.parametrize("n,limited,apb", [(40, False, 0), (40, True, 0), (70, False, 4), (600, False, 0), (600, True, 0),
+                                           (600, False, 2), (1024, True, 0), (1100, False, 0)])
+def test_bits_all_ones(n, limited, apb, part):
+    """NaN with every bit set, everywhere or in most entries, the rest 0 (at
+    every candidate, so no draw matters): the last of all values, but a node
+    that has it is still placed."""
+    log(f"total_info all ones n={n} limited={limited} apb={apb} part={part}")
+    r = np.random.default_rng(n)
+    xy = r.integers(0, 300, size=(n, 2)).astype(np.float64)
+    dem = np.concatenate([[0], r.integers(1, 30, size=n - 1)]).astype(np.int32)
+    lim, svc = math.inf, 0.0
+    if limited:
+        svc = 2.0
+        lim = math.ceil(2.5 * float(np.hypot(*(xy - xy[0]).T).max()) + 4 * svc)
+    inst = Instance.from_coords(xy[:, 0], xy[:, 1], dem, 150, ca.DIST_NINT, max_dist=lim, service_time=svc)
+    nn = inst.nn_lists(K)
+    bits = np.where(r.random((n, n)) < part, 0xFFFFFFFF, 0).astype(np.uint32)
+    bits[np.arange(n)[:, None], nn] = 0xFFFFFFFF
+    ti = bits.view(np.float32)
+    with ca.GpuACO(inst, n_ants=ANTS, k=K, seed=3, selection=ca.SEL_KNN, rng=ca.RNG_PHILOX, ls_flags=0, use_graph=False,
+                   tau0_rule=ca.TAU0_NN_TOUR) as g:
+        g.init_aco()
+        if apb:
+            g.set_launch_shape(4, 16, 0, apb, 0)
+        g.set_pheromone(np.full((n, n), 0.5, np.float32), ti)
+        g.construct_solutions()
+        tours, sizes, _ = g.ants()
+    t, _ = tour_without_draws(inst, ti, nn)
+    for a in range(ANTS):
+        assert sizes[a] == len(t), a
+        np.testing.assert_array_equal(tours[a, : sizes[a]], t, err_msg=f"ant {a}")
 
 
 def test_customers_in_one_place():
