@@ -21,10 +21,9 @@
 // the contraction, so the product sums exactly the slices' terms, whatever
 // order the unit adds them in.
 //
-// Determinism: a wave's tiles follow from its index, a block's waves add their
-// gradients in wave order to one partial row, and the reduce kernel sums the
-// rows in a fixed order (runs of consecutive blocks, then the runs); there are
-// no atomics.
+// Determinism: a partial row of the gradient holds four consecutive tiles,
+// added one after another, and the reduce kernel sums the rows in a fixed
+// order (runs of consecutive rows, then the runs); there are no atomics.
 
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -85,8 +84,7 @@ __device__ __forceinline__ v4f mfma2(v4s a0, v4s a1, v4s b0, v4s b1, v4f c)
 }
 
 // Block-resident network: bf16 weights (W2 also transposed, for dH1),
-// fp32 biases, w3 rounded to bf16 and widened, and per-wave 16x16 bf16
-// transpose buffers.
+// fp32 biases, w3 rounded to bf16 and widened.
 struct NetLds {
     alignas(16) unsigned short w1[H][NFP];
     alignas(16) unsigned short w2[H][H];
@@ -95,7 +93,6 @@ struct NetLds {
     alignas(16) float b2[H];
     alignas(16) float w3[H];
     float b3;
-    alignas(16) unsigned short tr[kWaves][9][16][16];
 };
 
 // Every global read is requested before the first LDS write (8 or 16 bytes
@@ -233,18 +230,19 @@ __device__ __forceinline__ void fwd_tile(const Wt &W, v4s x, Fwd &F)
     F.z = s + W.b3();
 }
 
-// Accumulator-layout tile (rows 4g+j, column r) -> LDS, read back as the
-// operand of a product contracting over the former columns: lane gets
-// row r, columns 4g..4g+3.
-__device__ __forceinline__ v4s transpose_tile(unsigned short (*T)[16], v4s d, int lane)
+// Accumulator-layout tile (rows 4g+j, column r) -> LDS ...
+__device__ __forceinline__ void put_tile(unsigned short (*T)[16], v4s d, int lane)
 {
     const int r = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int j = 0; j < 4; ++j) T[4 * g + j][r] = (unsigned short)d[j];
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    const v4s out = ld4(&T[r][4 * g]);
-    return out;
+}
+
+// ... read back as the operand of a product contracting over the former
+// columns: lane gets row r, columns 4g..4g+3.
+__device__ __forceinline__ v4s take_tile(unsigned short (*T)[16], int lane)
+{
+    return ld4(&T[lane & 15][4 * (lane >> 4)]);
 }
 
 __device__ __forceinline__ v4s pack_bf16(v4f v)
@@ -290,17 +288,24 @@ __global__ __launch_bounds__(kThreads) void k_forward(const unsigned short *xb, 
 }
 
 // Fused forward + backward (positions [0, Eb) of idx, or of the data in order
-// without one): wave w of block b takes the tiles of 16 edges 4b + w, + 4
-// blocks, ...; the block's waves add their gradients in LDS in wave order and
-// write one partial row.  A wave's chain of products, conversions and
-// transposes is the launch's length, and a CU holds one block (the
-// accumulators), so a batch gets a block per four tiles up to kTrainBlocks,
-// one per CU, and more tiles per wave beyond: 16384 edges on 64 blocks of four
-// tiles per wave take 36 us, on 256 blocks of one 19.5 us; 65536 edges on 1024
-// blocks of one tile 70 us, on 256 blocks of four 37 us (30000: 37, 25).  A
-// constant, so the order of the sums does not depend on the device.
-constexpr int kTrainBlocks = 256;
-static int train_blocks(int Eb) { return std::min((Eb + 16 * kWaves - 1) / (16 * kWaves), kTrainBlocks); }
+// without one).  Four tiles of 16 edges make one partial row: their products
+// are accumulated tile after tile, which fixes the order of every sum, but
+// the chain of a tile up to that point is the launch's length, so each wave
+// of a block runs it for one of the four.  The tiles' operands (bf16) and
+// bias terms (fp32) pass through LDS; then wave w accumulates rows 16w ..
+// 16w+15 of both weight gradients, and the bias terms of the same rows, over
+// the four tiles in order.  A CU holds one block (LDS), and one that takes
+// every kTrainBlocks-th group reads the network once.  With a wave for all
+// four tiles of a row 16384 edges took 35.7 us on 64 of the CUs, now 13.7 us on
+// all (1024 edges 32.0, 11.3; 65536, where every CU is busy either way, 43.9,
+// 42.5).
+struct TrainLds {
+    alignas(16) unsigned short tr[kWaves][13][16][16];   // dz2, h1, x, dz1 of a wave's tile
+    alignas(16) float terms[3][4][kWaves][64][4];        // of b1, b2, w3: row block, tile, lane
+    float out[2][kWaves][16];                            // of b3 and the loss
+};
+constexpr int kTrainBlocks = 256;   // one per CU
+static int train_rows(int Eb) { return (Eb + 16 * kWaves - 1) / (16 * kWaves); }
 
 __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, const float *label,
                                                     const int *idx, int Eb,
@@ -308,149 +313,120 @@ __global__ __launch_bounds__(kThreads) void k_train(const unsigned short *xb, co
                                                     float pos_weight, float invE, float *partials)
 {
     __shared__ NetLds S;
+    __shared__ TrainLds B;
     load_net(S, wb, pf);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
-    const int tiles = (Eb + 15) / 16;
-    unsigned short(*T)[16][16] = S.tr[w];
+    const int tiles = (Eb + 15) / 16, groups = (tiles + kWaves - 1) / kWaves;
     const v4f zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
-    v4f dW2[4][4], dW1[4], db1[4], db2[4], dw3[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        dW1[a] = db1[a] = db2[a] = dw3[a] = zero4;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) dW2[a][b] = zero4;
-    }
-    float db3 = 0.0f, loss = 0.0f;
-    for (int tile = blockIdx.x * kWaves + w; tile < tiles; tile += gridDim.x * kWaves) {
-        const int pos = tile * 16 + r;
-        const bool valid = pos < Eb;
-        const int e = !valid ? 0 : idx ? idx[pos] : pos;
-        const v4s x = load_x(xb, e, valid, g);
-        const float y = valid ? label[e] : 0.0f;
-        Fwd F;
-        fwd_tile(LdsWeights{S, r, g}, x, F);
-        const float we = valid ? (y > 0.5f ? pos_weight : 1.0f) : 0.0f;
-        const float sig = 1.0f / (1.0f + expf(-F.z));
-        const float ge = we * (sig - y) * invE;
-        if (g == 0 && valid) {
-            loss += we * ((fmaxf(F.z, 0.0f) - y * F.z) + log1pf(expf(-fabsf(F.z))));
-            db3 += ge;
-        }
-        // layer 3 and the ReLU of layer 2
-        v4s dz2b[4];
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-            v4f d;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const bool on = F.z2[mt][j] > 0.0f;
-                dw3[mt][j] += ge * (on ? F.z2[mt][j] : 0.0f);
-                d[j] = on ? S.w3[16 * mt + 4 * g + j] * ge : 0.0f;
-                db2[mt][j] += d[j];
+    for (int group = blockIdx.x; group < groups; group += gridDim.x) {
+        const int tile = group * kWaves + w, count = min(kWaves, tiles - group * kWaves);
+        if (w < count) {
+            unsigned short(*T)[16][16] = B.tr[w];
+            const int pos = tile * 16 + r;
+            const bool valid = pos < Eb;
+            const int e = !valid ? 0 : idx ? idx[pos] : pos;
+            const v4s x = load_x(xb, e, valid, g);
+            const float y = valid ? label[e] : 0.0f;
+            Fwd F;
+            fwd_tile(LdsWeights{S, r, g}, x, F);
+            const float we = valid ? (y > 0.5f ? pos_weight : 1.0f) : 0.0f;
+            const float sig = 1.0f / (1.0f + expf(-F.z));
+            const float ge = we * (sig - y) * invE;
+            if (g == 0) {
+                B.out[0][w][r] = valid ? ge : 0.0f;
+                B.out[1][w][r] =
+                    valid ? we * ((fmaxf(F.z, 0.0f) - y * F.z) + log1pf(expf(-fabsf(F.z)))) : 0.0f;
             }
-            dz2b[mt] = pack_bf16(d);
-        }
-        // dH1 = W2^T dz2 (dz2 is already the B operand), ReLU of layer 1
-        v4s dz1b[4];
+            put_tile(T[8], x, lane);
+            // layer 3 and the ReLU of layer 2
+            v4s dz2b[4];
 #pragma unroll
-        for (int it = 0; it < 4; ++it) {
-            v4f c = mfma2(ld4(&S.w2t[16 * it + r][4 * g]), ld4(&S.w2t[16 * it + r][16 + 4 * g]), dz2b[0],
-                          dz2b[1], zero4);
-            c = mfma2(ld4(&S.w2t[16 * it + r][32 + 4 * g]), ld4(&S.w2t[16 * it + r][48 + 4 * g]), dz2b[2],
-                      dz2b[3], c);
-            v4f d;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                d[j] = F.z1[it][j] > 0.0f ? c[j] : 0.0f;
-                db1[it][j] += d[j];
-            }
-            dz1b[it] = pack_bf16(d);
-        }
-        // weight gradients contract over the 16 edges of the tile
-        v4s aT[4], hT[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            aT[q] = transpose_tile(T[q], dz2b[q], lane);
-            hT[q] = transpose_tile(T[4 + q], F.h1[q], lane);
-        }
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-            for (int it = 0; it < 4; ++it) dW2[mt][it] = mfma(aT[mt], hT[it], dW2[mt][it]);
-        const v4s xT = transpose_tile(T[8], x, lane);
-#pragma unroll
-        for (int ot = 0; ot < 4; ++ot) {
-            const v4s a1 = transpose_tile(T[ot], dz1b[ot], lane);
-            dW1[ot] = mfma(a1, xT, dW1[ot]);
-        }
-    }
-    // bias / w3 gradients: sum over the 16 edge lanes of each row group
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int o = 1; o < 16; o <<= 1) {
-                db1[t][j] += __shfl_xor(db1[t][j], o);
-                db2[t][j] += __shfl_xor(db2[t][j], o);
-                dw3[t][j] += __shfl_xor(dw3[t][j], o);
-            }
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) {
-        db3 += __shfl_xor(db3, o);
-        loss += __shfl_xor(loss, o);
-    }
-    // the block's partial row, wave after wave: a wave reads its 80 sums
-    // together before it writes any (an add at a time is a chain of LDS round
-    // trips)
-    __shared__ float sum[NPL];
-    for (int turn = 0; turn < kWaves; ++turn) {
-        if (turn == w) {
-            const bool more = turn > 0;
-            const int o2 = OFF_W2 + 4 * g * H + r, o1 = OFF_W1 + 4 * g * NF + (r < NF ? r : 0), ob = 4 * g;
-            float s2[4][4][4], s1[4][4], sb[3][4][4], s3 = 0.0f, sl = 0.0f;
-            if (more) {
-#pragma unroll
-                for (int a = 0; a < 4; ++a)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-                        for (int b = 0; b < 4; ++b) s2[a][b][j] = sum[o2 + (16 * a + j) * H + 16 * b];
-                        s1[a][j] = sum[o1 + (16 * a + j) * NF];
-                        sb[0][a][j] = sum[OFF_B1 + ob + 16 * a + j];
-                        sb[1][a][j] = sum[OFF_B2 + ob + 16 * a + j];
-                        sb[2][a][j] = sum[OFF_W3 + ob + 16 * a + j];
-                    }
-                s3 = sum[OFF_B3];
-                sl = sum[NP];
-            }
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int mt = 0; mt < 4; ++mt) {
+                v4f d, d3;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-#pragma unroll
-                    for (int b = 0; b < 4; ++b)
-                        sum[o2 + (16 * a + j) * H + 16 * b] = more ? s2[a][b][j] + dW2[a][b][j] : dW2[a][b][j];
-                    if (r < NF) sum[o1 + (16 * a + j) * NF] = more ? s1[a][j] + dW1[a][j] : dW1[a][j];
-                    if (r == 0) {
-                        sum[OFF_B1 + ob + 16 * a + j] = more ? sb[0][a][j] + db1[a][j] : db1[a][j];
-                        sum[OFF_B2 + ob + 16 * a + j] = more ? sb[1][a][j] + db2[a][j] : db2[a][j];
-                        sum[OFF_W3 + ob + 16 * a + j] = more ? sb[2][a][j] + dw3[a][j] : dw3[a][j];
-                    }
+                    const bool on = F.z2[mt][j] > 0.0f;
+                    d3[j] = ge * (on ? F.z2[mt][j] : 0.0f);
+                    d[j] = on ? S.w3[16 * mt + 4 * g + j] * ge : 0.0f;
                 }
-            if (lane == 0) {
-                sum[OFF_B3] = more ? s3 + db3 : db3;
-                sum[NP] = more ? sl + loss * invE : loss * invE;
+                *reinterpret_cast<v4f *>(B.terms[1][mt][w][lane]) = d;
+                *reinterpret_cast<v4f *>(B.terms[2][mt][w][lane]) = d3;
+                dz2b[mt] = pack_bf16(d);
+                put_tile(T[mt], dz2b[mt], lane);
+                put_tile(T[4 + mt], F.h1[mt], lane);
+            }
+            // dH1 = W2^T dz2 (dz2 is already the B operand), ReLU of layer 1
+#pragma unroll
+            for (int it = 0; it < 4; ++it) {
+                v4f c = mfma2(ld4(&S.w2t[16 * it + r][4 * g]), ld4(&S.w2t[16 * it + r][16 + 4 * g]), dz2b[0],
+                              dz2b[1], zero4);
+                c = mfma2(ld4(&S.w2t[16 * it + r][32 + 4 * g]), ld4(&S.w2t[16 * it + r][48 + 4 * g]), dz2b[2],
+                          dz2b[3], c);
+                v4f d;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) d[j] = F.z1[it][j] > 0.0f ? c[j] : 0.0f;
+                *reinterpret_cast<v4f *>(B.terms[0][it][w][lane]) = d;
+                put_tile(T[9 + it], pack_bf16(d), lane);
             }
         }
         __syncthreads();
+        // weight gradients contract over the 16 edges of each tile
+        v4f dW2[4], dW1 = zero4, db[3];
+#pragma unroll
+        for (int it = 0; it < 4; ++it) dW2[it] = zero4;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) db[q] = zero4;
+        float o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+        for (int t = 0; t < kWaves; ++t) {
+            if (t >= count) break;
+            unsigned short(*T)[16][16] = B.tr[t];
+            const v4s aT = take_tile(T[w], lane);
+#pragma unroll
+            for (int it = 0; it < 4; ++it) dW2[it] = mfma(aT, take_tile(T[4 + it], lane), dW2[it]);
+            dW1 = mfma(take_tile(T[9 + w], lane), take_tile(T[8], lane), dW1);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const v4f d = *reinterpret_cast<const v4f *>(B.terms[q][w][t][lane]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) db[q][j] += d[j];
+            }
+            o0 += B.out[0][t][r];
+            o1 += B.out[1][t][r];
+        }
+        float *P = partials + (size_t)group * NPL;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int row = 16 * w + 4 * g + j;
+#pragma unroll
+            for (int it = 0; it < 4; ++it) P[OFF_W2 + row * H + 16 * it + r] = dW2[it][j];
+            if (r < NF) P[OFF_W1 + row * NF + r] = dW1[j];
+            // bias / w3 gradients: sum over the 16 edge lanes of each row group
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+#pragma unroll
+                for (int o = 1; o < 16; o <<= 1) db[q][j] += __shfl_xor(db[q][j], o);
+            if (r == 0) {
+                P[OFF_B1 + row] = db[0][j];
+                P[OFF_B2 + row] = db[1][j];
+                P[OFF_W3 + row] = db[2][j];
+            }
+        }
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+            o0 += __shfl_xor(o0, o);
+            o1 += __shfl_xor(o1, o);
+        }
+        if (threadIdx.x == 0) {
+            P[OFF_B3] = o0;
+            P[NP] = o1 * invE;
+        }
+        if (group + (int)gridDim.x < groups) __syncthreads();   // the buffers are read
     }
-    float *P = partials + (size_t)blockIdx.x * NPL;
-    for (int i = threadIdx.x; i < NPL; i += kThreads) P[i] = sum[i];
 }
 
 // Per parameter: the sum of the partial rows in a fixed order (runs of
-// consecutive blocks, then the runs in order), then (update != 0) Adam in
+// consecutive rows, then the runs in order), then (update != 0) Adam in
 // fp32.  Parameter NP is the loss.
 struct AdamArgs {
     float lr, beta1, om_beta1, beta2, om_beta2, c1, c2, eps;
@@ -460,17 +436,19 @@ struct AdamArgs {
 // threads over consecutive runs of the partial rows, then the runs' sums are
 // added in run order (a fixed order: runs are deterministic).
 // Sixteen rows are requested together (same order of additions): 256 rows
-// 10.7 -> 4.1 us, which was bound by one row's latency after another.
+// 10.0 -> 4.0 us, 1024 rows 37.7 -> 7.3, which was bound by one row's latency
+// after another.
 constexpr int kReduceParams = 32, kReduceGroups = 8;
+// Rows per run for a batch: its partial rows rounded up to fours.
+static int train_run(int rows) { return ((rows + kWaves - 1) / kWaves * kWaves + kReduceGroups - 1) / kReduceGroups; }
 
 __global__ __launch_bounds__(kReduceParams * kReduceGroups) void k_reduce_adam(
-    const float *partials, int W, float *pf, float *m, float *v, unsigned short *wb, float *grad_out,
+    const float *partials, int W, int run, float *pf, float *m, float *v, unsigned short *wb, float *grad_out,
     float *loss_out, int update, AdamArgs a)
 {
     __shared__ float red[kReduceGroups][kReduceParams];
     const int i = threadIdx.x % kReduceParams, q = threadIdx.x / kReduceParams;
     const int p = blockIdx.x * kReduceParams + i;
-    const int run = (W + kReduceGroups - 1) / kReduceGroups;
     const int w0 = q * run, w1 = min(W, w0 + run);
     float part = 0.0f;
     if (p <= NP)
@@ -998,13 +976,13 @@ static int launch_batch(aco_prior *net, const unsigned short *xb, const float *l
                         int Eb, float pos_weight, float *partials, float *grad_out, float *loss_out,
                         bool update, const AdamArgs &aa)
 {
-    const int blocks = train_blocks(Eb);
-    hipLaunchKernelGGL(k_train, dim3(blocks), dim3(kThreads), 0, net->stream, xb, label, idx, Eb,
+    const int rows = train_rows(Eb);
+    hipLaunchKernelGGL(k_train, dim3(std::min(rows, kTrainBlocks)), dim3(kThreads), 0, net->stream, xb, label, idx, Eb,
                        net->wb, net->pf, pos_weight, 1.0f / (float)Eb, partials);
     PCHK(hipGetLastError());
     hipLaunchKernelGGL(k_reduce_adam, dim3((NPL + kReduceParams - 1) / kReduceParams),
                        dim3(kReduceParams * kReduceGroups), 0, net->stream, partials,
-                       blocks, net->pf, net->m, net->v, net->wb, grad_out, loss_out,
+                       rows, train_run(rows), net->pf, net->m, net->v, net->wb, grad_out, loss_out,
                        update ? 1 : 0, aa);
     PCHK(hipGetLastError());
     return ACO_OK;
@@ -1012,7 +990,7 @@ static int launch_batch(aco_prior *net, const unsigned short *xb, const float *l
 
 static size_t partial_bytes(int Eb)
 {
-    return (size_t)train_blocks(Eb) * NPL * sizeof(float);
+    return (size_t)train_rows(Eb) * NPL * sizeof(float);
 }
 
 extern "C" {
@@ -1216,7 +1194,7 @@ int aco_prior_adam_step(aco_prior *net, const float *grad, float lr, float beta1
     PCHK(hipMemcpyAsync(part.p, grad, NP * 4, hipMemcpyHostToDevice, net->stream));
     net->step += 1;
     hipLaunchKernelGGL(k_reduce_adam, dim3((NPL + kReduceParams - 1) / kReduceParams),
-                       dim3(kReduceParams * kReduceGroups), 0, net->stream, part.as<float>(), 1,
+                       dim3(kReduceParams * kReduceGroups), 0, net->stream, part.as<float>(), 1, 1,
                        net->pf, net->m, net->v, net->wb, nullptr, nullptr, 1,
                        adam_args(net->step, lr, beta1, beta2, eps));
     PCHK(hipGetLastError());
